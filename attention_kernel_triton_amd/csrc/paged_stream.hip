@@ -9,16 +9,26 @@
 //   g = y * TG + position * gpp + slice,   TG = total_pages * gpp,
 // where `position` indexes kv_page_indices, so sequence b's groups of head
 // group y are the contiguous range [y*TG + indptr[b]*gpp, y*TG + indptr[b+1]*gpp).
-// The W waves of the launch take equal contiguous ranges of that axis
-// (wave w: [w*N/W, (w+1)*N/W)), fixed before the launch: no tickets, no
-// workgroup barriers after the prologue.  A wave streams its range with two
-// groups in flight, keeps one online softmax for the unit it is in, and at
-// each unit boundary either writes the unit's output (a unit wholly inside
-// the wave) or stores a partial (m, l, o).  Only a wave's first and last
-// segments can be partial.  At its end a wave counts its partials in their
-// units' arrival counters; the wave that counts a unit's last partial merges
-// them (log-sum-exp over the contiguous waves that cover the unit, in wave
-// order, so results do not depend on timing) and writes the output.
+// The W waves of the launch take equal contiguous ranges of that axis (wave w:
+// [w*N/W, (w+1)*N/W)), fixed before the launch: no tickets, no workgroup
+// barrier between the prologue and the end of the stream.  A wave streams its range with two groups in flight, keeps one
+// online softmax for the unit it is in, and at each unit boundary either
+// writes the unit's output (a unit wholly inside the wave) or leaves the
+// segment's state (m, l, o) in LDS.  Only a wave's first and last segments
+// can be partial.
+//
+// Merge.  After its waves' streams a workgroup combines each unit's segments
+// from LDS (log-sum-exp in wave order).  A unit inside the workgroup's range is
+// then done.  Only the (at most two) units that reach into a neighbouring
+// workgroup's range cost a global partial: it is stored with device scope and
+// counted in the unit's arrival counter.  The wave that counts the last one
+// merges them at once if one round trip of loads takes them all; else its
+// workgroup does, wave v taking partials v, v + 8, ...; in an order that does
+// not depend on timing either way.  Measured against one partial per wave and
+// one wave merging a unit's partials ten to a round trip: a lone sequence of
+// 30001 tokens (B=1, Hq=32, Hkv=8, D=128; 256 partials to a unit, 26 dependent
+// round trips) 78.0 -> 33.8 us; 32 sequences of 256-8192 tokens 108.1 -> 106.4
+// us; 16 of 512-2048 tokens 26 -> 23 us.
 //
 // Per group: four (D=128) v_mfma_f32_16x16x32_f16 give the 16-token x 16-head
 // score block as S^T (lane (R, c) holds head c, tokens 4R .. 4R+3); the online
@@ -28,6 +38,8 @@
 // from an LDS copy of the group's V rows with ds_read_b64_tr_b16.
 #include <math.h>
 
+#include <algorithm>
+
 #include "akt_common.hpp"
 #include "akt_host.hpp"
 #include "paged_stream.hpp"
@@ -36,6 +48,17 @@ namespace akt {
 namespace {
 
 #define AKT_SNEG_INF (-__builtin_inff())
+
+// The kernel's arguments, re-read from the kernel-argument segment (the opaque
+// pointer keeps the compiler from reusing, and so holding, earlier reads): what
+// only the unit boundaries and the merge use would otherwise take scalar
+// registers from the stream's loop, which spills them to vector lanes.
+typedef const __attribute__((address_space(4))) StreamParams* StreamArgs;
+__device__ __forceinline__ StreamArgs reread_args() {
+  StreamArgs a = (StreamArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+}
 
 // Last index i in [0, n] with s[i] <= x, given a non-decreasing s[0..n];
 // -1 if s[0] > x.
@@ -91,10 +114,20 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   // non-decreasing).
   __shared__ int sm_s[kStreamMaxBatch + 1];
   __shared__ int sm_wmax[kSWaves];
+  __shared__ int sm_fin[2];  // units whose last partial this workgroup counted (-1: none)
   // Groups each wave has consumed (paired waves only).
   __shared__ int sm_prog[kSWaves];
-  // Each wave stages a group's V rows here for the transposing reads of P.V.
-  __shared__ __attribute__((aligned(16))) half_t sm_v[kSWaves][16 * VROW];
+  // Segment states a wave leaves for the merge: slot 0 (its first partial
+  // segment) and slot 1 (a later one, always its last).  Rows of OROW floats
+  // per head, padded against bank conflicts.  Until its stream ends a wave
+  // stages a group's V rows in its slot 1, for the transposing reads of P.V.
+  constexpr int OROW = D + 4;
+  constexpr int SEG = GT * OROW;
+  constexpr int SEG1 = SEG * 4 > 16 * VROW * 2 ? SEG : 16 * VROW / 2;
+  __shared__ __attribute__((aligned(16))) float sm_seg0[kSWaves][SEG];
+  __shared__ __attribute__((aligned(16))) float sm_seg1[kSWaves][SEG1];
+  __shared__ float4_t sm_ml[kSWaves][2][GT];  // max, fp16-P normaliser, fp32 normaliser, -
+  __shared__ int sm_unit[kSWaves][2];         // unit of each slot (-1: unused)
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -104,13 +137,16 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   const uint32_t kOnes = 0x3c003c00u;  // half2(1, 1)
   const int gw = (int)blockIdx.x * kSWaves + wave;
   const int W = p.W;
-  const int N = p.N;
-  // Wave w's range starts at floor(w N / W): no range is empty while W <= N.
-  // With more waves than groups, waves 0 .. N - 1 take one group each and the
-  // rest none, so that no empty wave lies inside a unit's run of waves (every
-  // wave of that run stores a partial and counts it).
+  // Wave w's range starts at w (N / W) + floor(w f), f = (N % W) / W in 20-bit
+  // fixed point: W <= N, so no wave below W is empty, and waves from W on have
+  // none.  (The long ranges are spread evenly on purpose: with the N % W
+  // longer ones all in the first workgroups, those held 3% more and a
+  // 115096-token launch took 3% longer; an exact floor(w N / W) costs each
+  // wave a chain of divisions before its first load.)
+  const int wq = p.wq;
+  const uint32_t wf20 = p.wf20;
   auto wstart = [&](int w) __attribute__((always_inline)) -> int {
-    return W <= N ? (int)(((int64_t)w * N) / W) : min(w, N);
+    return w >= W ? p.N : w * wq + (int)(((uint32_t)w * wf20) >> 20);  // w < 4096
   };
   const int g0 = wstart(gw);
   const int n = wstart(gw + 1) - g0;  // groups of this wave
@@ -273,11 +309,27 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     }
   };
 
+  // Four normalised output values of row `row` at dims d0 .. d0 + 3.
+  auto store_o4 = [&](half_t* o, int64_t row, int d0, float4_t O, float inv)
+                      __attribute__((always_inline)) {
+    half4_t hv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) hv[r] = (half_t)(O[r] * inv);
+    *reinterpret_cast<half4_t*>(o + row * D + d0) = hv;
+  };
+  auto store_lse = [&](float* lse, int64_t row, float M, float E) __attribute__((always_inline)) {
+    if (lse) lse[row] = E > 0.f ? (M + log2f(E)) * kLn2 : AKT_SNEG_INF;
+  };
+
   // ---- prologue ----------------------------------------------------------------
   // The first PD groups' page ids, then group 0's K and V, need only the
   // kernel arguments: they go out before the sequence table is built (its
   // barriers wait for LDS only).  The table gives the groups' sequences, hence
   // their q fragments and last-page lengths.
+  if (lane < 2) {
+    sm_unit[wave][lane] = -1;
+    if (wave == 0) sm_fin[lane] = -1;
+  }
   if (PAIRED && lane == 0)
     __hip_atomic_store(&sm_prog[wave], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   int y0 = 0, pp0 = 0, slice0 = 0;
@@ -332,14 +384,14 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   }
 
   // Sequences without pages have no groups: o = 0 and lse = -inf here.
-  for (int bb = gw; bb < p.B; bb += W) {
+  for (int bb = gw; bb < p.B; bb += (int)gridDim.x * kSWaves) {
     if (sm_s[bb] != sm_s[bb + 1]) continue;
     half_t* orow = p.o + (int64_t)bb * p.Hq * D;
     for (int i = lane; i < p.Hq * (D / 8); i += 64) st16(orow + 8 * i, uint4_t{0, 0, 0, 0});
     if (p.lse)
       for (int h = lane; h < p.Hq; h += 64) p.lse[(int64_t)bb * p.Hq + h] = AKT_SNEG_INF;
   }
-  if (n <= 0) return;  // wave-uniform; no barrier follows
+  if (n > 0) {  // wave-uniform
 
   // Sequences of groups 0 .. PD-1 (their last-page lengths are loaded into
   // pll), then the lookahead from group PD on.  Group 0's q
@@ -377,17 +429,9 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   float4_t acc[NT];
   int cur_b = -1, cur_y = 0;
   // Unit bookkeeping (wave-uniform): unit id y * B + b (the units' order on
-  // the axis, so that wave + unit, the partial slot, is unique: a later wave
-  // never holds an earlier unit), heads, covering waves.
-  int cu_unit = 0, cu_hq0 = 0, cu_nh = 0, cu_wf = 0, cu_nc = 1;
-  // Partial segments to count at the end (at most the first and the last).
-  int pa_unit = -1, pa_b = 0, pa_hq0 = 0, pa_nh = 0, pa_wf = 0, pa_nc = 0;
-  int pb_unit = -1, pb_b = 0, pb_hq0 = 0, pb_nh = 0, pb_wf = 0, pb_nc = 0;
-
-  // The wave whose range holds group g (the last w with wstart(w) <= g).
-  auto wave_of = [&](int g) __attribute__((always_inline)) -> int {
-    return W <= N ? (int)(((int64_t)(g + 1) * W - 1) / N) : g;
-  };
+  // the axis), first head, heads, whether the unit lies inside this wave.
+  int cu_unit = 0, cu_hq0 = 0, cu_nh = 0, cu_direct = 0;
+  int n_seg = 0;  // partial segments left in LDS so far
 
   auto begin_unit = [&](int b, int y) __attribute__((always_inline)) {
     m_run = AKT_SNEG_INF;
@@ -395,16 +439,14 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     e_part = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-    const int kvh = p.n_hg == 1 ? y : y / p.n_hg;
-    const int hg = y - kvh * p.n_hg;
-    cu_hq0 = kvh * p.G + hg * GT;
-    cu_nh = min(GT, p.G - hg * GT);
-    cu_unit = y * p.B + b;  // axis order: slot = wave + unit is then unique
+    const StreamArgs p = reread_args();
+    const int kvh = p->n_hg == 1 ? y : y / p->n_hg;
+    const int hg = y - kvh * p->n_hg;
+    cu_hq0 = kvh * p->G + hg * GT;
+    cu_nh = min(GT, p->G - hg * GT);
+    cu_unit = y * p->B + b;
     const int s0 = uniform(sm_s[b]), s1 = uniform(sm_s[b + 1]);
-    const int first = y * p.TG + s0 * p.gpp;
-    const int last = y * p.TG + s1 * p.gpp - 1;
-    cu_wf = wave_of(first);
-    cu_nc = wave_of(last) - cu_wf + 1;
+    cu_direct = y * p->TG + s0 * p->gpp >= g0 && y * p->TG + s1 * p->gpp <= g0 + n;
   };
 
   // Scores, online softmax and P.V of one loaded group.  Tokens past the
@@ -415,7 +457,7 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   //   from the staged rows with ds_read_b64_tr_b16 (lane (R, c) gets tokens
   //   4R .. 4R+3 of dim 16t + c), B = P^T straight from the score lanes
   //   (lane (R, c) holds head c's probabilities of tokens 4R .. 4R+3).
-  half_t* const vst = &sm_v[wave][0];
+  half_t* const vst = reinterpret_cast<half_t*>(&sm_seg1[wave][0]);
   auto consume = [&](const Buf& bf, int nv) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < VTOK; ++i)
@@ -467,58 +509,33 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
       acc[tt] = __builtin_amdgcn_mfma_f32_16x16x16f16(va[tt], pb, acc[tt], 0, 0, 0);
   };
 
-  // Four normalised output values of row `row` at dims d0 .. d0 + 3.
-  auto store_o4 = [&](int64_t row, int d0, float4_t O, float inv) __attribute__((always_inline)) {
-    half4_t hv;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) hv[r] = (half_t)(O[r] * inv);
-    *reinterpret_cast<half4_t*>(p.o + row * D + d0) = hv;
-  };
-  auto store_lse = [&](int64_t row, float M, float E) __attribute__((always_inline)) {
-    if (p.lse) p.lse[row] = E > 0.f ? (M + log2f(E)) * kLn2 : AKT_SNEG_INF;
-  };
-
   // End of the current unit's segment: wave reduction, then the output (a
-  // unit wholly inside this wave) or a partial at slot gw + unit.
+  // unit wholly inside this wave) or the segment's state in LDS.
   auto flush = [&]() __attribute__((always_inline)) {
     // Lane (R, c16) holds head c16's dims 16t + 4R + r: only the normalisers
     // are summed over the four rows.
     const float l_w = rows_sum(l_part);
     const float e_w = rows_sum(e_part);
-    const bool direct = cu_nc == 1;
-    const int64_t slot = (int64_t)gw + cu_unit;
-    if (c16 < cu_nh) {
-      if (direct) {
-        const int64_t row = (int64_t)cur_b * p.Hq + cu_hq0 + c16;
+    if (cu_direct) {
+      const StreamArgs a = reread_args();
+      if (c16 < cu_nh) {
+        const int64_t row = (int64_t)cur_b * a->Hq + cu_hq0 + c16;
         const float inv = l_w > 0.f ? 1.0f / l_w : 0.f;
 #pragma unroll
-        for (int tt = 0; tt < NT; ++tt) store_o4(row, 16 * tt + 4 * R, acc[tt], inv);
-        if (R == 0) store_lse(row, m_run, e_w);
-      } else {
-        const int64_t ph = slot * GT + c16;
+        for (int tt = 0; tt < NT; ++tt) store_o4(a->o, row, 16 * tt + 4 * R, acc[tt], inv);
+        if (R == 0) store_lse(a->lse, row, m_run, e_w);
+      }
+    } else {
+      float* seg = n_seg == 0 ? &sm_seg0[wave][0] : &sm_seg1[wave][0];
+      if (c16 < cu_nh) {
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt)
-          st16_device(p.part_o, (uint32_t)((ph * D + 16 * tt + 4 * R) * 4), as_uint4f(acc[tt]));
-        if (R == 0)
-          st16_device(p.part_ml, (uint32_t)(ph * 16), as_uint4f(float4_t{m_run, l_w, e_w, 0.f}));
+          *reinterpret_cast<uint4_t*>(seg + c16 * OROW + 16 * tt + 4 * R) = as_uint4f(acc[tt]);
+        if (R == 0) sm_ml[wave][n_seg][c16] = float4_t{m_run, l_w, e_w, 0.f};
       }
+      if (lane == 0) sm_unit[wave][n_seg] = cu_unit;
+      n_seg = 1;  // a second partial segment is the wave's last
     }
-    // Value selects (a branch between the two sets makes the compiler select
-    // between their addresses, on the stack).
-    const bool to_a = !direct && pa_unit < 0;
-    const bool to_b = !direct && !to_a;
-    pa_b = to_a ? cur_b : pa_b;
-    pa_hq0 = to_a ? cu_hq0 : pa_hq0;
-    pa_nh = to_a ? cu_nh : pa_nh;
-    pa_wf = to_a ? cu_wf : pa_wf;
-    pa_nc = to_a ? cu_nc : pa_nc;
-    pa_unit = to_a ? cu_unit : pa_unit;
-    pb_b = to_b ? cur_b : pb_b;
-    pb_hq0 = to_b ? cu_hq0 : pb_hq0;
-    pb_nh = to_b ? cu_nh : pb_nh;
-    pb_wf = to_b ? cu_wf : pb_wf;
-    pb_nc = to_b ? cu_nc : pb_nc;
-    pb_unit = to_b ? cu_unit : pb_unit;
   };
 
   // ---- stream the range, PD groups in flight --------------------------------
@@ -566,77 +583,183 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     }
   }
 
-  // ---- count the partials; the last arrival merges its unit -----------------
-  if (pa_unit < 0) return;
-  // Every partial store of this wave (device scope) is complete before any
-  // count; the merging wave reads the partials with device-scope loads.
-  __builtin_amdgcn_s_waitcnt(0);
-  // Merge layout: lane l owns NVL consecutive float4 vectors of the unit's
-  // output (vectors l*NVL .. l*NVL + NVL - 1), all of one head (64 is a
-  // multiple of GT), so it needs one (m, l, e) row per partial; U partials
-  // are loaded per round trip.
+  }  // n > 0
+
+  // ---- merge ------------------------------------------------------------------
+  // Layout of a merging wave: lane l owns NVL consecutive float4 vectors of the
+  // unit's output (vectors l*NVL .. l*NVL + NVL - 1), all of one head (64 is a
+  // multiple of GT), so it needs one (m, l, e) row per state; U states are
+  // loaded per round trip.
+  const StreamArgs a = reread_args();
   constexpr int NV = GT * D / 4;               // float4 vectors of a unit's output
   constexpr int NVL = NV >= 64 ? NV / 64 : 1;  // per lane
   constexpr int U = 32 / (NVL + 1) > 0 ? 32 / (NVL + 1) : 1;
-  // Counts of both partials, issued before either result is awaited.
-  int prev_a = 0, prev_b = 0;
-  if (lane == 0) {
-    prev_a = atomicAdd(&p.arrive[pa_unit], 1);
-    if (pb_unit >= 0) prev_b = atomicAdd(&p.arrive[pb_unit], 1);
-  }
-  const bool last_a = __builtin_amdgcn_readfirstlane(prev_a) == pa_nc - 1;
-  const bool last_b = pb_unit >= 0 && __builtin_amdgcn_readfirstlane(prev_b) == pb_nc - 1;
-  // The wave that counted a unit's last partial resets its counter and merges
-  // the unit's partials in wave order.
-  auto merge = [&](int unit, int b, int hq0, int nh, int wf, int nc) __attribute__((always_inline)) {
-    if (lane == 0) atomicExch(&p.arrive[unit], 0);
-    const int vec0 = (NV < 64 ? min(lane, NV - 1) : lane * NVL);
-    const int h = (vec0 * 4) / D;
-    const int d0 = vec0 * 4 - h * D;
-    float M = AKT_SNEG_INF, L = 0.f, E = 0.f;
-    float4_t Acc[NVL];
+  const int vec0 = NV < 64 ? min(lane, NV - 1) : lane * NVL;
+  const bool has_vec = NV >= 64 || lane < NV;
+  const int mh = (vec0 * 4) / D;
+  const int md = vec0 * 4 - mh * D;
+  float M, L, E;
+  float4_t Acc[NVL];
+  auto merge_begin = [&]() __attribute__((always_inline)) {
+    M = AKT_SNEG_INF;
+    L = E = 0.f;
 #pragma unroll
     for (int i = 0; i < NVL; ++i) Acc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < nc; c0 += U) {
-      float4_t ml[U], ov[U][NVL];
+  };
+  // Adds one state (its ml row and this lane's vectors).
+  auto merge_add = [&](float4_t ml, const float4_t (&ov)[NVL]) __attribute__((always_inline)) {
+    const float m = ml[0];
+    if (m == AKT_SNEG_INF) return;
+    if (m > M) {
+      const float sc = fast_exp2(M - m);  // 0 while M = -inf (Acc, L, E are 0 then)
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int c = min(c0 + u, nc - 1);
-        const int64_t ph = ((int64_t)wf + c + unit) * GT + h;
-        ml[u] = as_float4u(ld16_device(p.part_ml, (uint32_t)(ph * 16)));
-#pragma unroll
-        for (int i = 0; i < NVL; ++i)
-          ov[u][i] = as_float4u(ld16_device(p.part_o, (uint32_t)((ph * D + d0 + 4 * i) * 4)));
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float m = ml[u][0];
-        if (c0 + u >= nc || m == AKT_SNEG_INF) continue;
-        if (m > M) {
-          const float s = fast_exp2(M - m);  // 0 while M = -inf (Acc, L, E are 0 then)
-#pragma unroll
-          for (int i = 0; i < NVL; ++i) Acc[i] *= s;
-          L *= s;
-          E *= s;
-          M = m;
-        }
-        const float f = fast_exp2(m - M);
-#pragma unroll
-        for (int i = 0; i < NVL; ++i) Acc[i] += f * ov[u][i];
-        L += f * ml[u][1];
-        E += f * ml[u][2];
-      }
+      for (int i = 0; i < NVL; ++i) Acc[i] *= sc;
+      L *= sc;
+      E *= sc;
+      M = m;
     }
-    if ((NV >= 64 || lane < NV) && h < nh) {
-      const int64_t row = (int64_t)b * p.Hq + hq0 + h;
+    const float f = fast_exp2(m - M);
+#pragma unroll
+    for (int i = 0; i < NVL; ++i) Acc[i] += f * ov[i];
+    L += f * ml[1];
+    E += f * ml[2];
+  };
+  auto merge_lds = [&](const float* seg, float4_t ml) __attribute__((always_inline)) {
+    float4_t ov[NVL];
+#pragma unroll
+    for (int i = 0; i < NVL; ++i)
+      ov[i] = as_float4u(*reinterpret_cast<const uint4_t*>(seg + mh * OROW + md + 4 * i));
+    merge_add(ml, ov);
+  };
+  // The unit's place: head group y, sequence b, groups [first, last] of the axis.
+  auto unit_place = [&](int unit, int& y, int& b, int& first, int& last)
+                        __attribute__((always_inline)) {
+    y = unit / a->B;
+    b = unit - y * a->B;
+    first = y * a->TG + uniform(sm_s[b]) * a->gpp;
+    last = y * a->TG + uniform(sm_s[b + 1]) * a->gpp - 1;
+  };
+  auto merge_out = [&](int y, int b) __attribute__((always_inline)) {
+    const int kvh = a->n_hg == 1 ? y : y / a->n_hg;
+    const int hg = y - kvh * a->n_hg;
+    if (has_vec && mh < min(GT, a->G - hg * GT)) {
+      const int64_t row = (int64_t)b * a->Hq + kvh * a->G + hg * GT + mh;
       const float inv = L > 0.f ? 1.0f / L : 0.f;
 #pragma unroll
-      for (int i = 0; i < NVL; ++i) store_o4(row, d0 + 4 * i, Acc[i], inv);
-      if (d0 == 0) store_lse(row, M, E);
+      for (int i = 0; i < NVL; ++i) store_o4(a->o, row, md + 4 * i, Acc[i], inv);
+      if (md == 0) store_lse(a->lse, row, M, E);
     }
   };
-  if (last_a) merge(pa_unit, pa_b, pa_hq0, pa_nh, pa_wf, pa_nc);
-  if (last_b) merge(pb_unit, pb_b, pb_hq0, pb_nh, pb_wf, pb_nc);
+  auto mstart = [&](int w) __attribute__((always_inline)) -> int {
+    return w >= a->W ? a->N : w * a->wq + (int)(((uint32_t)w * a->wf20) >> 20);
+  };
+  // The wave whose range holds group g: the float estimate is off by at most
+  // one (W <= 4096, 24-bit products), and the range starts settle it.
+  auto wave_of = [&](int g) __attribute__((always_inline)) -> int {
+    int w = min((int)((float)g * a->w_per_g), a->W - 1);
+    while (w > 0 && mstart(w) > g) --w;
+    while (mstart(w + 1) <= g) ++w;
+    return w;
+  };
+  // Partials c0, c0 + step, ... (U of them, clamped to the last) of a unit
+  // whose run starts at workgroup wf.
+  auto load_partials = [&](int unit, int wf, int c0, int step, int nc, float4_t (&ml)[U],
+                           float4_t (&ov)[U][NVL]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = min(c0 + u * step, nc - 1);
+      const int64_t ph = ((int64_t)wf + c + unit) * GT + mh;
+      ml[u] = as_float4u(ld16_device(a->part_ml, (uint32_t)(ph * 16)));
+#pragma unroll
+      for (int i = 0; i < NVL; ++i)
+        ov[u][i] = as_float4u(ld16_device(a->part_o, (uint32_t)((ph * D + md + 4 * i) * 4)));
+    }
+  };
+  const int wave0 = (int)blockIdx.x * kSWaves;
+  const int wg0 = mstart(wave0), wg1 = mstart(wave0 + kSWaves);  // the workgroup's groups
+
+  __syncthreads();  // every wave's segments are in LDS
+  // Each unit's segments are combined by the wave that holds the unit's first
+  // one in this workgroup; the waves after it hold theirs in slot 0 (a unit
+  // that began before a wave's range is that wave's first segment).
+#pragma unroll
+  for (int sl = 0; sl < 2; ++sl) {
+    const int unit = uniform(sm_unit[wave][sl]);
+    if (unit < 0) continue;
+    int y, b, first, last;
+    unit_place(unit, y, b, first, last);
+    if (wave > 0 && first < mstart(wave0 + wave)) continue;  // an earlier wave's
+    const int wl = wave_of(last) - wave0;
+    merge_begin();
+    merge_lds(sl == 0 ? &sm_seg0[wave][0] : &sm_seg1[wave][0], sm_ml[wave][sl][mh]);
+    for (int w = wave + 1; w <= min(wl, kSWaves - 1); ++w)
+      merge_lds(&sm_seg0[w][0], sm_ml[w][0][mh]);
+    if (first >= wg0 && last < wg1) {
+      merge_out(y, b);
+      continue;
+    }
+    // A partial of the workgroup, at slot workgroup + unit (both grow along the
+    // axis, so no two partials share a slot).
+    if (has_vec) {
+      const int64_t ph = ((int64_t)blockIdx.x + unit) * GT + mh;
+#pragma unroll
+      for (int i = 0; i < NVL; ++i)
+        st16_device(a->part_o, (uint32_t)((ph * D + md + 4 * i) * 4), as_uint4f(Acc[i]));
+      if (md == 0) st16_device(a->part_ml, (uint32_t)(ph * 16), as_uint4f(float4_t{M, L, E, 0.f}));
+    }
+    // The stores (device scope) are complete before the count.
+    __builtin_amdgcn_s_waitcnt(0);
+    const int nc = wave_of(last) / kSWaves - wave_of(first) / kSWaves + 1;
+    int prev = 0;
+    if (lane == 0) prev = atomicAdd(&a->arrive[unit], 1);
+    if (uniform(prev) != nc - 1) continue;
+    if (lane == 0) atomicExch(&a->arrive[unit], 0);
+    if (nc > U) {
+      if (lane == 0) sm_fin[first < wg0 ? 0 : 1] = unit;
+      continue;
+    }
+    // One round trip's worth: merged here, without the workgroup's barriers.
+    float4_t ml[U], ov[U][NVL];
+    load_partials(unit, wave_of(first) / kSWaves, 0, 1, nc, ml, ov);
+    merge_begin();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < nc) merge_add(ml[u], ov[u]);
+    merge_out(y, b);
+  }
+  __syncthreads();
+  // Longer units whose last partial this workgroup counted: wave v takes partials v,
+  // v + kSWaves, ... of the unit's run, then one wave combines the waves.
+#pragma unroll 1
+  for (int k = 0; k < 2; ++k) {
+    const int unit = uniform(sm_fin[k]);
+    if (unit < 0) continue;  // workgroup-uniform
+    int y, b, first, last;
+    unit_place(unit, y, b, first, last);
+    const int wf = wave_of(first) / kSWaves;
+    const int nc = wave_of(last) / kSWaves - wf + 1;
+    merge_begin();
+    for (int c0 = wave; c0 < nc; c0 += U * kSWaves) {
+      float4_t ml[U], ov[U][NVL];
+      load_partials(unit, wf, c0, kSWaves, nc, ml, ov);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c0 + u * kSWaves < nc) merge_add(ml[u], ov[u]);
+    }
+    if (has_vec) {
+#pragma unroll
+      for (int i = 0; i < NVL; ++i)
+        *reinterpret_cast<uint4_t*>(&sm_seg0[wave][mh * OROW + md + 4 * i]) = as_uint4f(Acc[i]);
+      if (md == 0) sm_ml[wave][0][mh] = float4_t{M, L, E, 0.f};
+    }
+    __syncthreads();
+    if (wave == 0) {
+      merge_begin();
+      for (int w = 0; w < min(nc, kSWaves); ++w) merge_lds(&sm_seg0[w][0], sm_ml[w][0][mh]);
+      merge_out(y, b);
+    }
+    __syncthreads();  // the buffers are reused by the second unit
+  }
 }
 
 // Launches instance (D, GT) on the resident workgroups (two per CU at
@@ -674,7 +797,10 @@ int launch_stream_t(StreamParams p, hipStream_t st) {
   int64_t blocks = wave_cap_t<D, GT>() / waves;
   const int64_t want = ceil_div(p.N > 0 ? p.N : 1, waves);
   if (blocks > want) blocks = want;
-  p.W = (int)(blocks * waves);
+  p.W = (int)std::max<int64_t>(1, std::min<int64_t>(blocks * waves, p.N));
+  p.wq = p.N / p.W;
+  p.wf20 = (uint32_t)(((int64_t)(p.N % p.W) << 20) / p.W);
+  p.w_per_g = p.N > 0 ? (float)p.W / (float)p.N : 0.f;
   KernelTimer timer;
   timer.launch(kernel, dim3((unsigned)blocks), dim3(threads), 0, st, p);
   return check_launch("paged_stream_kernel");

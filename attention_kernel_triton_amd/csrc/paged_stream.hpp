@@ -10,8 +10,8 @@ namespace akt {
 
 // Largest batch whose sequence table fits the kernel's LDS.
 constexpr int kStreamMaxBatch = 1024;
-// Most waves a launch uses.  A wave stores its partial of unit u at slot
-// wave + u, so a launch needs (its waves + units) partial slots.
+// Most waves a launch uses.  A workgroup stores its partial of unit u at slot
+// workgroup + u; the workspace is sized for one slot per wave and unit.
 constexpr int kStreamMaxWaves = 4096;
 
 struct StreamParams {
@@ -24,8 +24,8 @@ struct StreamParams {
   half_t* o;      // [B, Hq, D] contiguous
   float* lse;     // [B, Hq] or null
   int* arrive;    // [B * Y] arrival counters (zero between launches)
-  float* part_o;  // [waves + B * Y, GT, D]
-  float* part_ml; // [waves + B * Y, GT, 4]: max, fp16-P normaliser, fp32 normaliser, pad
+  float* part_o;  // [workgroups + B * Y, GT, D]
+  float* part_ml; // [workgroups + B * Y, GT, 4]: max, fp16-P normaliser, fp32 normaliser, pad
   int64_t q_sb, q_sh;
   int64_t k_sa, k_head, v_sa, v_head;  // page and kv-head strides (elements)
   int k_sb, v_sb;                      // row strides (elements, < 2^26)
@@ -34,7 +34,11 @@ struct StreamParams {
   int total_pages;
   int TG;              // groups per head group: total_pages * gpp
   int N;               // groups of the launch: Y * TG (< 2^31)
-  int W;               // waves of the launch (set by paged_stream_launch)
+  // Set by paged_stream_launch: waves with groups (at most N), N / W, the
+  // fraction (N % W) / W in 20-bit fixed point, W / N.
+  int W, wq;
+  uint32_t wf20;
+  float w_per_g;
   int num_pool_pages;
   float qk_scale;      // softmax_scale * log2(e)
 };

@@ -399,3 +399,25 @@ def test_decode_more_units_than_the_fixed_arrival_area(dev):
     assert torch.equal(full, torch.cat(parts))
     ro, _ = naive.decode(q[:100].cpu(), K[:100].cpu(), V[:100].cpu(), 0.125, 1)
     assert_close(parts[0], ro, what="first slice")
+
+
+# Long units: a unit's run covers a few workgroups (merged by one wave in one
+# round trip) up to more than a round trip holds (merged by a workgroup), with
+# unit starts inside and at the edges of a workgroup's range, for every head
+# count a unit can have and both workgroup sizes.
+@pytest.mark.parametrize("lens", [[30001], [16 * 8 * 40], [9000, 1, 700, 16 * 8 * 33, 40],
+                                  [128] * 40 + [5000]])
+@pytest.mark.parametrize("G,D", [(1, 128), (3, 128), (8, 128), (16, 128), (4, 64), (4, 256)])
+def test_paged_units_over_many_workgroups(dev, lens, G, D):
+    from attention_kernel_triton_amd import _ops
+    g = torch.Generator().manual_seed(sum(lens) + 10 * G + D)
+    indptr, indices, last, P = syn.block_table(g, lens, 16)
+    pool = torch.randn(P, 2, 1, 16, D, generator=g).half()
+    q = torch.randn(len(lens), G, 1, D, generator=g).half()
+    args = (q.to(dev), pool.to(dev), indptr.to(dev), indices.to(dev), last.to(dev))
+    o, lse = _ops.decode_paged(*args, return_lse=True)
+    ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)
+    assert_close(o, ro, what=f"G={G} D={D}")
+    assert_close(lse, rl, atol=1e-4, what="lse")
+    again = _ops.decode_paged(*args, return_lse=True)
+    assert torch.equal(again[0], o) and torch.equal(again[1], lse)
