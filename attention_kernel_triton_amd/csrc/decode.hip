@@ -1358,6 +1358,27 @@ int check_common(int64_t B, int64_t Hq, int64_t Hkv, int64_t D) {
 using namespace akt;
 
 // ----------------------------- dense decode --------------------------------
+// The stream-K kernel (paged_stream.hip) serves the automatic chunk length;
+// explicit chunk lengths, small launches and the few shapes it cannot address
+// keep the chunked split kernel (k_row, v_row: row strides; the workspace size does not
+// know them and covers both kernels).
+static bool dense_stream(int D, int64_t chunk_tokens, int64_t batch, int64_t seq_len, int64_t Y,
+                         int64_t k_row, int64_t v_row) {
+  return chunk_tokens == 0 && dense_stream_eligible(D, batch, seq_len, Y, k_row, v_row);
+}
+
+static WsLayout dense_split_layout(int64_t batch, int64_t Y, int gt, int64_t D, int64_t seq_len,
+                                   int64_t chunk_tokens) {
+  const int64_t chunk = chunk_tokens > 0 ? chunk_tokens : auto_chunk(seq_len * batch, Y);
+  const int64_t nch = ceil_div(seq_len, chunk);
+  return ws_layout(batch * Y, nch > 1 ? batch * Y * nch : 0, gt, D);
+}
+
+static WsLayout dense_stream_layout(int64_t batch, int64_t Y, int gt, int64_t D,
+                                    int64_t seq_len) {
+  return ws_layout(0, dense_stream_parts((int)D, gt, batch * Y, ceil_div(seq_len, 16)), gt, D);
+}
+
 extern "C" size_t akt_decode_workspace_size(int64_t batch, int64_t num_q_heads,
                                             int64_t num_kv_heads, int64_t seq_len,
                                             int64_t head_dim, int64_t chunk_tokens) {
@@ -1365,9 +1386,10 @@ extern "C" size_t akt_decode_workspace_size(int64_t batch, int64_t num_q_heads,
   const int G = (int)(num_q_heads / num_kv_heads);
   const int gt = pick_gt(G, (int)head_dim);
   const int64_t Y = num_kv_heads * ceil_div(G, gt);
-  const int64_t chunk = chunk_tokens > 0 ? chunk_tokens : auto_chunk(seq_len * batch, Y);
-  const int64_t nch = ceil_div(seq_len, chunk);
-  return ws_layout(batch * Y, nch > 1 ? batch * Y * nch : 0, gt, head_dim).total;
+  const WsLayout split = dense_split_layout(batch, Y, gt, head_dim, seq_len, chunk_tokens);
+  if (!dense_stream((int)head_dim, chunk_tokens, batch, seq_len, Y, 0, 0)) return split.total;
+  const WsLayout stream = dense_stream_layout(batch, Y, gt, head_dim, seq_len);
+  return split.fits && split.total > stream.total ? split.total : stream.total;
 }
 
 extern "C" int akt_decode_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -1391,12 +1413,39 @@ extern "C" int akt_decode_fwd(const void* q, const void* k, const void* v, void*
   const int gt = pick_gt(G, D);
   const int n_hg = (int)ceil_div(G, gt);
   const int64_t Y = num_kv_heads * n_hg;
-  const int64_t chunk = chunk_tokens > 0 ? chunk_tokens : auto_chunk(seq_len * batch, Y);
-  const int64_t nch = ceil_div(seq_len, chunk);
-  const WsLayout wl = ws_layout(batch * Y, nch > 1 ? batch * Y * nch : 0, gt, D);
+  const bool use_stream = dense_stream(D, chunk_tokens, batch, seq_len, Y, k_stride[2], v_stride[2]);
+  const WsLayout wl = use_stream
+                          ? dense_stream_layout(batch, Y, gt, D, seq_len)
+                          : dense_split_layout(batch, Y, gt, D, seq_len, chunk_tokens);
   rc = check_workspace(wl, workspace, workspace_bytes);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
+  if (use_stream) {
+    StreamParams sp = {};
+    sp.q = (const half_t*)q;
+    sp.kbase = (const half_t*)k;
+    sp.vbase = (const half_t*)v;
+    sp.o = (half_t*)o;
+    sp.lse = lse;
+    char* c = (char*)workspace;
+    sp.arrive = (int*)(c + wl.arrive);
+    sp.part_o = (float*)(c + wl.part_o);
+    sp.part_ml = (float*)(c + wl.part_ml);
+    sp.q_sb = q_stride[0];
+    sp.q_sh = q_stride[1];
+    sp.k_sa = k_stride[0]; sp.k_head = k_stride[1]; sp.k_sb = (int)k_stride[2];
+    sp.v_sa = v_stride[0]; sp.v_head = v_stride[1]; sp.v_sb = (int)v_stride[2];
+    sp.B = (int)batch; sp.Hq = (int)num_q_heads; sp.G = G; sp.Y = (int)Y; sp.n_hg = n_hg;
+    sp.S = (int)seq_len;
+    sp.gpp = (int)ceil_div(seq_len, 16);
+    sp.total_pages = (int)batch;
+    sp.TG = sp.total_pages * sp.gpp;
+    sp.N = (int)(Y * sp.TG);
+    sp.qk_scale = softmax_scale * kLog2e;
+    return dense_stream_launch(sp, D, gt, st);
+  }
+  const int64_t chunk = chunk_tokens > 0 ? chunk_tokens : auto_chunk(seq_len * batch, Y);
+  const int64_t nch = ceil_div(seq_len, chunk);
   if (nch == 0) {  // empty cache: every row is o = 0, lse = -inf
     const int64_t rows = batch * num_q_heads;
     hipLaunchKernelGGL(empty_rows_kernel, dim3((unsigned)ceil_div(rows * (D / 8), kThreads)),
@@ -1513,10 +1562,6 @@ int paged_decode_impl(const void* q, const void* kv_cache, const int32_t* kv_pag
     sp.N = (int)(Y * sp.TG);
     sp.num_pool_pages = (int)(num_pool_pages < (1ll << 31) ? num_pool_pages : (1ll << 31) - 1);
     sp.qk_scale = softmax_scale * kLog2e;
-    SplitParams cp = {};
-    cp.arrive = sp.arrive;
-    rc = clear_extra_arrivals(cp, wl, st);
-    if (rc) return rc;
     return paged_stream_launch(sp, D, gt, st);
   }
   const int64_t chunk = paged_chunk(chunk_tokens, total_pages, page_size, Y, batch);

@@ -1,5 +1,12 @@
-// Stream-K paged var-len decode for gfx950 (the automatic-chunk path of
-// decode_flash_attention_redundant_var_len_paged.py:70-224).
+// Stream-K decode for gfx950: the automatic-chunk path of the paged var-len
+// decode (decode_flash_attention_redundant_var_len_paged.py:70-224) and of the
+// dense one (decode_flash_attention_redundant.py:71-229).
+//
+// A dense cache is a paged one whose sequence b is one page, page b of
+// ceil(S / 16) groups: its DENSE instances read no table and, in the last
+// group, no row past S.  (Against the split kernel's tickets, workgroup merge
+// per chunk and P.V on the VALU: B=32, Hq=64, Hkv=8, S=4100, D=128 119.9 ->
+// 94.4 us, 5.7 TB/s; B=8, Hq=64, Hkv=16, S=1024, D=64 14.4 -> 11.5 us.)
 //
 // Work decomposition.  A "unit" is one (sequence b, head group y): the up to
 // GT query heads of one kv head that read the same K/V rows.  Every unit's
@@ -49,6 +56,9 @@ namespace {
 
 #define AKT_SNEG_INF (-__builtin_inff())
 
+// Compute units of MI355X: the workgroups assumed where no device can be queried.
+constexpr int64_t kCUs = 256;
+
 // The kernel's arguments, re-read from the kernel-argument segment (the opaque
 // pointer keeps the compiler from reusing, and so holding, earlier reads): what
 // only the unit boundaries and the merge use would otherwise take scalar
@@ -58,6 +68,26 @@ __device__ __forceinline__ StreamArgs reread_args() {
   StreamArgs a = (StreamArgs)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(a));
   return a;
+}
+
+// First group of wave w's range (WAVES to a workgroup).
+// - Stream-K: w (N / W) + floor(w f), f = (N % W) / W in 20-bit fixed point:
+//   W <= N, so no wave below W is empty, and waves from W on have none.  (The
+//   long ranges are spread evenly on purpose: with the N % W longer ones all
+//   in the first workgroups, those held 3% more and a 115096-token launch took
+//   3% longer; an exact floor(w N / W) costs each wave a chain of divisions
+//   before its first load.)
+// - Whole units (DENSE, wgs_log >= 0): 2^wgs_log workgroups to a unit, the
+//   unit's groups shared evenly by their waves (one each while they last, in
+//   a single workgroup, for a unit with fewer groups than waves).
+template <bool DENSE, int WAVES, typename P>
+__device__ __forceinline__ int wave_start(const P& p, int w) {
+  if (DENSE && p.wgs_log >= 0) {
+    const int s = p.wgs_log + (WAVES == 8 ? 3 : 2);
+    const int u = w >> s, j = w & ((1 << s) - 1);
+    return u * p.gpp + (p.gpp < (1 << s) ? min(j, p.gpp) : (int)(((int64_t)j * p.gpp) >> s));
+  }
+  return w >= p.W ? p.N : w * p.wq + (int)(((uint32_t)w * p.wf20) >> 20);  // w < 4096
 }
 
 // Last index i in [0, n] with s[i] <= x, given a non-decreasing s[0..n];
@@ -94,11 +124,12 @@ constexpr int stream_depth() {
   return 2;
 }
 
-template <int D, int GT>
+template <int D, int GT, bool DENSE>
 __global__ __launch_bounds__((stream_threads<D, GT>()))
 __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_stream_kernel(
     StreamParams p) {
   constexpr int PD = stream_depth<D, GT>();
+  constexpr int kTable = DENSE ? 1 : kStreamMaxBatch;  // sequences of the LDS table
   constexpr int kSThreads = stream_threads<D, GT>();
   constexpr int kSWaves = kSThreads / kWave;
   constexpr bool PAIRED = kSWaves == 8;
@@ -112,7 +143,7 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   // Sequence page ranges: sequence b owns positions [sm_s[b], sm_s[b + 1]) of
   // kv_page_indices (indptr clamped to [0, total_pages] and made
   // non-decreasing).
-  __shared__ int sm_s[kStreamMaxBatch + 1];
+  __shared__ int sm_s[kTable + 1];
   __shared__ int sm_wmax[kSWaves];
   __shared__ int sm_fin[2];  // units whose last partial this workgroup counted (-1: none)
   // Groups each wave has consumed (paired waves only).
@@ -136,20 +167,8 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   const int c16 = lane & 15;
   const uint32_t kOnes = 0x3c003c00u;  // half2(1, 1)
   const int gw = (int)blockIdx.x * kSWaves + wave;
-  const int W = p.W;
-  // Wave w's range starts at w (N / W) + floor(w f), f = (N % W) / W in 20-bit
-  // fixed point: W <= N, so no wave below W is empty, and waves from W on have
-  // none.  (The long ranges are spread evenly on purpose: with the N % W
-  // longer ones all in the first workgroups, those held 3% more and a
-  // 115096-token launch took 3% longer; an exact floor(w N / W) costs each
-  // wave a chain of divisions before its first load.)
-  const int wq = p.wq;
-  const uint32_t wf20 = p.wf20;
-  auto wstart = [&](int w) __attribute__((always_inline)) -> int {
-    return w >= W ? p.N : w * wq + (int)(((uint32_t)w * wf20) >> 20);  // w < 4096
-  };
-  const int g0 = wstart(gw);
-  const int n = wstart(gw + 1) - g0;  // groups of this wave
+  const int g0 = wave_start<DENSE, kSWaves>(p, gw);
+  const int n = wave_start<DENSE, kSWaves>(p, gw + 1) - g0;  // groups of this wave
 
   // Axis position of group g: head group y, page position pp, 16-row slice.
   auto locate = [&](int g, int& y, int& pp, int& slice) __attribute__((always_inline)) {
@@ -177,6 +196,10 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   auto seq_end = [&](int b) __attribute__((always_inline)) -> int {
     return b < p.B ? uniform(sm_s[b + 1]) : INT32_MAX;
   };
+  // First position of sequence b (a dense cache: position b, one each).
+  auto seq_start = [&](int b) __attribute__((always_inline)) -> int {
+    return DENSE ? b : uniform(sm_s[b]);
+  };
   // One group forward; `track`: keep la_b / la_end (the table exists).
   auto advance = [&](bool track) __attribute__((always_inline)) {
     if (++la_slice < p.gpp) return;
@@ -185,9 +208,9 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
       la_pp = 0;
       ++la_y;
       la_b = -1;
-      if (track) la_end = uniform(sm_s[0]);
+      if (!DENSE && track) la_end = uniform(sm_s[0]);
     }
-    if (track)
+    if (!DENSE && track)
       while (la_b < p.B && la_pp >= la_end) la_end = seq_end(++la_b);
   };
   // Sequence of position pp from the table (the last b with start <= pp).
@@ -202,6 +225,14 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     int b, y, slot, last;
   };
   auto fetch = [&](Fetch& f) __attribute__((always_inline)) {
+    if constexpr (DENSE) {
+      f.page = f.b = la_pp;
+      f.y = la_y;
+      f.slot = la_slice * 16;
+      f.last = 1;
+      advance(true);
+      return;
+    }
     f.page = __builtin_amdgcn_raw_buffer_load_b32(idx_rsrc, (uint32_t)la_pp * 4u, 0, 0);
     const bool seq_ok = la_b >= 0 && la_b < p.B;
     const int lb = min(max(la_b, 0), p.B - 1);
@@ -254,8 +285,10 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   // repeat head hq0: each column's scores, softmax and P.V stay in that
   // column's lanes, and those lanes store nothing.  (Zeroing them would make
   // the compiler wait for the loads right where they are issued.)  b < 0 (no
-  // unit) reads sequence 0's rows, so that every group issues the same loads.
+  // unit; y may then lie past the last head group) reads sequence 0's first
+  // rows, so that every group issues the same loads.
   auto load_q = [&](int b, int y, half8_t (&qd)[KS]) __attribute__((always_inline)) {
+    y = b < 0 ? 0 : y;
     b = max(b, 0);
     const int kvh = p.n_hg == 1 ? y : y / p.n_hg;
     const int hg = y - kvh * p.n_hg;
@@ -280,22 +313,26 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   Fetch fr[PD];
   auto issue = [&](int j, Buf& bf, bool seq, Fetch& f, bool take_ll)
                    __attribute__((always_inline)) {
-    const int page = uniform(f.page);
+    const int page = DENSE ? f.page : uniform(f.page);
     const int y = f.y, slot = f.slot;
     bf.b = j < n ? f.b : -1;
     bf.y = y;
     bf.slot = slot;
     bf.last = f.last;
-    const bool use = j < n && page >= 0 && page < p.num_pool_pages;
+    const bool use = j < n && (DENSE || (page >= 0 && page < p.num_pool_pages));
     bf.use = use;
-    if (take_ll) set_usable(bf, f.ll);
+    if constexpr (DENSE) bf.nv = use ? min(p.S - slot, 16) : 0;
+    else if (take_ll) set_usable(bf, f.ll);
+    // A dense cache ends with its last row: lanes of rows past it re-read it.
+    const int row_max = DENSE ? max(bf.nv - 1, 0) : 15;
     if (seq) fetch(f);
     if (seq) load_q(bf.b, y, bf.q);
     const int kvh = p.n_hg == 1 ? y : y / p.n_hg;
     const char* kg = reinterpret_cast<const char*>(
         use ? p.kbase + (int64_t)kvh * p.k_head + (int64_t)page * p.k_sa + (int64_t)slot * p.k_sb
             : p.q);
-    const uint32_t ko = use ? lane_kofs : lane_qofs;
+    uint32_t ko = use ? lane_kofs : lane_qofs;
+    if (DENSE && row_max < 15 && use) ko = (uint32_t)(min(c16, row_max) * p.k_sb + 8 * R) * 2u;
 #pragma unroll
     for (int s = 0; s < KS; ++s) bf.k[s] = ld16(kg + ko + 64 * s);
     const char* vg = reinterpret_cast<const char*>(
@@ -303,7 +340,8 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
             : p.q);
 #pragma unroll
     for (int i = 0; i < VTOK; ++i) {
-      const uint32_t vo = use ? lane_v0ofs + (uint32_t)i * vstep : lane_dofs;
+      uint32_t vo = use ? lane_v0ofs + (uint32_t)i * vstep : lane_dofs;
+      if (DENSE && row_max < 15 && use) vo = (uint32_t)(min(tt0 + i, row_max) * p.v_sb + dim0) * 2u;
 #pragma unroll
       for (int jj = 0; jj < VLD; ++jj) bf.v[i][jj] = ld16(vg + vo + 16 * jj);
     }
@@ -337,89 +375,98 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   la_y = y0;
   la_pp = pp0;
   la_slice = slice0;
-#pragma unroll
-  for (int i = 0; i < PD; ++i) {
-    fr[i].page = __builtin_amdgcn_raw_buffer_load_b32(idx_rsrc, (uint32_t)la_pp * 4u, 0, 0);
-    fr[i].y = la_y;
-    fr[i].slot = la_slice * 16;
-    fr[i].b = -1;
-    fr[i].last = 0;
-    fr[i].ll = 0;
-    advance(false);
-  }
-  constexpr int ENT = (kStreamMaxBatch + 1 + kSThreads - 1) / kSThreads;  // table entries per thread
-  int tv[ENT];
-#pragma unroll
-  for (int j = 0; j < ENT; ++j) {
-    const int e = ENT * tid + j;
-    tv[j] = e <= p.B ? min(max(p.indptr[e], 0), p.total_pages) : 0;
-  }
   Buf bufs[PD];
-  if (n > 0) issue(0, bufs[0], false, fr[0], false);
-  // Sequence table: indptr clamped to [0, total_pages] and made
-  // non-decreasing (a max-scan).
-  {
+  if constexpr (!DENSE) {
 #pragma unroll
-    for (int j = 1; j < ENT; ++j) tv[j] = max(tv[j], tv[j - 1]);
-    int incl = tv[ENT - 1];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int t = __shfl_up(incl, off, 64);
-      if (lane >= off) incl = max(incl, t);
+    for (int i = 0; i < PD; ++i) {
+      fr[i].page = __builtin_amdgcn_raw_buffer_load_b32(idx_rsrc, (uint32_t)la_pp * 4u, 0, 0);
+      fr[i].y = la_y;
+      fr[i].slot = la_slice * 16;
+      fr[i].b = -1;
+      fr[i].last = 0;
+      fr[i].ll = 0;
+      advance(false);
     }
-    if (lane == 63) sm_wmax[wave] = incl;
-    __syncthreads();
-    int before = 0;
-#pragma unroll
-    for (int w = 0; w < kSWaves; ++w)
-      if (w < wave) before = max(before, sm_wmax[w]);
-    const int up = __shfl_up(incl, 1, 64);
-    const int excl = lane > 0 ? max(before, up) : before;
+    constexpr int ENT = (kStreamMaxBatch + 1 + kSThreads - 1) / kSThreads;  // table entries per thread
+    int tv[ENT];
 #pragma unroll
     for (int j = 0; j < ENT; ++j) {
       const int e = ENT * tid + j;
-      if (e <= p.B) sm_s[e] = max(excl, tv[j]);
+      tv[j] = e <= p.B ? min(max(p.indptr[e], 0), p.total_pages) : 0;
     }
-    __syncthreads();
-  }
+    if (n > 0) issue(0, bufs[0], false, fr[0], false);
+    // Sequence table: indptr clamped to [0, total_pages] and made
+    // non-decreasing (a max-scan).
+    {
+#pragma unroll
+      for (int j = 1; j < ENT; ++j) tv[j] = max(tv[j], tv[j - 1]);
+      int incl = tv[ENT - 1];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(incl, off, 64);
+        if (lane >= off) incl = max(incl, t);
+      }
+      if (lane == 63) sm_wmax[wave] = incl;
+      __syncthreads();
+      int before = 0;
+#pragma unroll
+      for (int w = 0; w < kSWaves; ++w)
+        if (w < wave) before = max(before, sm_wmax[w]);
+      const int up = __shfl_up(incl, 1, 64);
+      const int excl = lane > 0 ? max(before, up) : before;
+#pragma unroll
+      for (int j = 0; j < ENT; ++j) {
+        const int e = ENT * tid + j;
+        if (e <= p.B) sm_s[e] = max(excl, tv[j]);
+      }
+      __syncthreads();
+    }
 
-  // Sequences without pages have no groups: o = 0 and lse = -inf here.
-  for (int bb = gw; bb < p.B; bb += (int)gridDim.x * kSWaves) {
-    if (sm_s[bb] != sm_s[bb + 1]) continue;
-    half_t* orow = p.o + (int64_t)bb * p.Hq * D;
-    for (int i = lane; i < p.Hq * (D / 8); i += 64) st16(orow + 8 * i, uint4_t{0, 0, 0, 0});
-    if (p.lse)
-      for (int h = lane; h < p.Hq; h += 64) p.lse[(int64_t)bb * p.Hq + h] = AKT_SNEG_INF;
+    // Sequences without pages have no groups: o = 0 and lse = -inf here.
+    for (int bb = gw; bb < p.B; bb += (int)gridDim.x * kSWaves) {
+      if (sm_s[bb] != sm_s[bb + 1]) continue;
+      half_t* orow = p.o + (int64_t)bb * p.Hq * D;
+      for (int i = lane; i < p.Hq * (D / 8); i += 64) st16(orow + 8 * i, uint4_t{0, 0, 0, 0});
+      if (p.lse)
+        for (int h = lane; h < p.Hq; h += 64) p.lse[(int64_t)bb * p.Hq + h] = AKT_SNEG_INF;
+    }
   }
   if (n > 0) {  // wave-uniform
 
-  // Sequences of groups 0 .. PD-1 (their last-page lengths are loaded into
-  // pll), then the lookahead from group PD on.  Group 0's q
-  // fragment, group PD's fetch, then groups 1 .. PD-1: each buffer's loads in
-  // the order of the main loop's, so that the compiler's wait counts at the
-  // loop's entry match those of its iterations.
-  la_y = y0;
-  la_pp = pp0;
-  la_slice = slice0;
-  seek(pp0);
-  int pll[PD];
+  if constexpr (DENSE) {
 #pragma unroll
-  for (int i = 0; i < PD; ++i) {
-    const bool seq_ok = la_b >= 0 && la_b < p.B;
-    fr[i].b = seq_ok ? la_b : -1;
-    fr[i].last = seq_ok && la_pp == la_end - 1;
-    const int lb = min(max(la_b, 0), p.B - 1);
-    pll[i] = __builtin_amdgcn_raw_buffer_load_b32(ll_rsrc, (uint32_t)lb * 4u, 0, 0);
-    advance(true);
+    for (int i = 0; i < PD; ++i) fetch(fr[i]);
+#pragma unroll
+    for (int i = 0; i < PD; ++i) issue(i, bufs[i], true, fr[i], true);
+  } else {
+    // Sequences of groups 0 .. PD-1 (their last-page lengths are loaded into
+    // pll), then the lookahead from group PD on.  Group 0's q
+    // fragment, group PD's fetch, then groups 1 .. PD-1: each buffer's loads in
+    // the order of the main loop's, so that the compiler's wait counts at the
+    // loop's entry match those of its iterations.
+    la_y = y0;
+    la_pp = pp0;
+    la_slice = slice0;
+    seek(pp0);
+    int pll[PD];
+#pragma unroll
+    for (int i = 0; i < PD; ++i) {
+      const bool seq_ok = la_b >= 0 && la_b < p.B;
+      fr[i].b = seq_ok ? la_b : -1;
+      fr[i].last = seq_ok && la_pp == la_end - 1;
+      const int lb = min(max(la_b, 0), p.B - 1);
+      pll[i] = __builtin_amdgcn_raw_buffer_load_b32(ll_rsrc, (uint32_t)lb * 4u, 0, 0);
+      advance(true);
+    }
+    bufs[0].b = fr[0].b;
+    bufs[0].last = fr[0].last;
+    load_q(bufs[0].b, bufs[0].y, bufs[0].q);
+    fetch(fr[0]);
+#pragma unroll
+    for (int i = 1; i < PD; ++i) issue(i, bufs[i], true, fr[i], false);
+#pragma unroll
+    for (int i = 0; i < PD; ++i) set_usable(bufs[i], pll[i]);
   }
-  bufs[0].b = fr[0].b;
-  bufs[0].last = fr[0].last;
-  load_q(bufs[0].b, bufs[0].y, bufs[0].q);
-  fetch(fr[0]);
-#pragma unroll
-  for (int i = 1; i < PD; ++i) issue(i, bufs[i], true, fr[i], false);
-#pragma unroll
-  for (int i = 0; i < PD; ++i) set_usable(bufs[i], pll[i]);
 
   // ---- state of the unit being streamed ------------------------------------
   float m_run = AKT_SNEG_INF;  // running max of head c16 (log2 units)
@@ -445,7 +492,7 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     cu_hq0 = kvh * p->G + hg * GT;
     cu_nh = min(GT, p->G - hg * GT);
     cu_unit = y * p->B + b;
-    const int s0 = uniform(sm_s[b]), s1 = uniform(sm_s[b + 1]);
+    const int s0 = seq_start(b), s1 = seq_start(b + 1);
     cu_direct = y * p->TG + s0 * p->gpp >= g0 && y * p->TG + s1 * p->gpp <= g0 + n;
   };
 
@@ -636,8 +683,8 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
                         __attribute__((always_inline)) {
     y = unit / a->B;
     b = unit - y * a->B;
-    first = y * a->TG + uniform(sm_s[b]) * a->gpp;
-    last = y * a->TG + uniform(sm_s[b + 1]) * a->gpp - 1;
+    first = y * a->TG + seq_start(b) * a->gpp;
+    last = y * a->TG + seq_start(b + 1) * a->gpp - 1;
   };
   auto merge_out = [&](int y, int b) __attribute__((always_inline)) {
     const int kvh = a->n_hg == 1 ? y : y / a->n_hg;
@@ -651,24 +698,42 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     }
   };
   auto mstart = [&](int w) __attribute__((always_inline)) -> int {
-    return w >= a->W ? a->N : w * a->wq + (int)(((uint32_t)w * a->wf20) >> 20);
+    return wave_start<DENSE, kSWaves>(*a, w);
   };
-  // The wave whose range holds group g: the float estimate is off by at most
-  // one (W <= 4096, 24-bit products), and the range starts settle it.
-  auto wave_of = [&](int g) __attribute__((always_inline)) -> int {
-    int w = min((int)((float)g * a->w_per_g), a->W - 1);
-    while (w > 0 && mstart(w) > g) --w;
-    while (mstart(w + 1) <= g) ++w;
-    return w;
+  // The workgroups [wf, wf + nc) whose ranges hold the unit's groups.
+  auto unit_run = [&](int unit, int first, int last, int& wf, int& nc)
+                      __attribute__((always_inline)) {
+    if (DENSE && a->wgs_log >= 0) {
+      nc = 1 << a->wgs_log;
+      wf = unit << a->wgs_log;
+      return;
+    }
+    // The wave whose range holds group g: the float estimate is off by at most
+    // one (W <= 4096, 24-bit products), and the range starts settle it.
+    auto wave_of = [&](int g) __attribute__((always_inline)) -> int {
+      int w = min((int)((float)g * a->w_per_g), a->W - 1);
+      while (w > 0 && mstart(w) > g) --w;
+      while (mstart(w + 1) <= g) ++w;
+      return w;
+    };
+    wf = wave_of(first) / kSWaves;
+    nc = wave_of(last) / kSWaves - wf + 1;
+  };
+  // Partial slots of a unit whose run starts in workgroup wf: workgroup w's is
+  // w + min(wf, unit), both of which grow along the axis, the second by at
+  // least one from a unit to the next that shares a workgroup with it, so no
+  // two partials share a slot (whole units: w itself).
+  auto first_slot = [&](int unit, int wf) __attribute__((always_inline)) -> int {
+    return DENSE && a->wgs_log >= 0 ? wf : wf + min(wf, unit);
   };
   // Partials c0, c0 + step, ... (U of them, clamped to the last) of a unit
-  // whose run starts at workgroup wf.
-  auto load_partials = [&](int unit, int wf, int c0, int step, int nc, float4_t (&ml)[U],
+  // whose slots start at slot0.
+  auto load_partials = [&](int slot0, int c0, int step, int nc, float4_t (&ml)[U],
                            float4_t (&ov)[U][NVL]) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = min(c0 + u * step, nc - 1);
-      const int64_t ph = ((int64_t)wf + c + unit) * GT + mh;
+      const int64_t ph = ((int64_t)slot0 + c) * GT + mh;
       ml[u] = as_float4u(ld16_device(a->part_ml, (uint32_t)(ph * 16)));
 #pragma unroll
       for (int i = 0; i < NVL; ++i)
@@ -689,38 +754,39 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     int y, b, first, last;
     unit_place(unit, y, b, first, last);
     if (wave > 0 && first < mstart(wave0 + wave)) continue;  // an earlier wave's
-    const int wl = wave_of(last) - wave0;
     merge_begin();
     merge_lds(sl == 0 ? &sm_seg0[wave][0] : &sm_seg1[wave][0], sm_ml[wave][sl][mh]);
-    for (int w = wave + 1; w <= min(wl, kSWaves - 1); ++w)
+    for (int w = wave + 1; w < kSWaves && uniform(sm_unit[w][0]) == unit; ++w)
       merge_lds(&sm_seg0[w][0], sm_ml[w][0][mh]);
     if (first >= wg0 && last < wg1) {
       merge_out(y, b);
       continue;
     }
-    // A partial of the workgroup, at slot workgroup + unit (both grow along the
-    // axis, so no two partials share a slot).
+    // A partial of the workgroup.
+    int wf, nc;
+    unit_run(unit, first, last, wf, nc);
+    const int slot0 = first_slot(unit, wf);
     if (has_vec) {
-      const int64_t ph = ((int64_t)blockIdx.x + unit) * GT + mh;
+      const int64_t ph = ((int64_t)slot0 + (int)blockIdx.x - wf) * GT + mh;
 #pragma unroll
       for (int i = 0; i < NVL; ++i)
         st16_device(a->part_o, (uint32_t)((ph * D + md + 4 * i) * 4), as_uint4f(Acc[i]));
       if (md == 0) st16_device(a->part_ml, (uint32_t)(ph * 16), as_uint4f(float4_t{M, L, E, 0.f}));
     }
-    // The stores (device scope) are complete before the count.
+    // The stores (device scope) are complete before the count.  Only one unit
+    // reaches out of a workgroup's end, so wf names the unit's counter.
     __builtin_amdgcn_s_waitcnt(0);
-    const int nc = wave_of(last) / kSWaves - wave_of(first) / kSWaves + 1;
     int prev = 0;
-    if (lane == 0) prev = atomicAdd(&a->arrive[unit], 1);
+    if (lane == 0) prev = atomicAdd(&a->arrive[wf], 1);
     if (uniform(prev) != nc - 1) continue;
-    if (lane == 0) atomicExch(&a->arrive[unit], 0);
+    if (lane == 0) atomicExch(&a->arrive[wf], 0);
     if (nc > U) {
       if (lane == 0) sm_fin[first < wg0 ? 0 : 1] = unit;
       continue;
     }
     // One round trip's worth: merged here, without the workgroup's barriers.
     float4_t ml[U], ov[U][NVL];
-    load_partials(unit, wave_of(first) / kSWaves, 0, 1, nc, ml, ov);
+    load_partials(slot0, 0, 1, nc, ml, ov);
     merge_begin();
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -736,12 +802,13 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
     if (unit < 0) continue;  // workgroup-uniform
     int y, b, first, last;
     unit_place(unit, y, b, first, last);
-    const int wf = wave_of(first) / kSWaves;
-    const int nc = wave_of(last) / kSWaves - wf + 1;
+    int wf, nc;
+    unit_run(unit, first, last, wf, nc);
+    const int slot0 = first_slot(unit, wf);
     merge_begin();
     for (int c0 = wave; c0 < nc; c0 += U * kSWaves) {
       float4_t ml[U], ov[U][NVL];
-      load_partials(unit, wf, c0, kSWaves, nc, ml, ov);
+      load_partials(slot0, c0, kSWaves, nc, ml, ov);
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (c0 + u * kSWaves < nc) merge_add(ml[u], ov[u]);
@@ -762,62 +829,83 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   }
 }
 
-// Launches instance (D, GT) on the resident workgroups (two per CU at
-// D <= 128 with up to 4 heads per unit), at most kStreamMaxWaves waves and no
-// more waves than groups.
-template <int D, int GT>
-int64_t wave_cap_t() {
-  constexpr int waves = stream_threads<D, GT>() / kWave;
-  const int cap = resident_blocks(paged_stream_kernel<D, GT>, stream_threads<D, GT>());
-  if (cap <= 0) return kStreamMaxWaves;
-  return (int64_t)cap * waves < kStreamMaxWaves ? (int64_t)cap * waves : kStreamMaxWaves;
-}
+// Waves of a launch of instance (D, GT, DENSE) over N groups on `blocks`
+// workgroups, and each wave's share.
+template <int D, int GT, bool DENSE>
+struct Stream {
+  static constexpr int kThreads = stream_threads<D, GT>();
+  static constexpr int kWaves = kThreads / kWave;
 
-template <int D>
-int64_t wave_cap_gt(int gt) {
-  switch (gt) {
-    case 1: return wave_cap_t<D, 1>();
-    case 2: return wave_cap_t<D, 2>();
-    case 4: return wave_cap_t<D, 4>();
-    case 8: return wave_cap_t<D, 8>();
-    case 16:
-      if constexpr (D != 256) return wave_cap_t<D, 16>();
-      break;
+  // Workgroups resident at once (at most kStreamMaxWaves waves); `unknown`
+  // where no device can be queried.
+  static int64_t blocks(int64_t unknown) {
+    const int64_t cap = resident_blocks(paged_stream_kernel<D, GT, DENSE>, kThreads);
+    return cap <= 0 ? unknown : std::min<int64_t>(cap, kStreamMaxWaves / kWaves);
   }
-  return kStreamMaxWaves;
-}
+  static int64_t wave_cap() { return blocks(kStreamMaxWaves / kWaves) * kWaves; }
 
-template <int D, int GT>
-int launch_stream_t(StreamParams p, hipStream_t st) {
-  auto kernel = paged_stream_kernel<D, GT>;
-  constexpr int threads = stream_threads<D, GT>();
-  constexpr int waves = threads / kWave;
-  if (resident_blocks(kernel, threads) <= 0)
-    return set_error(AKT_ERR_HIP, "occupancy query failed");
-  int64_t blocks = wave_cap_t<D, GT>() / waves;
-  const int64_t want = ceil_div(p.N > 0 ? p.N : 1, waves);
-  if (blocks > want) blocks = want;
-  p.W = (int)std::max<int64_t>(1, std::min<int64_t>(blocks * waves, p.N));
-  p.wq = p.N / p.W;
-  p.wf20 = (uint32_t)(((int64_t)(p.N % p.W) << 20) / p.W);
-  p.w_per_g = p.N > 0 ? (float)p.W / (float)p.N : 0.f;
-  KernelTimer timer;
-  timer.launch(kernel, dim3((unsigned)blocks), dim3(threads), 0, st, p);
-  return check_launch("paged_stream_kernel");
-}
-
-template <int D>
-int launch_stream_gt(int gt, const StreamParams& p, hipStream_t st) {
-  switch (gt) {
-    case 1: return launch_stream_t<D, 1>(p, st);
-    case 2: return launch_stream_t<D, 2>(p, st);
-    case 4: return launch_stream_t<D, 4>(p, st);
-    case 8: return launch_stream_t<D, 8>(p, st);
-    case 16:
-      if constexpr (D != 256) return launch_stream_t<D, 16>(p, st);
-      break;
+  static int64_t grid(int64_t N) {
+    return std::max<int64_t>(1, std::min(blocks(kCUs), ceil_div(N, kWaves)));
   }
-  return set_error(AKT_ERR_UNSUPPORTED, "no paged decode kernel for %d heads per unit", gt);
+  // Workgroups per unit of a dense launch as a power of two (whole units: no
+  // unit straddles a workgroup's end), or -1 for stream-K ranges.  The most
+  // workgroups per unit that stay resident at once, if they fill the device, or
+  // fill three quarters of it and a wave has at most 8 groups (balance matters
+  // less than the shorter merge then).  Measured (us, whole units / stream-K):
+  // D = 64, 128 units of 64 groups 10.6 / 11.0, 52 of 44 8.9 / 9.4; D = 128
+  // 17.2 / 17.6, 10.7 / 11.0; D = 256 26.8 / 27.1, 13.5 / 14.7.
+  static int dense_wgs_log(int64_t units, int64_t unit_groups) {
+    const int64_t most = blocks(kCUs);
+    if (units > most) return -1;
+    int k = 0;
+    while ((units << (k + 1)) <= most && unit_groups >= ((int64_t)kWaves << (k + 1))) ++k;
+    const int64_t used = units << k;
+    const bool even = used == most || (4 * used >= 3 * most && unit_groups <= ((int64_t)kWaves << (k + 3)));
+    return even ? k : -1;
+  }
+  static int64_t dense_grid(int64_t units, int64_t unit_groups, int wgs_log) {
+    return wgs_log >= 0 ? units << wgs_log : grid(units * unit_groups);
+  }
+  // Partial slots of a dense launch (first_slot in the kernel).
+  static int64_t dense_parts(int64_t units, int64_t unit_groups) {
+    const int k = dense_wgs_log(units, unit_groups);
+    const int64_t g = dense_grid(units, unit_groups, k);
+    return k >= 0 ? g : g + std::min(units, g);
+  }
+
+  static int launch(StreamParams p, hipStream_t st) {
+    auto kernel = paged_stream_kernel<D, GT, DENSE>;
+    if (resident_blocks(kernel, kThreads) <= 0)
+      return set_error(AKT_ERR_HIP, "occupancy query failed");
+    p.wgs_log = DENSE ? dense_wgs_log((int64_t)p.Y * p.B, p.gpp) : -1;
+    const int64_t g = DENSE ? dense_grid((int64_t)p.Y * p.B, p.gpp, p.wgs_log) : grid(p.N);
+    p.W = (int)std::max<int64_t>(1, std::min<int64_t>(g * kWaves, p.N));
+    p.wq = p.N / p.W;
+    p.wf20 = (uint32_t)(((int64_t)(p.N % p.W) << 20) / p.W);
+    p.w_per_g = p.N > 0 ? (float)p.W / (float)p.N : 0.f;
+    KernelTimer timer;
+    timer.launch(kernel, dim3((unsigned)g), dim3(kThreads), 0, st, p);
+    return check_launch("paged_stream_kernel");
+  }
+};
+
+// Calls f with the instance for head dim D and gt heads per unit (both checked
+// by the callers; D = 256 units hold at most 8 heads).
+template <bool DENSE, int D, typename F>
+auto with_gt(int gt, F f) {
+  switch (gt) {
+    case 1: return f(Stream<D, 1, DENSE>());
+    case 2: return f(Stream<D, 2, DENSE>());
+    case 4: return f(Stream<D, 4, DENSE>());
+    case 8: return f(Stream<D, 8, DENSE>());
+  }
+  return f(Stream<D, D == 256 ? 8 : 16, DENSE>());
+}
+template <bool DENSE, typename F>
+auto with_instance(int D, int gt, F f) {
+  if (D == 64) return with_gt<DENSE, 64>(gt, f);
+  if (D == 128) return with_gt<DENSE, 128>(gt, f);
+  return with_gt<DENSE, 256>(gt, f);
 }
 
 }  // namespace
@@ -828,21 +916,36 @@ bool paged_stream_eligible(int64_t batch, int64_t page_size, int64_t total_pages
 }
 
 int64_t paged_stream_wave_cap(int D, int gt) {
-  switch (D) {
-    case 64: return wave_cap_gt<64>(gt);
-    case 128: return wave_cap_gt<128>(gt);
-    case 256: return wave_cap_gt<256>(gt);
-  }
-  return kStreamMaxWaves;
+  return with_instance<false>(D, gt, [](auto s) { return s.wave_cap(); });
 }
 
-int paged_stream_launch(StreamParams p, int D, int gt, hipStream_t st) {
-  switch (D) {
-    case 64: return launch_stream_gt<64>(gt, p, st);
-    case 128: return launch_stream_gt<128>(gt, p, st);
-    case 256: return launch_stream_gt<256>(gt, p, st);
-  }
-  return set_error(AKT_ERR_UNSUPPORTED, "head_dim %d not supported (64, 128, 256)", D);
+int paged_stream_launch(const StreamParams& p, int D, int gt, hipStream_t st) {
+  return with_instance<false>(D, gt, [&](auto s) { return s.launch(p, st); });
+}
+
+// Small launches keep the chunked split kernel, whose smaller workgroups start
+// and merge sooner: below 4096 groups in all (1024 at D = 64), unless there is
+// a unit for every CU.  Measured (us, this kernel / split): D = 128, N = 504
+// 11.1 / 9.3, 2504 20.0 / 16.8, 2560 in 256 units 9.1 / 10.5, 4864 12.6 / 13.8,
+// 8192 17.2 / 18.3, 64000 91.4 / 99.5 and with 8 heads to a unit 43.5 / 62.0;
+// D = 256, N = 2016 15.8 / 13.9, 4864 18.9 / 19.9; D = 64, N = 504 9.1 / 8.6,
+// 2016 9.3 / 10.0, 8192 10.6 / 14.0.
+bool dense_stream_eligible(int D, int64_t batch, int64_t seq_len, int64_t Y, int64_t k_row,
+                           int64_t v_row) {
+  const int64_t most = (int64_t)1 << 26;
+  if (batch < 1 || seq_len < 1 || k_row < 0 || k_row >= most || v_row < 0 || v_row >= most ||
+      batch >= ((int64_t)1 << 31) / Y / ceil_div(seq_len, 16))
+    return false;
+  const int64_t units = batch * Y, groups = units * ceil_div(seq_len, 16);
+  return groups >= (D == 64 ? 1024 : 4096) || units >= kCUs;
+}
+
+int64_t dense_stream_parts(int D, int gt, int64_t units, int64_t unit_groups) {
+  return with_instance<true>(D, gt, [&](auto s) { return s.dense_parts(units, unit_groups); });
+}
+
+int dense_stream_launch(const StreamParams& p, int D, int gt, hipStream_t st) {
+  return with_instance<true>(D, gt, [&](auto s) { return s.launch(p, st); });
 }
 
 }  // namespace akt

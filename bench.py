@@ -368,7 +368,7 @@ def bench_legs(args):
     d2 = [c2.to(dev) for _ in range(n2)]
     legs["decode_config2"] = _leg(
         "config 2", [lambda d=d: _ops.decode(d.q, d.K, d.V, d.scale) for d in d2], c2.bytes(),
-        "GB/s", "split_kernel<64,4,kModeDense>", args, note=f"inputs rotated over {n2} copies")
+        "GB/s", "paged_stream_kernel<64,4,dense>", args, note=f"inputs rotated over {n2} copies")
     del d2
     torch.cuda.empty_cache()
 

@@ -159,7 +159,9 @@ int akt_merge_states(const void* o_parts, int o_parts_dtype, const float* lse_pa
  *   softmax normaliser of the scaled scores).  head_dim: 64, 128 or 256.
  *   chunk_tokens: split-KV chunk length: 128, 256, 512 or 640 tokens, 0 = automatic
  *   (a hint: pages that do not hold whole 16-token groups, and paged batches
- *   over 1024 sequences, use 256).
+ *   over 1024 sequences, use 256).  Automatic dense calls large enough to gain
+ *   run the stream-K kernel (see akt_decode_paged_fwd); the workspace size then
+ *   depends on the current device.
  */
 size_t akt_decode_workspace_size(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
                                  int64_t seq_len, int64_t head_dim, int64_t chunk_tokens);

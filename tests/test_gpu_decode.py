@@ -421,3 +421,42 @@ def test_paged_units_over_many_workgroups(dev, lens, G, D):
     assert_close(lse, rl, atol=1e-4, what="lse")
     again = _ops.decode_paged(*args, return_lse=True)
     assert torch.equal(again[0], o) and torch.equal(again[1], lse)
+
+
+# The automatic dense path on large enough launches (whole units per workgroup
+# and ranges that cut units), against the oracle and the chunked kernel: every
+# remainder class of a 16-token group, head counts with several units per kv
+# head, layouts with other strides, and rows past S that must not be read into
+# any result.
+@pytest.mark.parametrize("B,Hkv,G,S,D", [
+    (256, 1, 4, 17, 64), (16, 16, 1, 33, 128), (16, 16, 2, 1, 256),   # a workgroup per unit
+    (64, 2, 4, 1029, 64), (64, 2, 3, 1040, 128), (52, 1, 8, 1297, 256),
+    (3, 2, 20, 12001, 64), (7, 8, 8, 1999, 128), (1, 5, 16, 14001, 128), (300, 1, 1, 250, 256),
+])
+@pytest.mark.parametrize("layout", ["contiguous", "padded", "sequence-major"])
+def test_dense_auto_path_layouts_and_edges(dev, B, Hkv, G, S, D, layout):
+    from attention_kernel_triton_amd import _ops
+    g = torch.Generator().manual_seed(S + G)
+    K, V = (torch.randn(B, Hkv, S, D, generator=g).half() for _ in range(2))
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    kd, vd = K.to(dev), V.to(dev)
+    if layout == "padded":  # NaN rows between one sequence's last row and the next one's first
+        def pad(t):
+            big = torch.full((B, Hkv, S + 15, D), float("nan"), dtype=t.dtype, device=dev)
+            big[:, :, :S] = t
+            return big[:, :, :S]
+        kd, vd = pad(kd), pad(vd)
+    elif layout == "sequence-major":
+        kd = kd.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+        vd = vd.permute(2, 1, 0, 3).contiguous().permute(2, 1, 0, 3)
+    scale = 1 / math.sqrt(D)
+    o, lse = _ops.decode(q.to(dev), kd, vd, scale, return_lse=True)
+    oc, lc = _ops.decode(q.to(dev), kd, vd, scale, return_lse=True, chunk_tokens=256)
+    # Two orders of fp32 sums: the fp16 results differ by at most one ulp (|o| < 2: 2^-10).
+    assert_close(o, oc, atol=2 ** -9, what="chunked kernel")
+    assert_close(lse, lc, atol=1e-5 * math.log(S + 2) + 1e-5, what="chunked lse")
+    if layout == "contiguous":
+        kr, vr = (t.repeat_interleave(G, 1).double() for t in (K, V))
+        sc = torch.matmul(q.double(), kr.transpose(2, 3)) * scale
+        assert_close(o, torch.matmul(torch.softmax(sc, -1), vr), what="oracle")
+        assert_close(lse, torch.logsumexp(sc, -1)[..., 0], atol=1e-4, what="oracle lse")
