@@ -38,10 +38,13 @@ COMMON_FLAGS = [
     "-mllvm", "-amdgpu-atomic-optimizer-strategy=None",
 ]
 # Extra flags of single sources.  prefill_wide.hip holds the head-dim 192 and 256
-# prefill instances; LLVM's iterative ILP scheduler runs them 8-12% faster than
-# the default scheduler (it is 1-2% slower for the D = 64 instances in prefill.hip).
+# prefill instances (one wave per SIMD): LLVM's iterative ILP scheduler runs them
+# 8-12% faster than the default one (1-2% slower for the D = 64 instances in
+# prefill.hip), and MFMA results selected into VGPRs save the copies between
+# AGPRs and VGPRs (a further 14% with V read a step ahead).
 SOURCE_FLAGS = {
-    "prefill_wide.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+    "prefill_wide.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp",
+                         "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -8,8 +8,7 @@
 //
 // Work decomposition.  A 256-thread workgroup serves one (batch, kv head) and
 // four "slots"; slot f = (query head f % G, row block f / G) of that kv head's
-// G query heads (64-row blocks at D = 64 and in the long-sequence D = 128
-// instance, 32-row blocks otherwise).  With G a multiple of 4 the four waves
+// G query heads (64-row blocks at D = 64, 32-row blocks otherwise).  With G a multiple of 4 the four waves
 // are four query heads at the same rows: they share every staged K/V tile and
 // have identical causal extents.  With 64-row blocks each wave owns its rows
 // as two 32-row MFMA blocks that share every K and V fragment read from LDS
@@ -101,27 +100,24 @@ constexpr int kPThreads = 256;
 constexpr int kSlots = 4;   // waves per workgroup
 constexpr int kNBuf = 4;    // LDS tile buffers
 // 32-row MFMA blocks per wave, query rows per slot, keys per staged tile and
-// waves per SIMD of an instance: two blocks and 64-key tiles at D = 64 (two
-// waves per SIMD in 237 VGPRs); from D = 128 one block and 32-key tiles.  At
-// D = 128 that holds a wave in 210 VGPRs and a workgroup's four K + V buffers
-// in 64 KB, so two waves share each SIMD.  The LONG instance of D = 128 (for
-// sequences of kLongRowsD128 rows or more) takes two blocks and 64-key tiles
-// at one wave per SIMD (registers and AGPRs past 256, 128 KB of LDS): it is
-// 4-6% slower at 1024 rows and 3.5-5% faster from 4096, where each
-// workgroup's longer walk amortises its start.  At D = 192 and 256 the
-// register budget allows one wave per SIMD either way.
-__host__ __device__ constexpr bool two_blocks(int D, bool LONG) {
-  return D == 64 || (D == 128 && LONG);
-}
-__host__ __device__ constexpr int rblocks_for(int D, bool LONG) { return two_blocks(D, LONG) ? 2 : 1; }
-__host__ __device__ constexpr int rows_for(int D, bool LONG) { return 32 * rblocks_for(D, LONG); }
-__host__ __device__ constexpr int tile_keys_for(int D, bool LONG) {
-  return two_blocks(D, LONG) ? 64 : 32;
-}
-__host__ __device__ constexpr int waves_per_simd(int D, bool LONG) {
-  return (D == 64 || (D == 128 && !LONG)) ? 2 : 1;
-}
-constexpr int kLongRowsD128 = 4096;
+// waves per SIMD of an instance: two blocks and 64-key tiles at D = 64, one
+// block and 32-key tiles from D = 128.  Up to D = 128 that holds a wave in 256
+// VGPRs and a workgroup's four K + V buffers in 64 KB, so two waves share each
+// SIMD.  (Two blocks at one wave per SIMD, 128 KB of LDS, were slower at D = 128
+// at every length: 536-578 against 524 us on B=1, Hq=32, Hkv=8, S=8192.)  At
+// D = 192 and 256 the register budget allows one wave per SIMD.
+__host__ __device__ constexpr int rblocks_for(int D) { return D == 64 ? 2 : 1; }
+__host__ __device__ constexpr int rows_for(int D) { return 32 * rblocks_for(D); }
+__host__ __device__ constexpr int tile_keys_for(int D) { return D == 64 ? 64 : 32; }
+__host__ __device__ constexpr int waves_per_simd(int D) { return D <= 128 ? 2 : 1; }
+// Issue order of a step (see step()): its first mix_mfma MFMAs are followed by
+// mix_valu VALU instructions each, the rest is the scheduler's.  Measured (us):
+// D = 128, B=8, Hq=32, Hkv=8, S=1024 / B=1, S=8192: 10 x 1 99.8 / 599, 16 x 1
+// 98.2 / 609, 8 x 2 100.7 / 598, 12 x 2 100.7 / 604; D = 64, B=8, Hq=64,
+// Hkv=16, S=1024: 16 x 2 94.8, 16 x 1 96.0, 12 x 2 96.3, 14 x 3 96.7; D = 192
+// 12 x 2 44.7, 24 x 2 45.9; D = 256 16 x 2 125.5, 32 x 2 127.7, 32 x 3 129.0.
+__host__ __device__ constexpr int mix_mfma(int D) { return D == 64 ? 16 : (D == 128 ? 10 : D / 16); }
+__host__ __device__ constexpr int mix_valu(int D) { return D == 128 ? 1 : 2; }
 constexpr float kRescaleSlack = 8.0f;
 // Largest row sum of one 32-key step that lets P stay unchecked: below it
 // every probability is under 32 * 2^kRescaleSlack, far inside fp16's range;
@@ -216,16 +212,15 @@ __device__ __forceinline__ int div_small(int n, int d, float inv) {
   return q;
 }
 
-template <int D, bool CAUSAL, bool VARLEN, bool BF16, bool LONG>
+template <int D, bool CAUSAL, bool VARLEN, bool BF16>
 __global__ __launch_bounds__(kPThreads)
-__attribute__((amdgpu_waves_per_eu(waves_per_simd(D, LONG), 2)))
+__attribute__((amdgpu_waves_per_eu(waves_per_simd(D), 2)))
 void prefill_kernel(PrefillParams p) {
   typedef Elt<BF16> E;
   typedef typename E::v8 v8;
-  static_assert(!LONG || D == 128, "only D = 128 has a long-sequence instance");
-  constexpr int NRB = rblocks_for(D, LONG);    // 32-row MFMA blocks per wave
-  constexpr int kRows = rows_for(D, LONG);     // query rows per slot
-  constexpr int kBN = tile_keys_for(D, LONG);  // keys per staged tile
+  constexpr int NRB = rblocks_for(D);     // 32-row MFMA blocks per wave
+  constexpr int kRows = rows_for(D);      // query rows per slot
+  constexpr int kBN = tile_keys_for(D);   // keys per staged tile
   constexpr int SPT = kBN / 32;           // 32-key steps per tile
   constexpr int KS = D / 16;              // MFMA k-steps over the head dim
   constexpr int HALF = D / 2;             // head dims per lane half in S^T operands
@@ -235,10 +230,6 @@ void prefill_kernel(PrefillParams p) {
   constexpr int TILEB = kBN * ROWB;       // bytes per K (or V) tile
   constexpr int BUFB = 2 * TILEB;         // bytes per tile buffer (K then V)
   static_assert((kBN * CPR) % kPThreads == 0, "tile split");
-  // D = 64 reads the V fragments of step t + 1 at the end of step t, so P.V
-  // starts without waiting for LDS; at D = 128 they would not fit in the
-  // register budget and are read at the top of their step.
-  constexpr bool kPrefetchV = (D == 64);
 
   __shared__ __attribute__((aligned(16))) char lds[kNBuf * BUFB];
 
@@ -465,11 +456,6 @@ void prefill_kernel(PrefillParams p) {
     load_kf(t, kf);
     qk_mfma(kf, sdst);
   };
-  auto pv = [&](int t, const uint32_t (&pk)[NRB][8]) {
-    v8 vf[2][NT];
-    load_vf(t, vf);
-    pv_mfma(vf, pk);
-  };
   // Probabilities of S(t) against the running max m_run: P rounded to the
   // operand type into pk and, in l_step, each lane's sum of the 16 rounded
   // probabilities it holds: row l32's keys of lane half g (v_dot2 against ones on the VALU, so
@@ -543,25 +529,24 @@ void prefill_kernel(PrefillParams p) {
                   const uint32_t (&pprev)[NRB][8], uint32_t (&pcur)[NRB][8]) {
     mask_step(t, scur);  // S(0) was masked before the loop too: masking is idempotent
     v8 kf[KS];
-    if constexpr (!kPrefetchV) load_vf(t > 0 ? t - 1 : 0, vf);
     load_kf(t + 1, kf);
 
     pv_mfma(vf, pprev);
     qk_mfma(kf, snext);
-    // V of step t, for P.V(t) at the top of step t + 1 (its tile is published).
-    if constexpr (kPrefetchV) load_vf(t, vf);
+    // V of step t, for P.V(t) at the top of step t + 1 (its tile is published):
+    // read a step ahead, so that P.V starts without waiting for LDS.
+    load_vf(t, vf);
 
     float l_step[NRB];
     softmax(scur, pcur, l_step);
-    // Issue order of the region: each P.V / QK MFMA followed by two VALU
-    // instructions, so one wave alternates its matrix and vector work instead
-    // of issuing them in clusters.  Two per MFMA, not more: the wave issues in
-    // order, and a longer VALU run between MFMAs (three) left the matrix pipe
-    // idle at D = 128 (16% slower there, the same at D = 64 and 256).
+    // Issue order of the region: an MFMA, then one or two VALU instructions, so
+    // one wave alternates its matrix and vector work instead of issuing them in
+    // clusters; not more, since the wave issues in order and a longer VALU run
+    // leaves the matrix pipe idle.
 #pragma unroll
-    for (int i = 0; i < (D >= 192 ? 2 * D / 16 : 16); ++i) {
+    for (int i = 0; i < mix_mfma(D); ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // two VALU
+      __builtin_amdgcn_sched_group_barrier(0x002, mix_valu(D), 0);
     }
     bool over = false;
 #pragma unroll
@@ -603,7 +588,7 @@ void prefill_kernel(PrefillParams p) {
   // raise branch.  Every row has a valid key in step 0 (key 0: causal rows
   // are >= 0 and S >= 1), so the start is finite for finite inputs.
   qk(0, sA);
-  if constexpr (kPrefetchV) load_vf(0, vf);  // P.V(-1) of step 0 multiplies P = 0
+  load_vf(0, vf);  // P.V(-1) of step 0 multiplies P = 0
   mask_step(0, sA);
 #pragma unroll
   for (int rb = 0; rb < NRB; ++rb) m_run[rb] = row_max(sA[rb]);
@@ -628,10 +613,7 @@ void prefill_kernel(PrefillParams p) {
     if constexpr (SPT == 1) tile_turn(j + 1);  // n_tiles is even
     if (t < n_h) {
       step(t + 1, sB, sA, pA, pB);
-      if (t + 2 == n_h) {  // drain: P.V(n_h - 1)
-        if constexpr (kPrefetchV) pv_mfma(vf, pB);
-        else pv(t + 1, pB);
-      }
+      if (t + 2 == n_h) pv_mfma(vf, pB);  // drain: P.V(n_h - 1)
     }
   }
 
@@ -687,52 +669,47 @@ void prefill_kernel(PrefillParams p) {
   }
 }
 
-template <int D, bool CAUSAL, bool VARLEN, bool BF16, bool LONG>
+template <int D, bool CAUSAL, bool VARLEN, bool BF16>
 int launch(const PrefillParams& p, dim3 grid, hipStream_t st) {
   KernelTimer timer;
-  timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16, LONG>, grid, dim3(kPThreads), 0, st, p);
+  timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16>, grid, dim3(kPThreads), 0, st, p);
   return check_launch("prefill_kernel");
 }
 
-template <int D, bool BF16, bool LONG>
+template <int D, bool BF16>
 int launch_dt(bool causal, bool varlen, const PrefillParams& p, dim3 grid, hipStream_t st) {
   if (causal)
-    return varlen ? launch<D, true, true, BF16, LONG>(p, grid, st)
-                  : launch<D, true, false, BF16, LONG>(p, grid, st);
-  return varlen ? launch<D, false, true, BF16, LONG>(p, grid, st)
-                : launch<D, false, false, BF16, LONG>(p, grid, st);
+    return varlen ? launch<D, true, true, BF16>(p, grid, st)
+                  : launch<D, true, false, BF16>(p, grid, st);
+  return varlen ? launch<D, false, true, BF16>(p, grid, st)
+                : launch<D, false, false, BF16>(p, grid, st);
 }
 
-template <int D, bool LONG>
-int launch_l(bool bf16, bool causal, bool varlen, const PrefillParams& p, dim3 grid,
-             hipStream_t st) {
-  return bf16 ? launch_dt<D, true, LONG>(causal, varlen, p, grid, st)
-              : launch_dt<D, false, LONG>(causal, varlen, p, grid, st);
-}
-
-// long_rows selects the long-sequence instance (D = 128 only).
 template <int D>
-int launch_d(bool bf16, bool causal, bool varlen, bool long_rows, const PrefillParams& p,
-             dim3 grid, hipStream_t st) {
-  if constexpr (D == 128) {
-    if (long_rows) return launch_l<D, true>(bf16, causal, varlen, p, grid, st);
-  }
-  return launch_l<D, false>(bf16, causal, varlen, p, grid, st);
+int launch_d(bool bf16, bool causal, bool varlen, const PrefillParams& p, dim3 grid,
+             hipStream_t st) {
+  return bf16 ? launch_dt<D, true>(causal, varlen, p, grid, st)
+              : launch_dt<D, false>(causal, varlen, p, grid, st);
 }
 
 }  // namespace
 
 // Head dims 192 and 256 are instantiated in a second translation unit of this
 // file (prefill_wide.hip, AKT_PREFILL_WIDE_TU), which the build compiles with
-// LLVM's iterative ILP machine scheduler: 8-12% faster at those head dims, and
-// 1-2% slower at D = 64, so D = 64 and 128 stay here with the default one.
+// LLVM's iterative ILP machine scheduler (8-12% faster at those head dims, 1-2%
+// slower at D = 64) and with MFMA results selected into VGPRs: past 256
+// registers a wave the compiler otherwise keeps every accumulator in AGPRs and
+// copies the scores out and their zeros in, about 150 moves a step at D = 256,
+// which leave no room to read V a step ahead.  The two together (B=2, Hq=16,
+// Hkv=4, S=1500, D=256, non-causal): 147.5 -> 125.5 us; B=1, Hq=16, Hkv=4,
+// S=8192, causal, D=256 767 -> 646, D=192 575 -> 490.
 int prefill_launch_wide(int head_dim, bool bf16, bool causal, bool varlen, const PrefillParams& p,
                         dim3 grid, hipStream_t st);
 #ifdef AKT_PREFILL_WIDE_TU
 int prefill_launch_wide(int head_dim, bool bf16, bool causal, bool varlen, const PrefillParams& p,
                         dim3 grid, hipStream_t st) {
-  return head_dim == 192 ? launch_d<192>(bf16, causal, varlen, false, p, grid, st)
-                         : launch_d<256>(bf16, causal, varlen, false, p, grid, st);
+  return head_dim == 192 ? launch_d<192>(bf16, causal, varlen, p, grid, st)
+                         : launch_d<256>(bf16, causal, varlen, p, grid, st);
 }
 #endif
 
@@ -795,8 +772,7 @@ int prefill_impl(const void* q, const void* k, const void* v, void* o, float* ls
   p.Hkv = (int)num_kv_heads;
   p.G = (int)(num_q_heads / num_kv_heads);
   p.S = (int)seq_len;
-  const bool long_rows = head_dim == 128 && seq_len >= kLongRowsD128;
-  p.n_rb = (int)ceil_div(seq_len, rows_for((int)head_dim, long_rows));
+  p.n_rb = (int)ceil_div(seq_len, rows_for((int)head_dim));
   p.n_sg = (int)ceil_div((int64_t)p.G * p.n_rb, kSlots);
   p.grid1d = (batch > 65535 || p.n_sg > 65535) ? 1 : 0;
   p.fast_div = ((int64_t)p.G * p.n_rb + kSlots < (1ll << 22)) ? 1 : 0;
@@ -816,8 +792,8 @@ int prefill_impl(const void* q, const void* k, const void* v, void* o, float* ls
   const bool is_var = varlen != nullptr;
   hipStream_t st = (hipStream_t)stream;
   const bool bf16 = dtype == AKT_DTYPE_BF16;
-  if (head_dim == 64) return launch_d<64>(bf16, is_causal, is_var, false, p, grid, st);
-  if (head_dim == 128) return launch_d<128>(bf16, is_causal, is_var, long_rows, p, grid, st);
+  if (head_dim == 64) return launch_d<64>(bf16, is_causal, is_var, p, grid, st);
+  if (head_dim == 128) return launch_d<128>(bf16, is_causal, is_var, p, grid, st);
   return prefill_launch_wide((int)head_dim, bf16, is_causal, is_var, p, grid, st);
 }
 }  // namespace
