@@ -87,6 +87,7 @@ struct PrefillParams {
   int varlen_bits;
   int n_rb;      // query row blocks (slots of one head) per sequence
   int n_sg;      // slot groups (workgroups) per (batch, kv head)
+  int split_keys;  // 1: prefill_split_kernel (small launches)
   int grid1d;    // 1: linear grid (a dimension past 65535); 0: grid (Hkv, B, n_sg)
   int fast_div;  // 1: G * n_rb + kSlots < 2^22, slot / G through g_inv
   float g_inv;   // 1 / G
@@ -669,9 +670,263 @@ void prefill_kernel(PrefillParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small launches: the keys of a row block split over a workgroup's waves.
+//
+// With few heads and rows the kernel above leaves most of the chip idle while
+// its heaviest workgroup walks every key tile in turn.  Here a workgroup serves
+// one query head and one 32-row block, and its kNSplit waves take the 32-key
+// steps t = wave, wave + kNSplit, ...: a quarter of the serial chain and, with
+// G = 4, 4 times the workgroups.  Each wave works alone: K fragments go from
+// global memory straight to registers, V rows through registers to the wave's
+// own LDS region for the transposing reads, each loaded again as soon as the
+// step has consumed it, so that the next step's rows arrive during the softmax
+// and P.V, and no barrier runs before the merge.  The waves' (m, l, O) are then
+// merged through LDS.  K and V are read once per query head and row block from
+// L2, so this pays only while the launch is small (use_split_keys).  Bound by
+// the latency of a step's loads and its serial softmax; B=1, Hq=32, Hkv=8,
+// D=128: S=333 12.4 -> 10.1 us, S=130 8.4 -> 6.4; 8 heads, D=64, S=1024 25.6 ->
+// 8.7; 1 head, S=8192 152 -> 40 (D=64), 288 -> 152 (D=256).
+// ---------------------------------------------------------------------------
+constexpr int kNSplit = 4;
+
+template <int D, bool CAUSAL, bool VARLEN, bool BF16>
+__global__ __launch_bounds__(64 * kNSplit)
+__attribute__((amdgpu_waves_per_eu(waves_per_simd(D), 2)))
+void prefill_split_kernel(PrefillParams p) {
+  typedef Elt<BF16> E;
+  typedef typename E::v8 v8;
+  constexpr int KS = D / 16;        // MFMA k-steps over the head dim
+  constexpr int NT = D / 32;        // 32-dim output tiles
+  constexpr int CPR = D / 8;        // 16-byte chunks per row
+  constexpr int ROWB = D * 2;       // bytes per row
+  constexpr int VPL = CPR / 2;      // V chunks per lane and step
+  constexpr int OB = 32 * D * 4;    // bytes of a wave's O (its staged V takes half of it)
+  __shared__ __attribute__((aligned(16))) char lds[kNSplit * OB];
+  __shared__ float sm_m[kNSplit][32], sm_l[kNSplit][32];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = uniform(tid >> 6);
+  const int l32 = lane & 31;
+  const int g = lane >> 5;
+
+  // Grid (Hkv, B, G * row blocks), heaviest row block first.
+  const int kvh = blockIdx.x, b = blockIdx.y;
+  const int rank = uniform(p.fast_div ? div_small(blockIdx.z, p.G, p.g_inv)
+                                      : (int)blockIdx.z / p.G);
+  const int h = kvh * p.G + (int)blockIdx.z - rank * p.G;
+  const int n_rb = (p.S + 31) / 32;
+  const int r0 = 32 * (CAUSAL ? n_rb - 1 - rank : rank);
+  const int S = p.S;
+  int len = S;
+  if constexpr (VARLEN) {
+    long long lv = (p.varlen_bits == 64) ? ((const long long*)p.varlen)[b]
+                                         : (long long)((const int*)p.varlen)[b];
+    len = uniform((int)(lv < 0 ? 0 : (lv > S ? S : lv)));
+  }
+  const int row_lim = VARLEN ? min(S, ((len + 63) / 64) * 64) : S;
+  if (r0 >= row_lim) return;  // workgroup-uniform
+  const int key_lim = (VARLEN && CAUSAL) ? len : S;  // rows at or past this read as zeros
+  const int n_steps = ((CAUSAL ? min(row_lim, r0 + 32) : S) + 31) / 32;
+
+  const half_t* __restrict__ Qh = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
+  const half_t* __restrict__ Kh = p.k + (int64_t)b * p.k_sb + (int64_t)kvh * p.k_sh;
+  const half_t* __restrict__ Vh = p.v + (int64_t)b * p.v_sb + (int64_t)kvh * p.v_sh;
+
+  // K fragment s of a step: key l32, dims 16 s + 8 g + e.  V chunk i: 16-byte
+  // chunk lane + 64 i of the step's 32 rows.
+  const int kofs = (int)(l32 * p.k_ss * 2) + 16 * g;
+  int vofs[VPL], vdst[VPL];
+  char* const vst = lds + wave * OB;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int q = lane + 64 * i, r = q / CPR, c = q % CPR;
+    vofs[i] = (int)(r * p.v_ss * 2) + 16 * c;
+    vdst[i] = r * ROWB + ((c ^ tswz<D>(r)) * 16);
+  }
+  uint4_t kf[KS], vr[VPL];
+  // Steps past the last one read an empty range (zeros, no memory touched).
+  auto rows_of = [&](int t) { return uniform(t < n_steps ? min(32, key_lim - 32 * t) : 0); };
+  auto load_k = [&](int t) {
+    const int rows = rows_of(t);
+    const int bytes = rows > 0 ? (int)((rows - 1) * p.k_ss * 2) + ROWB : 0;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(Kh + (int64_t)(32 * t) * p.k_ss), 0,
+                                                      bytes, kBufferWord3);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      kf[s] = __builtin_bit_cast(uint4_t,
+                                 __builtin_amdgcn_raw_buffer_load_b128(rs, kofs + 32 * s, 0, 0));
+  };
+  auto load_v = [&](int t) {
+    const int rows = rows_of(t);
+    const int bytes = rows > 0 ? (int)((rows - 1) * p.v_ss * 2) + ROWB : 0;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(Vh + (int64_t)(32 * t) * p.v_ss), 0,
+                                                      bytes, kBufferWord3);
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+      vr[i] = __builtin_bit_cast(uint4_t,
+                                 __builtin_amdgcn_raw_buffer_load_b128(rs, vofs[i], 0, 0));
+  };
+  load_k(wave);
+  load_v(wave);
+
+  const int row = r0 + l32;
+  v8 qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    uint4_t v = {0, 0, 0, 0};
+    if (row < (VARLEN ? len : S)) v = ld16(Qh + (int64_t)row * p.q_ss + 16 * s + 8 * g);
+    if (p.neg_q) v ^= uint4_t{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+    qf[s] = E::as8(v);
+  }
+  // Transposing V reads: as in prefill_kernel.
+  const int s16 = lane & 15;
+  const int vrow = 4 * g + (s16 >> 2);
+  const int vcl = 2 * ((lane >> 4) & 1) + ((s16 & 3) >> 1);
+  int voff[NT], voffh[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    voff[n] = vrow * ROWB + (((4 * n + vcl) ^ tswz<D>(vrow)) * 16) + (s16 & 1) * 8;
+    voffh[n] = (vrow + 8) * ROWB + (((4 * n + vcl) ^ tswz<D>(vrow + 8)) * 16) + (s16 & 1) * 8;
+  }
+
+  const float c = p.qk_scale;
+  const int lim = (CAUSAL ? min(row, S - 1) : S - 1) - 4 * g;  // last key of this lane's row
+  float m_run = AKT_P_NEG_INF, l_part = 0.f;
+  float16_t oacc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[n][r] = 0.f;
+
+  for (int t = wave; t < n_steps; t += kNSplit) {
+    const int kh0 = 32 * t;
+    float16_t sv;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sv[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) sv = E::mfma(E::as8(kf[s]), qf[s], sv);
+    load_k(t + kNSplit);
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) *reinterpret_cast<uint4_t*>(vst + vdst[i]) = vr[i];
+    load_v(t + kNSplit);
+    if ((CAUSAL && kh0 + 31 > r0) || kh0 + 32 > S) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (kh0 + 8 * (r >> 2) + (r & 3) > lim) sv[r] = AKT_P_NEG_INF;
+    }
+    // Running max of row l32 (NaN-propagating, as in prefill_kernel).
+    float mx = sv[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = __builtin_elementwise_maximum(mx, sv[r]);
+    float ma, mb;
+    swap32(mx, ma, mb);
+    mx = __builtin_elementwise_maximum(ma, mb) * c;
+    const float m_new = __builtin_elementwise_maximum(m_run, mx);
+    if (__any(!(m_new <= m_run))) {
+      const float alpha = m_run == AKT_P_NEG_INF ? 0.f : fast_exp2(m_run - m_new);
+      l_part *= alpha;
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[n][r] *= alpha;
+      m_run = m_new;
+    }
+    const float m_use = m_run == AKT_P_NEG_INF ? 0.f : m_run;
+    uint32_t pk[8];
+#pragma unroll
+    for (int r = 0; r < 16; r += 2)
+      pk[r >> 1] = E::pack2(fast_exp2(__builtin_fmaf(sv[r], c, -m_use)),
+                            fast_exp2(__builtin_fmaf(sv[r + 1], c, -m_use)));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) l_part = E::dot2(pk[i], E::kOnes, l_part);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const v8 bop = E::as8(uint4_t{pk[4 * u], pk[4 * u + 1], pk[4 * u + 2], pk[4 * u + 3]});
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const uint2 lo = ds_read_tr16(vst + voff[n] + u * 16 * ROWB);
+        const uint2 hi = ds_read_tr16(vst + voffh[n] + u * 16 * ROWB);
+        oacc[n] = E::mfma(E::as8(uint4_t{lo.x, lo.y, hi.x, hi.y}), bop, oacc[n]);
+      }
+    }
+  }
+
+  // ---- merge: quad 4 n + q of O (dims 32 n + 8 q + 4 g .. + 3 of row l32) of
+  // every lane at [wave][quad][lane]; wave w then sums quads NT w .. of all waves.
+  const float l_row = xor32_sum(l_part);
+  if (g == 0) {
+    sm_m[wave][l32] = m_run;
+    sm_l[wave][l32] = l_row;
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<uint4_t*>(vst + ((4 * n + q) * 64 + lane) * 16) = as_uint4f(
+          float4_t{oacc[n][4 * q], oacc[n][4 * q + 1], oacc[n][4 * q + 2], oacc[n][4 * q + 3]});
+  __syncthreads();
+  float M = AKT_P_NEG_INF, L = 0.f, f[kNSplit];
+#pragma unroll
+  for (int w = 0; w < kNSplit; ++w) M = __builtin_elementwise_maximum(M, sm_m[w][l32]);
+#pragma unroll
+  for (int w = 0; w < kNSplit; ++w) {
+    f[w] = sm_m[w][l32] == AKT_P_NEG_INF ? 0.f : fast_exp2(sm_m[w][l32] - M);
+    L += f[w] * sm_l[w][l32];
+  }
+  const float inv = L > 0.f ? __builtin_amdgcn_rcpf(L) : 0.f;
+  if (p.lse && wave == 0 && g == 0 && row < row_lim)
+    p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.lse_sh + (int64_t)row * p.lse_ss] =
+        L > 0.f ? (M + __log2f(L)) * kLn2 : AKT_P_NEG_INF;
+  half_t* orow = p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_ss;
+#pragma unroll
+  for (int i = 0; i < NT; i += 2) {
+    uint2 hv[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kNSplit; ++w)
+        a += f[w] * as_float4u(*reinterpret_cast<const uint4_t*>(
+                        lds + w * OB + ((NT * wave + i + k) * 64 + lane) * 16));
+      hv[k] = uint2{E::pack2(a[0] * inv, a[1] * inv), E::pack2(a[2] * inv, a[3] * inv)};
+    }
+    // The lane halves hold 8-byte halves of both 16-byte chunks: half 0 takes
+    // chunk i whole, half 1 chunk i + 1.
+    const uint2 send = g == 0 ? hv[1] : hv[0];
+    const uint2 recv = {(uint32_t)__shfl_xor((int)send.x, 32, 64),
+                        (uint32_t)__shfl_xor((int)send.y, 32, 64)};
+    const uint4_t v = g == 0 ? uint4_t{hv[0].x, hv[0].y, recv.x, recv.y}
+                             : uint4_t{recv.x, recv.y, hv[1].x, hv[1].y};
+    if (row < row_lim) st16(orow + 8 * (NT * wave + i + g), v);
+  }
+}
+
+// Whether a launch takes prefill_split_kernel: its workgroups (one per query
+// head and 32 rows) are resident at once, two to a CU up to D = 128 and one from
+// D = 192.  Past that each round of them costs a whole walk, while the other
+// kernel shares every tile among four waves.  Measured at D = 128 (us, other /
+// split): 512 workgroups, S=2048 47.2 / 33.9, 608, S=600 18.4 / 17.6, 640, S=130
+// 8.7 / 11.8, 1024, S=1024 27.2 / 30.1; D = 256: 256, S=1024 44.2 / 28.9, 320,
+// S=130 13.0 / 16.3; D = 64: 512, S=2048 44.1 / 18.9, 640, S=130 8.7 / 8.3 and
+// non-causal 8.9 / 9.5, 1408, S=333 12.6 / 16.0.  At D = 64 long causal
+// sequences still gain at twice that (their later rounds are the light row
+// blocks): 1024, S=1024 24.4 / 18.8, 608, S=600 16.7 / 10.9, 1216, S=600 17.3 / 18.0.
+bool use_split_keys(int head_dim, int64_t heads, int64_t seq_len, bool causal) {
+  const int64_t wgs = heads * ceil_div(seq_len, 32);
+  if (head_dim == 64 && causal && seq_len >= 512) return wgs <= 1024;
+  return wgs <= (head_dim <= 128 ? 512 : 256);
+}
+
 template <int D, bool CAUSAL, bool VARLEN, bool BF16>
 int launch(const PrefillParams& p, dim3 grid, hipStream_t st) {
   KernelTimer timer;
+  if (p.split_keys) {
+    timer.launch(prefill_split_kernel<D, CAUSAL, VARLEN, BF16>,
+                 dim3(grid.x, grid.y, p.G * ((p.S + 31) / 32)), dim3(64 * kNSplit), 0, st, p);
+    return check_launch("prefill_split_kernel");
+  }
   timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16>, grid, dim3(kPThreads), 0, st, p);
   return check_launch("prefill_kernel");
 }
@@ -785,6 +1040,7 @@ int prefill_impl(const void* q, const void* k, const void* v, void* o, float* ls
   p.neg_q = softmax_scale < 0.f ? 1 : 0;
   p.qk_scale = fmaxf(fabsf(softmax_scale) * kLog2e, FLT_MIN);
   const int64_t n_wg = batch * num_kv_heads * p.n_sg;
+  p.split_keys = use_split_keys((int)head_dim, batch * num_q_heads, seq_len, causal != 0) ? 1 : 0;
   AKT_CHECK(n_wg < (1ll << 31), "problem too large");
   const dim3 grid = p.grid1d ? dim3((unsigned)n_wg)
                              : dim3((unsigned)num_kv_heads, (unsigned)batch, (unsigned)p.n_sg);

@@ -309,3 +309,66 @@ def test_prefill_negative_scale_bf16(dev):
     out = pre.flash_attention_prefill(Q.to(dev), K.to(dev), V.to(dev), True, -0.125, Hq // Hkv)
     ref = naive.prefill(Q, K, V, True, -0.125, Hq // Hkv)
     assert_close(out, ref, atol=ATOL_BF16, what="bf16 negative scale")
+
+
+def _prefill_inputs(seed, B, Hq, Hkv, S, D, dtype):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, h, S, D, generator=g).to(dtype) for h in (Hq, Hkv, Hkv)]
+
+
+def _check_prefill(dev, Q, K, V, causal, scale, lens=None):
+    """O and LSE of every valid row against fp64; 16-bit rounding of P and O sets the bars."""
+    B, Hq, S, D = Q.shape
+    G = Hq // K.shape[1]
+    if lens is None:
+        o, lse = pre.flash_attention_prefill(Q.to(dev), K.to(dev), V.to(dev), causal, scale, G,
+                                             return_lse=True)
+    else:
+        o, lse = prevar.flash_attention_prefill(Q.to(dev), K.to(dev), V.to(dev), causal, scale, G,
+                                            varlen=torch.tensor(lens).to(dev), return_lse=True)
+    o, lse = o.cpu().double(), lse.cpu().double()
+    atol, ltol = (1.6e-2, 1e-2) if Q.dtype == torch.bfloat16 else (2e-3, 2e-3)
+    for b in range(B):
+        n = S if lens is None else lens[b]
+        for h in range(Hq):
+            k, v = K[b, h // G].double(), V[b, h // G].double()
+            if causal:
+                k, v = k[:n], v[:n]
+            s = Q[b, h, :n].double() @ k.T * scale
+            if causal:
+                s.masked_fill_(torch.ones_like(s, dtype=torch.bool).triu(1), -math.inf)
+            ref = torch.softmax(s, -1) @ v
+            what = f"b={b} h={h} n={n}"
+            assert float((o[b, h, :n] - ref).abs().max() if n else 0) <= atol, what
+            assert float((lse[b, h, :n] - torch.logsumexp(s, -1)).abs().max() if n else 0) <= ltol, what
+
+
+# Small launches split a row block's keys over a workgroup's waves: step counts
+# below, at and past the four waves, ragged last steps and row blocks.
+@pytest.mark.parametrize("D", [64, 128, 192, 256])
+@pytest.mark.parametrize("S", [1, 31, 33, 127, 129, 333])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_prefill_small_launch_splits_keys(dev, D, S, causal, dtype):
+    Q, K, V = _prefill_inputs(S + D, 1, 6, 2, S, D, dtype)
+    _check_prefill(dev, Q, K, V, causal, -1 / math.sqrt(D) if S == 127 else 1 / math.sqrt(D))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_prefill_small_launch_varlen_and_strides(dev, D):
+    lens = [200, 0, 1, 64, 65, 127]
+    Q, K, V = _prefill_inputs(D, len(lens), 4, 1, 200, D, torch.float16)
+    for b, n in enumerate(lens):
+        for t in (Q, K, V):
+            t[b, :, n:] = float("nan")
+    seq_major = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (Q, K, V)]
+    _check_prefill(dev, *seq_major, True, 1 / math.sqrt(D), lens)
+
+
+# The same edges in launches past the small ones.
+@pytest.mark.parametrize("D", [64, 128, 192, 256])
+@pytest.mark.parametrize("B,Hkv,G,S", [(130, 2, 4, 17), (34, 16, 1, 64), (24, 3, 3, 130), (12, 3, 4, 257)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_large_launch_edges(dev, D, B, Hkv, G, S, causal):
+    Q, K, V = _prefill_inputs(S + D, B, Hkv * G, Hkv, S, D, torch.float16)
+    _check_prefill(dev, Q, K, V, causal, 1 / math.sqrt(D))
