@@ -1,17 +1,17 @@
 // Split-KV decode family for gfx950.
 //
-// One kernel skeleton serves every single-query path of the reference:
+// One kernel skeleton serves the chunked single-query paths (explicit chunk
+// lengths, small dense launches, and what the stream-K kernel of
+// paged_stream.hip does not take):
 //   dense GQA decode      decode_flash_attention_redundant.py:71-229
 //   paged var-len decode  decode_flash_attention_redundant_var_len_paged.py:70-224
-//   sparse-token decode   sparsetoken_decode_flash_attention_redundant.py:11-124
-//   sparse paged decode   sparsetoken_decode_flash_attention_redundant_var_len_paged.py:11-167
-//   MagicPIG with norm    magicpig_sparsetoken_decode_flash_attention_redundant_var_len_paged_with_norm.py:16-164
+// and this file holds the C entry points of those and of the sparse decodes
+// (kernels in sparse_decode.hip).
 //
 // Work decomposition.  A "unit" is the set of query heads that read the same
-// K/V rows: for dense and paged caches all (up to GT) query heads of one kv
-// head (the reference instead re-reads K/V once per query head and pads the
-// query to 16 rows, decode_flash_attention_redundant.py:235); for sparse paths
-// one query head (each head keeps its own token set).  A unit's logical token
+// K/V rows: all (up to GT) query heads of one kv head (the reference instead
+// re-reads K/V once per query head and pads the query to 16 rows,
+// decode_flash_attention_redundant.py:235).  A unit's logical token
 // sequence is cut into chunks; one 256-thread workgroup owns one chunk of one
 // unit and its four waves take 16-token groups round-robin.  Each wave keeps
 // an online softmax in registers, the waves are merged through LDS, and the
@@ -38,10 +38,11 @@
 #include "akt_common.hpp"
 #include "akt_host.hpp"
 #include "paged_stream.hpp"
+#include "sparse_decode.hpp"
 
 namespace akt {
 
-enum : int { kModeDense = 0, kModePaged = 1, kModeSparseDense = 2, kModeSparsePaged = 3 };
+enum : int { kModeDense = 0, kModePaged = 1 };
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
@@ -63,11 +64,6 @@ struct SplitParams {
   const int32_t* indptr;
   const int32_t* indices;
   const int32_t* last_len;
-  const int32_t* sparse_ind;
-  const int32_t* sparse_nnz;
-  const int64_t* csr_ptr;  // CSR kept-index rows: row u = sparse_ind[csr_ptr[u] .. csr_ptr[u+1])
-  const float* lsh_k;
-  const float* lsh_l;
   half_t* o;      // [B, Hq, D] contiguous
   float* lse;     // [B, Hq] or null
   int* counters;  // [2]: work tickets, exited workgroups (zero between launches)
@@ -80,17 +76,13 @@ struct SplitParams {
   // paged: row_a = page id, row_b = slot, unit offset = kvh*s_head.
   int64_t k_sa, k_sb, k_batch, k_head;
   int64_t v_sa, v_sb, v_batch, v_head;
-  int64_t ind_sb, ind_sh, nnz_sb, nnz_sh;
   int B, Hq, Hkv, G;
-  int S;             // dense / sparse-dense: cache length
+  int S;             // dense: cache length
   int page_size;
   int num_pool_pages;
-  int l_max;
   int n_hg;          // head groups per kv head (dense / paged)
   int chunk;         // tokens per chunk (dense / paged), multiple of 64
-  int n_split;       // chunks per unit (sparse)
   float qk_scale;    // softmax_scale * log2(e)
-  float inv_sqrt_d;  // 1 / sqrt(head_dim) (MagicPIG)
 };
 
 __device__ __forceinline__ int paged_len(const int32_t* __restrict__ indptr,
@@ -137,53 +129,6 @@ __device__ bool locate_chunk(const SplitParams& p, int x, int& b_out, int& c_out
   return false;
 }
 
-// g(y) = log1p(y) - y for y > -1, without the cancellation of the direct
-// difference near 0.  With s = y / (2 + y), log1p(y) = 2 atanh(s) =
-// 2 (s + s^3/3 + s^5/5 + ...) and 2 s - y = -y s, so
-//   g(y) = -y s + 2 s^3 (1/3 + s^2/5 + s^4/7 + s^6/9 + s^8/11 + ...),
-// whose two parts never cancel for |y| < 0.25 (|s| < 1/7: the dropped terms
-// are below 1e-10 relative).  From |y| = 0.25 on, the direct difference
-// loses at most 3 bits.
-__device__ __forceinline__ float log1p_minus_id(float y) {
-  if (fabsf(y) < 0.25f) {
-    const float s = y / (2.0f + y);
-    const float s2 = s * s;
-    const float poly =
-        (1.0f / 3.0f) + s2 * ((1.0f / 5.0f) + s2 * ((1.0f / 7.0f) + s2 * ((1.0f / 9.0f) + s2 * (1.0f / 11.0f))));
-    return __builtin_fmaf(-y, s, 2.0f * s * s2 * poly);
-  }
-  return log1pf(y) - y;
-}
-
-// MagicPIG correction ln u for one token (eq. 11 of the reference's
-// attention_with_norm.png, as evaluated in
-// magicpig_sparsetoken_decode_flash_attention_redundant_var_len_paged_with_norm.py:110-160):
-//   p = 1 - acos(c) / pi (clamped to [0, 1]),  x = p^K,
-//   u = 1 - (1 - x)^L - L x (1 - x)^(L - 1),  clamped to >= 1e-10.
-// u is a difference of nearly equal terms when x is small or L is near 1, so
-// it is evaluated in fp32 in a form without that cancellation.  With m = L - 1,
-//   u = 1 - (1 - x)^m (1 + m x) = -expm1(f),
-//   f = m log1p(-x) + log1p(m x) = m g(-x) + g(m x),   g(y) = log1p(y) - y
-// (the linear terms -m x and +m x cancel exactly), and for L >= 1 both parts
-// of f are <= 0, so nothing cancels for any x in [0, 1) and any L >= 1.  The
-// relative error of u stays within a few fp32 ulps.  Outside that domain
-// (x >= 1 from K < 0, or m x <= -1 from L < 0) the reference's formula is
-// evaluated as written, with its clamp of 1 - x to [0, 1].
-__device__ __forceinline__ float magicpig_log_u(float cosv, float K, float L) {
-  const float pp = fminf(fmaxf(1.0f - acosf(cosv) * (float)M_1_PI, 0.0f), 1.0f);
-  const float x = pp > 0.0f ? __expf(K * __logf(pp)) : 0.0f;
-  const float m = L - 1.0f;
-  const float mx = m * x;
-  float u;
-  if (x < 1.0f && mx > -1.0f) {
-    u = -expm1f(__builtin_fmaf(m, log1p_minus_id(-x), log1p_minus_id(mx)));
-  } else {
-    const float om = fminf(fmaxf(1.0f - x, 0.0f), 1.0f);
-    u = 1.0f - powf(om, L) - L * x * powf(om, m);
-  }
-  return __logf(fmaxf(u, 1e-10f));
-}
-
 // ---------------------------------------------------------------------------
 // Split kernel.
 // ---------------------------------------------------------------------------
@@ -194,7 +139,6 @@ struct Item {
   int b, kvh, hq0, nh, t0, t1, pstart, np, direct;
   int nch, unit, pstep;
   int64_t pidx, pfirst;
-  int64_t ind_off;  // sparse: offset of the unit's kept-index row in sparse_ind
 };
 
 // Everything needed to issue the loads of one item's groups.
@@ -202,7 +146,6 @@ struct IssueCtx {
   const half_t* kb;  // K base of the unit (dense: + batch/head offset; paged: + head offset)
   const half_t* vb;
   int64_t k_dummy, v_dummy;  // offsets of the unit's q row from kb / vb
-  const int* ind_row;        // sparse: kept-index row
   int t1, g_begin, pstart, np;
   int page_pref, slot_pref;  // aligned paged: page id / slot of this wave's k-th group (lane k)
 };
@@ -215,7 +158,8 @@ struct IssueCtx {
 // groups continuously across items: the last two groups of an item are
 // followed by the first two of the next, issued before the item's
 // workgroup merge, so the memory pipeline never drains between items.
-// Otherwise (sparse units) one workgroup handles the item named by blockIdx.
+// Otherwise (paged batches past the LDS table) one workgroup handles the item
+// named by blockIdx.
 // Two workgroups per CU (two waves per SIMD) is what hides a unit's load
 // latency; instances whose state fits in 256 registers per lane are held to it.
 template <int D, int GT>
@@ -223,7 +167,7 @@ constexpr int split_min_waves() {
   return (D <= 128 && GT <= 4) ? 2 : 1;
 }
 
-template <int D, int GT, int MODE, bool ALIGNED, bool MAGIC, int GPW, bool PERSIST>
+template <int D, int GT, int MODE, bool ALIGNED, int GPW, bool PERSIST>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_kernel(SplitParams p) {
   constexpr int KPL = D / 4;                 // K elements per lane per group
@@ -232,12 +176,7 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
   constexpr int VDIM = (D == 256) ? 16 : 8;  // V dims per lane
   constexpr int VLD = VDIM / 8;              // 16-byte loads per V token
   constexpr int NPAIR = VTOK / 2;
-  constexpr bool SPARSE = (MODE == kModeSparseDense || MODE == kModeSparsePaged);
-  constexpr bool PAGED_ADDR = (MODE == kModePaged || MODE == kModeSparsePaged);
-  static_assert(!SPARSE || GT == 1, "sparse units hold one query head");
-  static_assert(SPARSE == (GPW == 0), "sparse units have a dynamic group count");
-  static_assert(!SPARSE || !PERSIST, "sparse units are not persistent");
-  static_assert(GPW == 0 || GPW >= 2, "the cross-item pipeline needs two groups per wave");
+  static_assert(GPW >= 2, "the cross-item pipeline needs two groups per wave");
   constexpr bool TABLE = PERSIST && MODE == kModePaged;
 
   __shared__ __attribute__((aligned(16))) float sm_o[kWaves][GT][D];
@@ -314,49 +253,6 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
       finish_item(w, blockIdx.x, blockIdx.y, c, nch, len);
       w.pstart = p.indptr[w.b];
       w.np = p.indptr[w.b + 1] - w.pstart;
-    } else if constexpr (SPARSE) {
-      // Block x is split c = x / rows of row u = x % rows: consecutive blocks,
-      // which the dispatcher deals to the XCDs in turn, are different rows,
-      // so that the splits of one row (and the short last splits) spread
-      // over the XCDs.
-      const int x = blockIdx.x;
-      const int rows = (int)gridDim.x / p.n_split;
-      const int c = x / rows;
-      const int u = x - c * rows;
-      w.b = u / p.Hq;
-      w.hq0 = u - w.b * p.Hq;
-      w.kvh = w.hq0 / p.G;
-      w.nh = 1;
-      int n;
-      if (p.csr_ptr) {  // CSR rows: any length, no padding
-        const int64_t r0 = p.csr_ptr[u], r1 = p.csr_ptr[u + 1];
-        w.ind_off = r0;
-        n = (int)min(max(r1 - r0, (int64_t)0), (int64_t)INT32_MAX);
-      } else {  // padded rows [B, Hq, l_max] with a count per row
-        w.ind_off = (int64_t)w.b * p.ind_sb + (int64_t)w.hq0 * p.ind_sh;
-        n = p.sparse_nnz[(int64_t)w.b * p.nnz_sb + (int64_t)w.hq0 * p.nnz_sh];
-        n = min(max(n, 0), p.l_max);
-        // A dense-cache row with no kept token attends to its first index
-        // slot, as the reference's PyTorch path does (it treats nnz == 0 as
-        // nnz == 1, sparsetoken_decode_flash_attention_redundant.py:191-194);
-        // with the harness's -1 padding that slot names the last row.
-        if constexpr (MODE == kModeSparseDense) n = max(n, min(1, p.l_max));
-      }
-      // Split c covers [c*per, min(n, (c+1)*per)); per is a multiple of 16 so
-      // every split starts on a 16-token group and splits never share a group.
-      const int per = ((n + p.n_split - 1) / p.n_split + 15) & ~15;
-      w.t0 = c * per;
-      w.t1 = max(w.t0, min(n, w.t0 + per));
-      w.pidx = (int64_t)u * p.n_split + c;
-      w.direct = (p.n_split == 1);
-      w.nch = p.n_split;
-      w.unit = u;
-      w.pfirst = (int64_t)u * p.n_split;
-      w.pstep = 1;
-      if constexpr (MODE == kModeSparsePaged) {
-        w.pstart = p.indptr[w.b];
-        w.np = p.indptr[w.b + 1] - w.pstart;
-      }
     }
     return w;
   };
@@ -383,18 +279,15 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
   // prefetches the page id and slot of this wave's k-th group (a chunk has at
   // most kMaxChunk tokens, so at most 10 groups per wave).
   auto setup = [&](const Item& w, IssueCtx& cx, half8_t (&qd)[KS]) {
-    const int64_t k_unit = PAGED_ADDR ? (int64_t)w.kvh * p.k_head
-                                      : (int64_t)w.b * p.k_batch + (int64_t)w.kvh * p.k_head;
-    const int64_t v_unit = PAGED_ADDR ? (int64_t)w.kvh * p.v_head
-                                      : (int64_t)w.b * p.v_batch + (int64_t)w.kvh * p.v_head;
+    const int64_t k_unit = MODE == kModePaged ? (int64_t)w.kvh * p.k_head
+                                              : (int64_t)w.b * p.k_batch + (int64_t)w.kvh * p.k_head;
+    const int64_t v_unit = MODE == kModePaged ? (int64_t)w.kvh * p.v_head
+                                              : (int64_t)w.b * p.v_batch + (int64_t)w.kvh * p.v_head;
     cx.kb = p.kbase + k_unit;
     cx.vb = p.vbase + v_unit;
     const half_t* qrow0 = p.q + (int64_t)w.b * p.q_sb + (int64_t)w.hq0 * p.q_sh;
     cx.k_dummy = qrow0 - cx.kb;
     cx.v_dummy = qrow0 - cx.vb;
-    cx.ind_row = nullptr;
-    if constexpr (SPARSE)
-      cx.ind_row = p.sparse_ind + w.ind_off;
     cx.t1 = w.t1;
     cx.g_begin = w.t0 >> 4;
     cx.pstart = w.pstart;
@@ -485,32 +378,13 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     bool kval = pos_k < t1;
     if constexpr (MODE == kModeDense) {
       ra = pos_k;
-    } else if constexpr (MODE == kModePaged) {
+    } else {
       const int pc = min(pos_k, t1 - 1);  // t1 <= len, so pc's page is in the table
       const int lp = pc / p.page_size;
       const int page = p.indices[cx.pstart + lp];
       kval = kval && page >= 0 && page < p.num_pool_pages;
       ra = page;
       rb = pc - lp * p.page_size;
-    } else if constexpr (MODE == kModeSparseDense) {
-      int t = cx.ind_row[min(pos_k, t1 - 1)];
-      // Indices follow torch indexing, as the reference's gather K[b, h, ind]
-      // does (sparsetoken_decode_flash_attention_redundant.py:196): -S <= t < 0
-      // names row S + t.
-      if (t < 0) t += p.S;
-      kval = kval && t >= 0 && t < p.S;
-      ra = t;
-    } else {  // sparse paged
-      const int t = cx.ind_row[min(pos_k, t1 - 1)];
-      const int lp = t >= 0 ? t / p.page_size : 0;
-      kval = kval && t >= 0 && lp < cx.np;
-      // np == 0 (no pages) reads the unit's first kept index (always mapped)
-      // instead of an empty page table; such tokens are never used.
-      const int* pptr = cx.np > 0 ? p.indices + cx.pstart + min(lp, cx.np - 1) : cx.ind_row;
-      const int page = *pptr;
-      kval = kval && page >= 0 && page < p.num_pool_pages;
-      ra = page;
-      rb = t - lp * p.page_size;
     }
     const uint32_t vmask = (uint32_t)__ballot(kval) & 0xffffu;  // bit t: token gpos + t usable
     bf.vmask = vmask;
@@ -542,7 +416,6 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
   // ---- per-item accumulation state ----------------------------------------
   Item it;
   half8_t qf[KS];
-  float q_norm = 0.f, lsh_k = 0.f, lsh_l = 0.f;  // MagicPIG
   float m_run;   // running max of head c16 (log2 units)
   // Partial normalisers over this lane's tokens: l_part sums the fp16-rounded
   // probabilities that multiply V (so O is normalised consistently), e_part
@@ -558,19 +431,6 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     for (int h = 0; h < GT; ++h)
 #pragma unroll
       for (int d = 0; d < VDIM; ++d) acc[h][d] = 0.f;
-    if constexpr (MAGIC) {
-      // |q|^2 of the unit's head (valid in lanes with c16 == 0).
-      float qs = 0.f;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        uint4_t u = as_uint4(qf[s]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) qs = dot2(u[j], u[j], qs);
-      }
-      q_norm = sqrtf(rows_sum(qs));
-      lsh_k = p.lsh_k[(int64_t)it.b * p.Hq + it.hq0];
-      lsh_l = p.lsh_l[(int64_t)it.b * p.Hq + it.hq0];
-    }
   };
 
   // Scores, online softmax and P.V for a loaded group of the current item.
@@ -581,40 +441,9 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     for (int s = 0; s < KS; ++s) sacc = mfma16x16x32(as_half8(bf.k[s]), qf[s], sacc);
 
     float t[4];
-    if constexpr (MAGIC) {
-      // A sparse unit is one head (column 0 of the score tile), so the group
-      // needs 16 corrections, one per token: lane l evaluates token l & 15
-      // (its dot product comes from lane 16 (tt / 4), register tt % 4, and
-      // |k|^2 from the K-lane layout), and each score lane then fetches the
-      // scores of its tokens 4R + r.  Lanes of columns past the head carry
-      // head 0's scores, which are never stored.
-      float ks = 0.f;
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ks = dot2(bf.k[s][j], bf.k[s][j], ks);
-      ks = rows_sum(ks);
-      const int tt = lane & 15;
-      const int src = (tt >> 2) << 4;
-      const float d0 = __shfl(sacc[0], src, 64), d1 = __shfl(sacc[1], src, 64);
-      const float d2 = __shfl(sacc[2], src, 64), d3 = __shfl(sacc[3], src, 64);
-      const int rr = tt & 3;
-      const float dotp = rr == 0 ? d0 : (rr == 1 ? d1 : (rr == 2 ? d2 : d3));
-      const float kn = sqrtf(__shfl(ks, tt, 64));
-      const float qn = __shfl(q_norm, 0, 64);  // |q| of the unit's head (lane 0)
-      float cosv = dotp / (qn * kn + 1e-8f);
-      cosv = fminf(fmaxf(cosv, -1.0f + 1e-7f), 1.0f - 1e-7f);
-      const float sc_t = dotp * p.inv_sqrt_d - magicpig_log_u(cosv, lsh_k, lsh_l);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float sc = __shfl(sc_t, 4 * R + r, 64);
-        t[r] = ((vmask >> (4 * R + r)) & 1) ? sc * kLog2e : AKT_NEG_INF;
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        t[r] = ((vmask >> (4 * R + r)) & 1) ? sacc[r] * p.qk_scale : AKT_NEG_INF;
-    }
+    for (int r = 0; r < 4; ++r)
+      t[r] = ((vmask >> (4 * R + r)) & 1) ? sacc[r] * p.qk_scale : AKT_NEG_INF;
 
     // online softmax (head c16)
     float mt = fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]));
@@ -1096,37 +925,13 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     IssueCtx cc;
     setup(it, cc, qf);
     begin_item();
-    const int g_end = (it.t1 + 15) >> 4;
-    if constexpr (GPW > 0) {
-      Buf bufs[2];
-      const int gw = cc.g_begin + wave;
-      issue(cc, gw, bufs[0]);
+    Buf bufs[2];
+    const int gw = cc.g_begin + wave;
+    issue(cc, gw, bufs[0]);
 #pragma unroll
-      for (int k = 0; k < GPW; ++k) {
-        if (k + 1 < GPW) issue(cc, gw + kWaves * (k + 1), bufs[(k + 1) & 1]);
-        consume(bufs[k & 1]);
-      }
-    } else {
-      // Dynamic group count (sparse units): ping-pong over two buffers.  The
-      // last prefetch re-reads the current group (an L2 hit) so that every
-      // iteration issues the same loads.
-      int g = cc.g_begin + wave;
-      if (g < g_end) {
-        Buf A, B;
-        issue(cc, g, A);
-        for (;;) {
-          int gn = g + kWaves;
-          issue(cc, gn < g_end ? gn : g, B);
-          consume(A);
-          if (gn >= g_end) break;
-          g = gn;
-          gn = g + kWaves;
-          issue(cc, gn < g_end ? gn : g, A);
-          consume(B);
-          if (gn >= g_end) break;
-          g = gn;
-        }
-      }
+    for (int k = 0; k < GPW; ++k) {
+      if (k + 1 < GPW) issue(cc, gw + kWaves * (k + 1), bufs[(k + 1) & 1]);
+      consume(bufs[k & 1]);
     }
     finish();
   }
@@ -1156,9 +961,9 @@ int pick_gt(int G, int D) {
 
 // Launches one split-kernel instance.  Persistent instances get a grid of
 // min(items, resident workgroups); `grid` carries the item upper bound in x.
-template <int D, int GT, int MODE, bool ALIGNED, bool MAGIC, int GPW, bool PERSIST>
+template <int D, int GT, int MODE, bool ALIGNED, int GPW, bool PERSIST>
 int launch_split(const SplitParams& p, dim3 grid, hipStream_t st) {
-  auto kernel = split_kernel<D, GT, MODE, ALIGNED, MAGIC, GPW, PERSIST>;
+  auto kernel = split_kernel<D, GT, MODE, ALIGNED, GPW, PERSIST>;
   if (PERSIST) {
     const int64_t items = (int64_t)grid.x * grid.y;
     const int cap = resident_blocks(kernel, kThreads);
@@ -1170,51 +975,44 @@ int launch_split(const SplitParams& p, dim3 grid, hipStream_t st) {
   return check_launch("split_kernel");
 }
 
-template <int D, int GT, int MODE, bool ALIGNED, bool MAGIC>
+template <int D, int GT, int MODE, bool ALIGNED>
 int launch_t(const SplitParams& p, dim3 grid, hipStream_t st) {
-  constexpr bool SPARSE = (MODE == kModeSparseDense || MODE == kModeSparsePaged);
-  if constexpr (SPARSE) {
-    return launch_split<D, GT, MODE, ALIGNED, MAGIC, 0, false>(p, grid, st);
-  } else if constexpr (MODE == kModePaged && !ALIGNED) {
+  if constexpr (MODE == kModePaged && !ALIGNED) {
     // Pages that do not hold whole 16-token groups: 256-token chunks only.
-    if (p.B <= kMaxTableB) return launch_split<D, GT, MODE, false, MAGIC, 4, true>(p, grid, st);
-    return launch_split<D, GT, MODE, false, MAGIC, 4, false>(p, grid, st);
+    if (p.B <= kMaxTableB) return launch_split<D, GT, MODE, false, 4, true>(p, grid, st);
+    return launch_split<D, GT, MODE, false, 4, false>(p, grid, st);
   } else {
     // A chunk of `chunk` tokens is chunk / 64 16-token groups per wave.
     if constexpr (MODE == kModePaged) {
-      if (p.B > kMaxTableB) return launch_split<D, GT, MODE, ALIGNED, MAGIC, 4, false>(p, grid, st);
+      if (p.B > kMaxTableB) return launch_split<D, GT, MODE, ALIGNED, 4, false>(p, grid, st);
     }
-    if (p.chunk == 128) return launch_split<D, GT, MODE, ALIGNED, MAGIC, 2, true>(p, grid, st);
-    if (p.chunk == 256) return launch_split<D, GT, MODE, ALIGNED, MAGIC, 4, true>(p, grid, st);
-    if (p.chunk == 640) return launch_split<D, GT, MODE, ALIGNED, MAGIC, 10, true>(p, grid, st);
-    return launch_split<D, GT, MODE, ALIGNED, MAGIC, 8, true>(p, grid, st);
+    if (p.chunk == 128) return launch_split<D, GT, MODE, ALIGNED, 2, true>(p, grid, st);
+    if (p.chunk == 256) return launch_split<D, GT, MODE, ALIGNED, 4, true>(p, grid, st);
+    if (p.chunk == 640) return launch_split<D, GT, MODE, ALIGNED, 10, true>(p, grid, st);
+    return launch_split<D, GT, MODE, ALIGNED, 8, true>(p, grid, st);
   }
 }
 
-template <int D, int MODE, bool ALIGNED, bool MAGIC>
+template <int D, int MODE, bool ALIGNED>
 int launch_gt(int gt, const SplitParams& p, dim3 grid, hipStream_t st) {
-  if constexpr (MODE == kModeSparseDense || MODE == kModeSparsePaged) {
-    return launch_t<D, 1, MODE, ALIGNED, MAGIC>(p, grid, st);
-  } else {
-    switch (gt) {
-      case 1: return launch_t<D, 1, MODE, ALIGNED, MAGIC>(p, grid, st);
-      case 2: return launch_t<D, 2, MODE, ALIGNED, MAGIC>(p, grid, st);
-      case 4: return launch_t<D, 4, MODE, ALIGNED, MAGIC>(p, grid, st);
-      case 8: return launch_t<D, 8, MODE, ALIGNED, MAGIC>(p, grid, st);
-      case 16:
-        if constexpr (D != 256) return launch_t<D, 16, MODE, ALIGNED, MAGIC>(p, grid, st);
-        break;
-    }
-    return set_error(AKT_ERR_UNSUPPORTED, "no decode kernel for %d heads per unit", gt);
+  switch (gt) {
+    case 1: return launch_t<D, 1, MODE, ALIGNED>(p, grid, st);
+    case 2: return launch_t<D, 2, MODE, ALIGNED>(p, grid, st);
+    case 4: return launch_t<D, 4, MODE, ALIGNED>(p, grid, st);
+    case 8: return launch_t<D, 8, MODE, ALIGNED>(p, grid, st);
+    case 16:
+      if constexpr (D != 256) return launch_t<D, 16, MODE, ALIGNED>(p, grid, st);
+      break;
   }
+  return set_error(AKT_ERR_UNSUPPORTED, "no decode kernel for %d heads per unit", gt);
 }
 
-template <int MODE, bool ALIGNED, bool MAGIC>
+template <int MODE, bool ALIGNED>
 int launch_d(int D, int gt, const SplitParams& p, dim3 grid, hipStream_t st) {
   switch (D) {
-    case 64: return launch_gt<64, MODE, ALIGNED, MAGIC>(gt, p, grid, st);
-    case 128: return launch_gt<128, MODE, ALIGNED, MAGIC>(gt, p, grid, st);
-    case 256: return launch_gt<256, MODE, ALIGNED, MAGIC>(gt, p, grid, st);
+    case 64: return launch_gt<64, MODE, ALIGNED>(gt, p, grid, st);
+    case 128: return launch_gt<128, MODE, ALIGNED>(gt, p, grid, st);
+    case 256: return launch_gt<256, MODE, ALIGNED>(gt, p, grid, st);
   }
   return set_error(AKT_ERR_UNSUPPORTED, "head_dim %d not supported (64, 128, 256)", D);
 }
@@ -1272,11 +1070,11 @@ __global__ __launch_bounds__(kThreads) void zero_words_kernel(int* p, int64_t n)
 }
 
 // Zero-fills the arrival counters past the fixed area (see ws_layout).
-int clear_extra_arrivals(const SplitParams& p, const WsLayout& w, hipStream_t st) {
+int clear_extra_arrivals(int* arrive, const WsLayout& w, hipStream_t st) {
   if (w.extra_bytes == 0) return AKT_OK;
   const int64_t n = (int64_t)(w.extra_bytes / 4);
   hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)ceil_div(n, kThreads)), dim3(kThreads), 0,
-                     st, p.arrive + kArriveSlots, n);
+                     st, arrive + kArriveSlots, n);
   return check_launch("zero_words_kernel");
 }
 
@@ -1469,9 +1267,9 @@ extern "C" int akt_decode_fwd(const void* q, const void* k, const void* v, void*
   p.n_hg = n_hg;
   p.chunk = (int)chunk;
   p.qk_scale = softmax_scale * kLog2e;
-  rc = clear_extra_arrivals(p, wl, st);
+  rc = clear_extra_arrivals(p.arrive, wl, st);
   if (rc) return rc;
-  return launch_d<kModeDense, false, false>(D, gt, p, dim3((unsigned)(batch * nch), (unsigned)Y), st);
+  return launch_d<kModeDense, false>(D, gt, p, dim3((unsigned)(batch * nch), (unsigned)Y), st);
 }
 
 // ----------------------------- paged decode --------------------------------
@@ -1590,10 +1388,10 @@ int paged_decode_impl(const void* q, const void* kv_cache, const int32_t* kv_pag
   // grid.x >= batch: the non-persistent form writes empty sequences' rows from
   // workgroups blockIdx.x < batch.
   const dim3 grid((unsigned)gx, (unsigned)Y);
-  rc = clear_extra_arrivals(p, wl, st);
+  rc = clear_extra_arrivals(p.arrive, wl, st);
   if (rc) return rc;
-  if (page_size % 16 == 0) return launch_d<kModePaged, true, false>(D, gt, p, grid, st);
-  return launch_d<kModePaged, false, false>(D, gt, p, grid, st);
+  if (page_size % 16 == 0) return launch_d<kModePaged, true>(D, gt, p, grid, st);
+  return launch_d<kModePaged, false>(D, gt, p, grid, st);
 }
 }  // namespace akt
 
@@ -1625,7 +1423,7 @@ extern "C" size_t akt_sparse_decode_workspace_size(int64_t batch, int64_t num_q_
 
 namespace {
 
-int sparse_common(SplitParams& p, const void* q, const int32_t* sparse_ind,
+int sparse_common(SparseParams& p, const void* q, const int32_t* sparse_ind,
                   const int32_t* sparse_nnz, const int64_t* csr_ptr, void* o, float* lse,
                   int64_t batch,
                   int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t l_max,
@@ -1656,7 +1454,10 @@ int sparse_common(SplitParams& p, const void* q, const int32_t* sparse_ind,
   p.csr_ptr = csr_ptr;
   p.o = (half_t*)o;
   p.lse = lse;
-  bind_workspace(p, workspace, wl);
+  char* ws = (char*)workspace;
+  p.arrive = (int*)(ws + wl.arrive);
+  p.part_o = (float*)(ws + wl.part_o);
+  p.part_ml = (float*)(ws + wl.part_ml);
   p.q_sb = q_stride[0];
   p.q_sh = q_stride[1];
   if (!csr_ptr) {
@@ -1665,7 +1466,8 @@ int sparse_common(SplitParams& p, const void* q, const int32_t* sparse_ind,
     p.nnz_sb = nnz_stride[0];
     p.nnz_sh = nnz_stride[1];
   }
-  p.B = (int)batch; p.Hq = (int)num_q_heads; p.Hkv = (int)num_kv_heads;
+  p.Hq = (int)num_q_heads;
+  p.rows = (int)rows;
   p.G = (int)(num_q_heads / num_kv_heads);
   p.l_max = (int)l_max;
   p.n_split = (int)ns;
@@ -1685,7 +1487,7 @@ static int sparse_dense_impl(const void* q, const void* k, const void* v,
                              float softmax_scale, int64_t num_splits, void* workspace,
                              size_t workspace_bytes, void* stream) {
   clear_error();
-  SplitParams p = {};
+  SparseParams p = {};
   int64_t ns = 0;
   WsLayout wl = {};
   int rc = sparse_common(p, q, sparse_ind, sparse_nnz, csr_ptr, o, lse, batch, num_q_heads,
@@ -1700,15 +1502,12 @@ static int sparse_dense_impl(const void* q, const void* k, const void* v,
   p.kbase = (const half_t*)k;
   p.vbase = (const half_t*)v;
   p.k_sa = k_stride[2]; p.k_sb = 0; p.k_batch = k_stride[0]; p.k_head = k_stride[1];
-  p.v_sa = v_stride[2]; p.v_sb = 0; p.v_batch = v_stride[0]; p.v_head = v_stride[1];
+  p.v_sa = v_stride[2]; p.v_batch = v_stride[0]; p.v_head = v_stride[1];
   p.S = (int)seq_len;
   p.qk_scale = softmax_scale * kLog2e;
-  const int64_t rows = batch * num_q_heads;
-  rc = clear_extra_arrivals(p, wl, (hipStream_t)stream);
+  rc = clear_extra_arrivals(p.arrive, wl, (hipStream_t)stream);
   if (rc) return rc;
-  return launch_d<kModeSparseDense, false, false>((int)head_dim, 1, p,
-                                                  dim3((unsigned)(rows * ns), 1),
-                                                  (hipStream_t)stream);
+  return sparse_launch(p, (int)head_dim, false, false, (hipStream_t)stream);
 }
 
 extern "C" int akt_sparse_decode_fwd(const void* q, const void* k, const void* v,
@@ -1755,7 +1554,7 @@ static int sparse_paged_impl(bool magic, const void* q, const void* kv_cache,
                              float softmax_scale, int64_t num_splits, void* workspace,
                              size_t workspace_bytes, void* stream) {
   clear_error();
-  SplitParams p = {};
+  SparseParams p = {};
   int64_t ns = 0;
   WsLayout wl = {};
   int rc = sparse_common(p, q, sparse_ind, sparse_nnz, csr_ptr, o, lse, batch, num_q_heads,
@@ -1773,20 +1572,17 @@ static int sparse_paged_impl(bool magic, const void* q, const void* kv_cache,
   p.indptr = kv_page_indptr;
   p.indices = kv_page_indices;
   p.k_sa = kv_stride[0]; p.k_sb = kv_stride[3]; p.k_head = kv_stride[2];
-  p.v_sa = kv_stride[0]; p.v_sb = kv_stride[3]; p.v_head = kv_stride[2];
+  p.v_sa = kv_stride[0]; p.v_head = kv_stride[2];
   p.page_size = (int)page_size;
   p.num_pool_pages = (int)(num_pool_pages < (1ll << 31) ? num_pool_pages : (1ll << 31) - 1);
   p.qk_scale = softmax_scale * kLog2e;
   p.inv_sqrt_d = 1.0f / sqrtf((float)head_dim);
   p.lsh_k = lsh_k;
   p.lsh_l = lsh_l;
-  const int64_t rows = batch * num_q_heads;
-  const dim3 grid((unsigned)(rows * ns), 1);
   hipStream_t st = (hipStream_t)stream;
-  rc = clear_extra_arrivals(p, wl, st);
+  rc = clear_extra_arrivals(p.arrive, wl, st);
   if (rc) return rc;
-  if (magic) return launch_d<kModeSparsePaged, false, true>((int)head_dim, 1, p, grid, st);
-  return launch_d<kModeSparsePaged, false, false>((int)head_dim, 1, p, grid, st);
+  return sparse_launch(p, (int)head_dim, true, magic, st);
 }
 
 extern "C" int akt_sparse_decode_paged_fwd(

@@ -393,7 +393,7 @@ def bench_legs(args):
     legs["sparse_config4a"] = _leg(
         "config 4a", [lambda kv=kv: _ops.sparse_decode(q4, kv[0], kv[1], ind4, nnz4, s4.scale,
                                                       return_lse=True) for kv in kv4],
-        b4, "GB/s", "split_kernel<128,1,kModeSparseDense>", args,
+        b4, "GB/s", "sparse_kernel<128>", args,
         note=f"O + LSE; K/V rotated over {n4} copies; bytes = unique kept rows per kv head")
     del kv4
     torch.cuda.empty_cache()
@@ -427,14 +427,14 @@ def bench_legs(args):
         "config 4b", [lambda st=st: _ops.sparse_decode_paged(p5.q, p5.pool, p5.indptr, p5.indices,
                                                              st[0], st[1], return_lse=True)
                       for st in sets],
-        b5, "GB/s", "split_kernel<256,1,kModeSparsePaged>", args,
+        b5, "GB/s", "sparse_kernel<256,paged>", args,
         note=f"O + LSE; {len(sets)} kept-index sets rotated")
     lk, ll = s5.lsh_k.to(dev), s5.lsh_l.to(dev)
     legs["magicpig_config4b"] = _leg(
         "config 4b MagicPIG", [lambda st=st: _ops.sparse_decode_paged(
             p5.q, p5.pool, p5.indptr, p5.indices, st[0], st[1], return_lse=True, lsh_k=lk,
             lsh_l=ll) for st in sets],
-        b5, "GB/s", "split_kernel<256,1,kModeSparsePaged,magicpig>", args,
+        b5, "GB/s", "sparse_kernel<256,paged,magicpig>", args,
         note=f"O + LSE with norm; {len(sets)} kept-index sets rotated")
     ind5, nnz5 = sets[0][0].cpu(), sets[0][1].cpu()
     del p5, sets

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from attention_kernel_triton_amd import kept_index
+from attention_kernel_triton_amd import _ops, kept_index
 from attention_kernel_triton_amd import magicpig_sparsetoken_decode_flash_attention_redundant_var_len_paged_with_norm as mp
 from attention_kernel_triton_amd import sparsetoken_decode_flash_attention_redundant as sp
 from attention_kernel_triton_amd import sparsetoken_decode_flash_attention_redundant_var_len_paged as spp
@@ -385,3 +385,40 @@ def test_sparse_paged_and_magicpig_on_the_reference_harness_fixture(dev):
     assert_close(ml, l64, atol=1e-3, what="harness fixture, MagicPIG lse vs fp64 oracle")
     print(f"harness fixture: sparse paged err {err:.3e}, MagicPIG err {merr:.3e}, "
           f"kept per head {float(zc.float().mean()):.0f}")
+
+
+# A wave resolves its kept tokens 64 at a time: lists that give the four waves of
+# a row's workgroups 0, 1, 4, 5, 8 and 9 groups, with ragged last groups.
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_sparse_groups_per_wave_edges(dev, D, splits):
+    counts = [1, 15, 16, 17, 64, 65, 255, 256, 257, 321, 511, 512, 513, 577, 769, 1000]
+    g = torch.Generator().manual_seed(D + splits)
+    Hq, Hkv, page, lens = len(counts), 4, 16, [3000, 2001]
+    indptr, indices, last, P = syn.block_table(g, lens, page)
+    pool = torch.randn(P, 2, Hkv, page, D, generator=g).half()
+    q = torch.randn(2, Hq, 1, D, generator=g).half()
+    ind = torch.full((2, Hq, 1100), -1, dtype=torch.int32)
+    for b in range(2):
+        for h, n in enumerate(counts):
+            ind[b, h, :n] = torch.randperm(lens[b], generator=g)[:n].sort().values.int()
+    nnz = torch.tensor(counts, dtype=torch.int32).expand(2, Hq).unsqueeze(-1).contiguous()
+    lk, ll = (torch.rand(2, Hq, generator=g) * 5 + 1 for _ in range(2))
+    dargs = [t.to(dev) for t in (q, pool, indptr, indices, ind, nnz)]
+    args = (q, pool, indptr, indices, ind, nnz)
+    o, lse = _ops.sparse_decode_paged(*dargs, return_lse=True, num_splits=splits)
+    ro, rl = naive.sparsetoken_naive_paged_attention(*args)
+    assert_close(o, ro, what="paged")
+    assert_close(lse, rl, atol=1e-4, what="paged lse")
+    o, lse = _ops.sparse_decode_paged(*dargs, return_lse=True, num_splits=splits,
+                                      lsh_k=lk.to(dev), lsh_l=ll.to(dev))
+    ro, rl = naive.magicpig_sparsetoken_naive_paged_attention(*args, lk, ll)
+    assert_close(o, ro, what="MagicPIG")
+    assert_close(lse, rl, atol=1e-3, what="MagicPIG lse")
+    K, V = (torch.randn(2, Hkv, 3000, D, generator=g).half() for _ in range(2))
+    K2 = K.transpose(1, 2).contiguous().transpose(1, 2)  # K and V of different strides
+    o, lse = _ops.sparse_decode(dargs[0], K2.to(dev), V.to(dev), dargs[4], dargs[5],
+                                1 / math.sqrt(D), return_lse=True, num_splits=splits)
+    ro, rl = naive.sparsetoken_naive_decode(q, K, V, ind, nnz, 1 / math.sqrt(D), Hq // Hkv)
+    assert_close(o, ro, what="dense")
+    assert_close(lse, rl, atol=1e-4, what="dense lse")

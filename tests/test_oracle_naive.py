@@ -372,7 +372,7 @@ def _eq11_exact(x, L):
 
 
 def _g32(y):
-    """log1p(y) - y in float32 as the kernels evaluate it (decode.hip log1p_minus_id)."""
+    """log1p(y) - y in float32 as the kernels evaluate it (sparse_decode.hip log1p_minus_id)."""
     f = np.float32
     y = f(y)
     if abs(y) < f(0.25):
