@@ -422,3 +422,29 @@ def test_sparse_groups_per_wave_edges(dev, D, splits):
     ro, rl = naive.sparsetoken_naive_decode(q, K, V, ind, nnz, 1 / math.sqrt(D), Hq // Hkv)
     assert_close(o, ro, what="dense")
     assert_close(lse, rl, atol=1e-4, what="dense lse")
+
+
+# Both ways of reading mask rows (whole words, single bytes) and the fp32 draws, at
+# the edges of runs, chunks, waves and steps, against torch.nonzero.
+@pytest.mark.parametrize("n", [1, 3, 4, 15, 16, 17, 255, 1024, 2047, 2049, 32767, 32768, 32772, 70001])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+@pytest.mark.parametrize("density", [0.02, 0.6])
+def test_kept_index_sources_and_edges(dev, n, offset, density):
+    g = torch.Generator().manual_seed(n + offset)
+    rows = 3
+    flat = torch.rand(rows * n + offset, generator=g)
+    u = flat[offset:].view(rows, n)
+    lens = torch.tensor([n, max(0, n - 5), n // 2], dtype=torch.int32)
+    l_max = max(1, n - 2 if density > 0.5 else n // 2)
+    mask = (flat.to(dev) < density)[offset:].view(rows, n)  # starts `offset` bytes into its storage
+    for src in (dict(mask=mask), dict(uniform=u.to(dev), kept_ratio=density)):
+        for rl in (None, lens):
+            ind, nnz = kept_index.select_kept(l_max, row_len=None if rl is None else rl.to(dev), **src)
+            for r in range(rows):
+                m = n if rl is None else int(rl[r])
+                want = torch.nonzero(u[r, :m] < density).view(-1).int()
+                want = want if want.numel() else torch.zeros(1, dtype=torch.int32)
+                assert int(nnz[r]) == want.numel()
+                k = min(want.numel(), l_max)
+                got = ind[r].cpu()
+                assert torch.equal(got[:k], want[:k]) and bool((got[k:] == -1).all())
