@@ -1278,10 +1278,17 @@ static int64_t paged_grid_x(int64_t total_pages, int64_t page_size, int64_t chun
 }
 
 // The stream-K kernel (paged_stream.hip) serves the automatic chunk length
-// whenever it can; explicit chunk lengths keep the chunked split kernel.
+// whenever it can, except for small launches; explicit chunk lengths keep the
+// chunked split kernel.  Small: below 2048 16-token groups in fewer than 128
+// units, where the split kernel's smaller workgroups start and merge sooner.
+// Measured (us, stream / split at its automatic chunk): D = 128, 504 groups in 8
+// units 12.4 / 10.1, 500 in 1 24.7 / 21.1, 2000 in 8 16.5 / 14.0, 2448 in 128
+// 13.3 / 14.2, 4704 in 128 17.0 / 19.7; D = 256, 500 in 1 63.4 / 37.3, 2448 in
+// 128 18.2 / 18.8; D = 64, 1552 in 32 11.6 / 11.0, 2448 in 128 11.6 / 13.6.
 static bool use_stream(int64_t chunk_tokens, int64_t batch, int64_t page_size,
                        int64_t total_pages, int64_t Y) {
-  return chunk_tokens == 0 && paged_stream_eligible(batch, page_size, total_pages, Y);
+  if (chunk_tokens != 0 || !paged_stream_eligible(batch, page_size, total_pages, Y)) return false;
+  return Y * total_pages * (page_size / 16) >= 2048 || batch * Y >= 128;
 }
 
 static WsLayout paged_layout(int64_t batch, int64_t Y, int gt, int64_t D, int64_t page_size,

@@ -405,8 +405,8 @@ def test_decode_more_units_than_the_fixed_arrival_area(dev):
 # round trip) up to more than a round trip holds (merged by a workgroup), with
 # unit starts inside and at the edges of a workgroup's range, for every head
 # count a unit can have and both workgroup sizes.
-@pytest.mark.parametrize("lens", [[30001], [16 * 8 * 40], [9000, 1, 700, 16 * 8 * 33, 40],
-                                  [128] * 40 + [5000]])
+@pytest.mark.parametrize("lens", [[40001], [16 * 8 * 256], [9000, 1, 700, 16 * 8 * 200, 40],
+                                  [128] * 300 + [5000]])
 @pytest.mark.parametrize("G,D", [(1, 128), (3, 128), (8, 128), (16, 128), (4, 64), (4, 256)])
 def test_paged_units_over_many_workgroups(dev, lens, G, D):
     from attention_kernel_triton_amd import _ops
