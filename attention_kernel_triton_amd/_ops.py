@@ -74,9 +74,6 @@ def prefill(Q, K, V, causal, softmax_scale, varlen=None, return_lse=False):
 
 
 # --------------------------------------------------------------------------- merge
-_DTYPE_CODE = {torch.float16: 0, torch.float32: 1}
-
-
 def merge_states(o, lse, out_dtype=None):
     """Log-sum-exp merge of N partial attention states.
 
@@ -84,38 +81,10 @@ def merge_states(o, lse, out_dtype=None):
     lse: [N, ...] fp32 natural-log normalisers.  Returns (o_merged [..., D]
     in out_dtype (default o's dtype), lse_merged [...] fp32).
     """
-    _need_gpu("o", o)
-    _need_gpu("lse", lse)
-    _same_device(o.device, lse=lse)
-    if o.dtype not in _DTYPE_CODE:
-        raise TypeError(f"o must be float16 or float32, got {o.dtype}")
-    if lse.dtype != torch.float32:
-        raise TypeError(f"lse must be float32, got {lse.dtype}")
-    if o.dim() < 2 or tuple(lse.shape) != tuple(o.shape[:-1]):
-        raise ValueError(f"lse shape {tuple(lse.shape)} must equal o.shape[:-1] = "
-                         f"{tuple(o.shape[:-1])}")
-    out_dtype = o.dtype if out_dtype is None else out_dtype
-    if out_dtype not in _DTYPE_CODE:
+    if out_dtype is not None and out_dtype not in (torch.float16, torch.float32):
         raise TypeError(f"out_dtype must be float16 or float32, got {out_dtype}")
-    n, D = o.shape[0], o.shape[-1]
-    rest = tuple(o.shape[1:-1])
-    rows = 1
-    for r in rest:
-        rows *= r
-    o3 = o.reshape(n, rows, D)
-    esz = o.element_size()
-    if (o3.stride(-1) != 1 or o3.data_ptr() % 16 or any((s * esz) % 16 for s in o3.stride()[:2])):
-        o3 = o3.contiguous()
-    l2 = lse.reshape(n, rows)
-    out = torch.empty(rest + (D,), dtype=out_dtype, device=o.device)
-    lse_out = torch.empty(rest, dtype=torch.float32, device=o.device)
-    lib = N.load()
-    rc = lib.akt_merge_states(N.ptr(o3), _DTYPE_CODE[o.dtype], N.ptr(l2), N.ptr(out),
-                              _DTYPE_CODE[out_dtype], N.ptr(lse_out), n, rows, D,
-                              N.i64s(o3.stride(0), o3.stride(1)), N.i64s(l2.stride(0), l2.stride(1)),
-                              D, 1, N.stream_of(o))
-    N.check(rc, "akt_merge_states")
-    return out, lse_out
+    return N.torch_ext().merge_states(o, lse, -1 if out_dtype is None
+                                      else int(out_dtype is torch.float32))
 
 
 # --------------------------------------------------------------------------- decode

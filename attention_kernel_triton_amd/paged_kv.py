@@ -19,7 +19,6 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from ._ops import _half_rows, _int32, _need_gpu, _same_device
 
 
 def append_paged_kv(k_new, v_new, append_indptr, paged_kv_cache, kv_page_indptr,
@@ -30,32 +29,8 @@ def append_paged_kv(k_new, v_new, append_indptr, paged_kv_cache, kv_page_indptr,
     positions under the page table (which must already count them).  Runs
     asynchronously on the current stream.
     """
-    pool = paged_kv_cache
-    _need_gpu("paged_kv_cache", pool)
-    if pool.dtype != torch.float16:
-        raise TypeError(f"paged_kv_cache must be float16, got {pool.dtype}")
-    if pool.stride(-1) != 1:
-        raise ValueError("paged_kv_cache needs a unit head_dim stride (it is written in place)")
-    dev = pool.device
-    k_new = _half_rows("k_new", k_new)
-    v_new = _half_rows("v_new", v_new)
-    _same_device(dev, k_new=k_new, v_new=v_new)
-    ap = _int32("append_indptr", append_indptr, dev).contiguous()
-    indptr = _int32("kv_page_indptr", kv_page_indptr, dev).contiguous()
-    indices = _int32("kv_page_indices", kv_page_indices, dev).contiguous()
-    last = _int32("kv_last_page_len", kv_last_page_len, dev).contiguous()
-    P, _, Hkv, page, D = pool.shape
-    if k_new.dim() != 3 or k_new.shape[1:] != (Hkv, D) or v_new.shape != k_new.shape:
-        raise ValueError(f"k_new / v_new must be [total_new, {Hkv}, {D}]")
-    B = indptr.numel() - 1
-    if ap.numel() != B + 1 or last.numel() != B:
-        raise ValueError("append_indptr needs B+1 entries and kv_last_page_len B")
-    lib = N.load()
-    rc = lib.akt_paged_kv_append(N.ptr(k_new), N.ptr(v_new), N.ptr(ap), N.ptr(pool), N.ptr(indptr),
-                                 N.ptr(indices), N.ptr(last), B, k_new.shape[0], Hkv, D, page, P,
-                                 N.strides(k_new), N.strides(v_new), N.strides(pool),
-                                 N.stream_of(pool))
-    N.check(rc, "akt_paged_kv_append")
+    N.torch_ext().append_paged_kv(k_new, v_new, append_indptr, paged_kv_cache, kv_page_indptr,
+                                  kv_page_indices, kv_last_page_len)
 
 
 class PagedKVCache:
