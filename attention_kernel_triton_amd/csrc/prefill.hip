@@ -6,15 +6,16 @@
 // with an MFMA kernel designed around CDNA4's v_mfma_f32_32x32x16_f16 (or its
 // bf16 form for bf16 tensors) and the transposing LDS read (ds_read_b64_tr_b16).
 //
-// Work decomposition.  A 256-thread workgroup serves one (batch, kv head) and
-// four "slots"; slot f = (query head f % G, row block f / G) of that kv head's
-// G query heads (64-row blocks at D = 64, 32-row blocks otherwise).  With G a multiple of 4 the four waves
+// Work decomposition.  A workgroup of four waves (eight in large launches at
+// D = 128) serves one (batch, kv head) and one "slot" per wave; slot f = (query
+// head f % G, row block f / G) of that kv head's G query heads (64-row blocks at
+// D = 64, 32-row blocks otherwise).  With G a multiple of 4 four waves
 // are four query heads at the same rows: they share every staged K/V tile and
 // have identical causal extents.  With 64-row blocks each wave owns its rows
 // as two 32-row MFMA blocks that share every K and V fragment read from LDS
 // (see rblocks_for).
 //
-// K/V staging.  Each tile of K and V (64 keys with two row blocks, else 32) goes
+// K/V staging.  Each tile of K and V (64 or 32 keys, see tile_keys_for) goes
 // global -> registers -> one of four LDS tile buffers: while tile j is
 // computed, tile j + 1 is already
 // published, tile j + 2 is being written and tile j + 3 is in flight from
@@ -87,9 +88,10 @@ struct PrefillParams {
   int varlen_bits;
   int n_rb;      // query row blocks (slots of one head) per sequence
   int n_sg;      // slot groups (workgroups) per (batch, kv head)
+  int waves;       // waves (slots) per workgroup
   int split_keys;  // 1: prefill_split_kernel (small launches)
   int grid1d;    // 1: linear grid (a dimension past 65535); 0: grid (Hkv, B, n_sg)
-  int fast_div;  // 1: G * n_rb + kSlots < 2^22, slot / G through g_inv
+  int fast_div;  // 1: G * n_rb + waves < 2^22, slot / G through g_inv
   float g_inv;   // 1 / G
   float qk_scale;  // |softmax_scale| * log2(e), at least FLT_MIN
   int neg_q;       // 1: softmax_scale < 0, computed as (-Q) K^T at |softmax_scale|
@@ -97,19 +99,21 @@ struct PrefillParams {
 
 namespace {
 
-constexpr int kPThreads = 256;
-constexpr int kSlots = 4;   // waves per workgroup
 constexpr int kNBuf = 4;    // LDS tile buffers
 // 32-row MFMA blocks per wave, query rows per slot, keys per staged tile and
 // waves per SIMD of an instance: two blocks and 64-key tiles at D = 64, one
 // block and 32-key tiles from D = 128.  Up to D = 128 that holds a wave in 256
 // VGPRs and a workgroup's four K + V buffers in 64 KB, so two waves share each
-// SIMD.  (Two blocks at one wave per SIMD, 128 KB of LDS, were slower at D = 128
+// SIMD.  Large launches at D = 128 run eight waves over 64-key tiles (128 KB) in a
+// workgroup, one to a CU: half the barriers, tile loads and LDS stores per wave
+// (see wide_workgroups).  (Two blocks at one wave per SIMD, 128 KB of LDS, were slower at D = 128
 // at every length: 536-578 against 524 us on B=1, Hq=32, Hkv=8, S=8192.)  At
 // D = 192 and 256 the register budget allows one wave per SIMD.
 __host__ __device__ constexpr int rblocks_for(int D) { return D == 64 ? 2 : 1; }
 __host__ __device__ constexpr int rows_for(int D) { return 32 * rblocks_for(D); }
-__host__ __device__ constexpr int tile_keys_for(int D) { return D == 64 ? 64 : 32; }
+__host__ __device__ constexpr int tile_keys_for(int D, int WAVES) {
+  return D == 64 || WAVES == 8 ? 64 : 32;
+}
 __host__ __device__ constexpr int waves_per_simd(int D) { return D <= 128 ? 2 : 1; }
 // Issue order of a step (see step()): its first mix_mfma MFMAs are followed by
 // mix_valu VALU instructions each, the rest is the scheduler's.  Measured (us):
@@ -213,15 +217,17 @@ __device__ __forceinline__ int div_small(int n, int d, float inv) {
   return q;
 }
 
-template <int D, bool CAUSAL, bool VARLEN, bool BF16>
-__global__ __launch_bounds__(kPThreads)
+template <int D, bool CAUSAL, bool VARLEN, bool BF16, int WAVES>
+__global__ __launch_bounds__(64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), 2)))
 void prefill_kernel(PrefillParams p) {
   typedef Elt<BF16> E;
   typedef typename E::v8 v8;
+  constexpr int kPThreads = 64 * WAVES;
+  constexpr int kSlots = WAVES;           // one slot per wave
   constexpr int NRB = rblocks_for(D);     // 32-row MFMA blocks per wave
   constexpr int kRows = rows_for(D);      // query rows per slot
-  constexpr int kBN = tile_keys_for(D);   // keys per staged tile
+  constexpr int kBN = tile_keys_for(D, WAVES);  // keys per staged tile
   constexpr int SPT = kBN / 32;           // 32-key steps per tile
   constexpr int KS = D / 16;              // MFMA k-steps over the head dim
   constexpr int HALF = D / 2;             // head dims per lane half in S^T operands
@@ -919,6 +925,20 @@ bool use_split_keys(int head_dim, int64_t heads, int64_t seq_len, bool causal) {
   return wgs <= (head_dim <= 128 ? 512 : 256);
 }
 
+// Whether a launch runs eight-wave workgroups (D = 128): at least 768 workgroups
+// of four slots (one and a half rounds of the resident ones; below that the
+// eight waves crowd on one CU while others idle), and, if causal, a workgroup's
+// slots (8 / G row blocks) within an eighth of the sequence, so that its early
+// waves do not wait long for the last.  Measured (us, four / eight waves), causal
+// with G = 4 unless noted: 256 workgroups 29.4 / 34.2, 512 59.0 / 60.7, 752 93.8 /
+// 92.6, 1024 151.2 / 143.2, 2048 (S = 8192) 562.3 / 530.0; G = 1: 640 (S = 600)
+// 27.8 / 32.7, 1024 (S = 1024) 53.5 / 55.1, 2048 (S = 2048) 167.3 / 166.9;
+// non-causal 512 74.4 / 70.5, 1024 145.0 / 140.3, 2048 282.4 / 276.3.
+bool wide_workgroups(int head_dim, int64_t kv_heads, int64_t G, int64_t seq_len, bool causal) {
+  return head_dim == 128 && kv_heads * ceil_div(G * ceil_div(seq_len, 32), 4) >= 768 &&
+         (!causal || G * seq_len >= 2048);
+}
+
 template <int D, bool CAUSAL, bool VARLEN, bool BF16>
 int launch(const PrefillParams& p, dim3 grid, hipStream_t st) {
   KernelTimer timer;
@@ -927,7 +947,13 @@ int launch(const PrefillParams& p, dim3 grid, hipStream_t st) {
                  dim3(grid.x, grid.y, p.G * ((p.S + 31) / 32)), dim3(64 * kNSplit), 0, st, p);
     return check_launch("prefill_split_kernel");
   }
-  timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16>, grid, dim3(kPThreads), 0, st, p);
+  if constexpr (D == 128) {
+    if (p.waves == 8) {
+      timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16, 8>, grid, dim3(512), 0, st, p);
+      return check_launch("prefill_kernel");
+    }
+  }
+  timer.launch(prefill_kernel<D, CAUSAL, VARLEN, BF16, 4>, grid, dim3(256), 0, st, p);
   return check_launch("prefill_kernel");
 }
 
@@ -1028,9 +1054,10 @@ int prefill_impl(const void* q, const void* k, const void* v, void* o, float* ls
   p.G = (int)(num_q_heads / num_kv_heads);
   p.S = (int)seq_len;
   p.n_rb = (int)ceil_div(seq_len, rows_for((int)head_dim));
-  p.n_sg = (int)ceil_div((int64_t)p.G * p.n_rb, kSlots);
+  p.waves = wide_workgroups((int)head_dim, batch * num_kv_heads, p.G, seq_len, causal != 0) ? 8 : 4;
+  p.n_sg = (int)ceil_div((int64_t)p.G * p.n_rb, p.waves);
   p.grid1d = (batch > 65535 || p.n_sg > 65535) ? 1 : 0;
-  p.fast_div = ((int64_t)p.G * p.n_rb + kSlots < (1ll << 22)) ? 1 : 0;
+  p.fast_div = ((int64_t)p.G * p.n_rb + p.waves < (1ll << 22)) ? 1 : 0;
   p.g_inv = 1.0f / (float)p.G;
   // Any finite scale: a negative one flips Q's sign in the kernel; a zero (or
   // subnormal) one becomes FLT_MIN, whose product with any score below 2^100

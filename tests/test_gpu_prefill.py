@@ -372,3 +372,14 @@ def test_prefill_small_launch_varlen_and_strides(dev, D):
 def test_prefill_large_launch_edges(dev, D, B, Hkv, G, S, causal):
     Q, K, V = _prefill_inputs(S + D, B, Hkv * G, Hkv, S, D, torch.float16)
     _check_prefill(dev, Q, K, V, causal, 1 / math.sqrt(D))
+
+
+# Eight-wave workgroups over 64-key tiles: large launches at D = 128.
+@pytest.mark.parametrize("B,Hkv,G,S,causal", [(24, 8, 4, 130, False), (12, 4, 16, 130, True),
+                                              (6, 8, 8, 257, True), (12, 4, 3, 700, True),
+                                              (48, 16, 1, 33, False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_prefill_d128_eight_wave_workgroups(dev, B, Hkv, G, S, causal, dtype):
+    Q, K, V = _prefill_inputs(S + G, B, Hkv * G, Hkv, S, 128, dtype)
+    lens = [(37 * b) % (S + 1) for b in range(B)] if causal and dtype == torch.float16 else None
+    _check_prefill(dev, Q, K, V, causal, 1 / math.sqrt(128), lens)
