@@ -919,10 +919,12 @@ void prefill_split_kernel(PrefillParams p) {
 // non-causal 8.9 / 9.5, 1408, S=333 12.6 / 16.0.  At D = 64 long causal
 // sequences still gain at twice that (their later rounds are the light row
 // blocks): 1024, S=1024 24.4 / 18.8, 608, S=600 16.7 / 10.9, 1216, S=600 17.3 / 18.0.
+// At D = 128 two steps of keys (S <= 64) repay one workgroup to a CU but not a
+// second: 256, S=64 7.3 / 5.9, 288, S=55 with the LSE 7.40 / 7.48.
 bool use_split_keys(int head_dim, int64_t heads, int64_t seq_len, bool causal) {
   const int64_t wgs = heads * ceil_div(seq_len, 32);
   if (head_dim == 64 && causal && seq_len >= 512) return wgs <= 1024;
-  return wgs <= (head_dim <= 128 ? 512 : 256);
+  return wgs <= (head_dim == 64 || (head_dim == 128 && seq_len > 64) ? 512 : 256);
 }
 
 // Whether a launch runs eight-wave workgroups (D = 128): at least 768 workgroups
