@@ -2,8 +2,8 @@
 
 ``flash_attention_decode`` keeps the reference signature and result shape
 (decode_flash_attention_redundant.py:233-271) but does not replicate q to 16
-rows: the gfx950 split-KV kernel (csrc/decode.hip) serves all query heads of a
-kv head from one read of K/V.  ``return_lse=True`` additionally returns the
+rows: the gfx950 kernels (csrc/paged_stream.hip, csrc/decode.hip) serve all query
+heads of a kv head from one read of K/V.  ``return_lse=True`` additionally returns the
 natural-log softmax normaliser [B, Hq] (fp32) of the scaled scores.
 """
 from __future__ import annotations
