@@ -460,3 +460,51 @@ def test_dense_auto_path_layouts_and_edges(dev, B, Hkv, G, S, D, layout):
         sc = torch.matmul(q.double(), kr.transpose(2, 3)) * scale
         assert_close(o, torch.matmul(torch.softmax(sc, -1), vr), what="oracle")
         assert_close(lse, torch.logsumexp(sc, -1)[..., 0], atol=1e-4, what="oracle lse")
+
+
+def _assert_same_with_nonfinite(got, ref, what):
+    """Infinities and NaN where the reference has them, the rest within ATOL."""
+    g, r = got.detach().cpu().double(), ref.detach().cpu().double().reshape(got.shape)
+    assert torch.equal(torch.isnan(g), torch.isnan(r)), f"{what}: NaN positions"
+    inf = torch.isinf(r)
+    assert torch.equal(torch.isinf(g), inf) and torch.equal(g[inf], r[inf]), f"{what}: infinities"
+    assert_close(g, r, what=what, mask=torch.isfinite(r))
+
+
+# An infinite V element of a used token makes its output element infinite, both
+# signs together or a NaN make it NaN, and nothing else changes; on every kernel
+# that a decode can take (stream-K from 4096 groups here, the chunked one below).
+# Scores are within +-6, so every probability is far above fp16's smallest.
+@pytest.mark.parametrize("D,G", [(64, 4), (128, 4), (128, 16), (256, 8)])
+@pytest.mark.parametrize("S", [300, 16 * 2050 + 5])
+@pytest.mark.parametrize("paged", [False, True])
+def test_decode_infinite_v_elements(dev, paged, S, D, G):
+    g = torch.Generator().manual_seed(S + D + G)
+    Hkv, page = 2, 16
+    q = torch.randn(1, Hkv * G, 1, D, generator=g).half()
+    K = torch.randn(1, Hkv, S, D, generator=g).clamp(-2, 2).half()
+    V = torch.randn(1, Hkv, S, D, generator=g).half()
+    q *= 6 * math.sqrt(D) / torch.matmul(q.float(), K.float().repeat_interleave(G, 1)
+                                         .transpose(2, 3)).abs().amax(-1, keepdim=True).half()
+    inf = float("inf")
+    top = torch.matmul(q[0, 0].float(), K[0, 0].float().t()).argmax()  # head 0's largest P
+    V[0, 0, top, 0] = inf
+    for i in range(12):  # every dim class, positions all over the cache
+        V[0, i % 2, (37 * i + i * S // 13) % S, 1 + 5 * i] = inf if i % 3 else -inf
+    V[0, 1, S - 1, 2], V[0, 1, S // 2, 2] = inf, -inf
+    V[0, 1, S // 3, 4] = float("nan")
+    ref, rl = naive.decode(q, K, V, 1 / math.sqrt(D), G)
+    if paged:
+        indptr, indices, last, P = syn.block_table(g, [S], page)
+        pool = torch.full((P, 2, Hkv, page, D), inf).half()  # rows past S hold anything
+        for i, pg_id in enumerate(indices.tolist()):
+            n = min(page, S - i * page)
+            pool[pg_id, 0, :, :n] = K[0, :, i * page:i * page + n]
+            pool[pg_id, 1, :, :n] = V[0, :, i * page:i * page + n]
+        o, lse = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev),
+                                                 indices.to(dev), last.to(dev), return_lse=True)
+    else:
+        o, lse = dec.flash_attention_decode(q.to(dev), K.to(dev), V.to(dev), 1 / math.sqrt(D), G,
+                                            return_lse=True)
+    _assert_same_with_nonfinite(o, ref, f"paged={paged} S={S} D={D} G={G}")
+    assert_close(lse, rl, atol=1e-4, what="lse")
