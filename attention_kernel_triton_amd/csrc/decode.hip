@@ -80,33 +80,63 @@ struct SplitParams {
   int S;             // dense: cache length
   int page_size;
   int num_pool_pages;
+  int total_pages;   // paged: entries of indices
   int n_hg;          // head groups per kv head (dense / paged)
   int chunk;         // tokens per chunk (dense / paged), multiple of 64
   float qk_scale;    // softmax_scale * log2(e)
 };
 
-__device__ __forceinline__ int paged_len(const int32_t* __restrict__ indptr,
-                                         const int32_t* __restrict__ last_len, int b, int P) {
-  int np = indptr[b + 1] - indptr[b];
-  if (np <= 0) return 0;
-  int ll = min(max(last_len[b], 0), P);
-  return (np - 1) * P + ll;
+// Page tables.  Sequence b owns positions [s(b), s(b + 1)) of kv_page_indices,
+// where s is indptr clamped to [0, total_pages] and made non-decreasing (a
+// running maximum), as in the stream-K kernel: whatever indptr holds, no
+// position lies outside the table and the sequences' chunks together are at
+// most the paged_grid_x that the partials are sized for.
+__device__ __forceinline__ int clamp_pos(const SplitParams& p, int v) {
+  return min(max(v, 0), p.total_pages);
+}
+// Tokens of a sequence of np pages whose last page holds `last` tokens.
+__device__ __forceinline__ int pages_len(const SplitParams& p, int np, int last) {
+  return np > 0 ? (np - 1) * p.page_size + min(max(last, 0), p.page_size) : 0;
+}
+// Wave-cooperative: lane l's sequence base + l, its first position and length
+// (0 past the batch).  `top`: the running maximum so far.  Consistent entries
+// are their own running maximum, so the scan runs only for others (batches past
+// 1024 walk the whole table per workgroup: always scanning cost them 11-15%).
+__device__ __forceinline__ void wave_sequences(const SplitParams& p, int base, int& top, int& start,
+                                               int& len) {
+  const int lane = threadIdx.x & 63;
+  const int bb = base + lane;
+  int lo = INT32_MAX, hi = INT32_MAX, last = 0;  // lanes past the batch
+  if (bb < p.B) {  // one round trip
+    lo = p.indptr[bb];
+    hi = p.indptr[bb + 1];
+    last = p.last_len[bb];
+  }
+  start = lo;
+  if (!__all(bb >= p.B || (lo >= top && hi >= lo && hi <= p.total_pages))) {  // wave-uniform
+    start = max(clamp_pos(p, lo), top);
+    hi = clamp_pos(p, hi);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int t = __shfl_up(start, off, 64);
+      if (lane >= off) start = max(start, t);
+    }
+  }
+  top = __builtin_amdgcn_readlane(start, 63);  // (past the batch: no entries follow)
+  len = bb < p.B ? pages_len(p, max(hi - start, 0), last) : 0;
 }
 
 // Wave-cooperative: find the sequence that owns global chunk x, where sequence
 // b owns ceil(len_b / chunk) consecutive chunks.  Returns false if x is past
 // the last chunk.
 __device__ bool locate_chunk(const SplitParams& p, int x, int& b_out, int& c_out, int& nch_out,
-                             int& len_out) {
+                             int& len_out, int& start_out) {
   const int lane = threadIdx.x & 63;
-  int carry = 0;
+  int carry = 0, top = 0;
   for (int base = 0; base < p.B; base += 64) {
-    const int bb = base + lane;
-    int len = 0, n = 0;
-    if (bb < p.B) {
-      len = paged_len(p.indptr, p.last_len, bb, p.page_size);
-      n = (len + p.chunk - 1) / p.chunk;
-    }
+    int first, len;
+    wave_sequences(p, base, top, first, len);
+    const int n = (len + p.chunk - 1) / p.chunk;
     int incl = n;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -122,6 +152,7 @@ __device__ bool locate_chunk(const SplitParams& p, int x, int& b_out, int& c_out
       c_out = x - __shfl(start, src, 64);
       nch_out = __shfl(n, src, 64);
       len_out = __shfl(len, src, 64);
+      start_out = __shfl(first, src, 64);
       return true;
     }
     carry += __shfl(incl, 63, 64);
@@ -191,6 +222,7 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
   __shared__ int sm_len[TABLE ? kMaxTableB : 1];
   __shared__ int sm_ps[TABLE ? kMaxTableB : 1];
   __shared__ int sm_wtot[kWaves];
+  __shared__ int sm_bad[kWaves];  // the wave read an indptr entry that has to be clamped
   __shared__ int sm_next;
   // The next item's ticket (low word) and the count of items whose ticket
   // thread 0 has published (high word), written and read as one word.
@@ -246,13 +278,12 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     Item w = {};
     if constexpr (MODE == kModePaged) {
       int c, nch, len;
-      if (!locate_chunk(p, blockIdx.x, w.b, c, nch, len)) {
+      if (!locate_chunk(p, blockIdx.x, w.b, c, nch, len, w.pstart)) {
         w.b = -1;
         return w;
       }
       finish_item(w, blockIdx.x, blockIdx.y, c, nch, len);
-      w.pstart = p.indptr[w.b];
-      w.np = p.indptr[w.b + 1] - w.pstart;
+      w.np = (len + p.page_size - 1) / p.page_size;
     }
     return w;
   };
@@ -738,14 +769,20 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     // must read 0 before any wave can compare it (barriers below).
     if (tid == 0) sm_tick = 0;
     if constexpr (TABLE) {
-      // Chunk prefix over sequences (block-wide exclusive scan), once.
+      // Chunk prefix over sequences (block-wide exclusive scan), once, from
+      // entries taken as they are: a consistent table needs no running
+      // maximum.  If any wave saw an entry that does, wave 0 builds it again.
       int carry = 0;
+      bool bad = false;
       for (int base = 0; base < p.B; base += kThreads) {
         const int bb = base + tid;
         int n = 0, len = 0, ps = 0;
         if (bb < p.B) {
           ps = p.indptr[bb];
-          len = paged_len(p.indptr, p.last_len, bb, p.page_size);
+          const int pe = p.indptr[bb + 1];
+          const bool ok = ps >= 0 && pe >= ps && pe <= p.total_pages;
+          bad |= !ok;
+          len = ok ? pages_len(p, pe - ps, p.last_len[bb]) : 0;
           n = (len + p.chunk - 1) / p.chunk;
         }
         int incl = n;
@@ -771,7 +808,32 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
         __syncthreads();
       }
       if (tid == 0) sm_cs[p.B] = carry;
+      if (const bool any_bad = __any(bad); lane == 0) sm_bad[wave] = any_bad;
       __syncthreads();
+      if (sm_bad[0] | sm_bad[1] | sm_bad[2] | sm_bad[3]) {  // workgroup-uniform
+        if (wave == 0) {
+          int cs = 0, top = 0;
+          for (int base = 0; base < p.B; base += 64) {
+            int first, len;
+            wave_sequences(p, base, top, first, len);
+            const int n = (len + p.chunk - 1) / p.chunk;
+            int incl = n;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+              const int t = __shfl_up(incl, off, 64);
+              if (lane >= off) incl += t;
+            }
+            if (base + lane < p.B) {
+              sm_cs[base + lane] = cs + incl - n;
+              sm_len[base + lane] = len;
+              sm_ps[base + lane] = first;
+            }
+            cs += __shfl(incl, 63, 64);
+          }
+          if (lane == 0) sm_cs[p.B] = cs;
+        }
+        __syncthreads();
+      }
       n_items = sm_cs[p.B] * Y;
       // Sequences without tokens have no items: their rows are written here.
       for (int bb = blockIdx.x; bb < p.B; bb += gridDim.x)
@@ -914,10 +976,14 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     }
   } else {
     if constexpr (MODE == kModePaged) {
-      // Sequences without tokens have no chunk (grid.x >= B).
-      if (blockIdx.y == 0 && (int)blockIdx.x < p.B &&
-          paged_len(p.indptr, p.last_len, blockIdx.x, p.page_size) == 0)
-        zero_sequence(blockIdx.x);
+      // Sequences without tokens have no chunk (grid.x >= B).  (Their entries
+      // alone say so in a consistent table; in another one a sequence that only
+      // the running maximum leaves without pages keeps its rows unwritten.)
+      if (blockIdx.y == 0 && (int)blockIdx.x < p.B) {
+        const int b = blockIdx.x;
+        const int np = clamp_pos(p, p.indptr[b + 1]) - clamp_pos(p, p.indptr[b]);
+        if (pages_len(p, np, p.last_len[b]) == 0) zero_sequence(b);
+      }
     }
     it = resolve_block();
     if (it.b < 0) return;  // workgroup-uniform
@@ -1389,6 +1455,7 @@ int paged_decode_impl(const void* q, const void* kv_cache, const int32_t* kv_pag
   p.B = (int)batch; p.Hq = (int)num_q_heads; p.Hkv = (int)num_kv_heads; p.G = G;
   p.page_size = (int)page_size;
   p.num_pool_pages = (int)(num_pool_pages < (1ll << 31) ? num_pool_pages : (1ll << 31) - 1);
+  p.total_pages = (int)total_pages;
   p.n_hg = n_hg;
   p.chunk = (int)chunk;
   p.qk_scale = softmax_scale * kLog2e;

@@ -181,7 +181,9 @@ int akt_decode_fwd(const void* q, const void* k, const void* v, void* o, float* 
  *   kv_last_page_len [batch]: int32 CSR page table.  Sequence b has
  *   (indptr[b+1]-indptr[b]-1)*page_size + last_page_len[b] tokens (0 when it
  *   has no pages; last_page_len is clamped to [0, page_size]).  Page ids
- *   outside [0, num_pool_pages) are skipped.
+ *   outside [0, num_pool_pages) are skipped.  indptr must lie in
+ *   [0, total_pages] and not decrease; where it does not, its entries are taken
+ *   clamped and as a running maximum, and nothing outside the arrays is touched.
  *   o: contiguous [batch, num_q_heads, head_dim]; lse optional [batch, num_q_heads].
  *   chunk_tokens 0 (automatic) runs the stream-K kernel when batch <= 1024,
  *   page_size is a multiple of 16 and the launch is not small: every wave of the launch takes a fixed

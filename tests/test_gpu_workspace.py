@@ -25,7 +25,7 @@ def _dirty_workspace(nbytes, dev):
     return ws
 
 
-def _paged_capi(p, ws):
+def _paged_capi(p, ws, chunk=0):
     lib = N.load()
     B, Hq, D = p.q.shape[0], p.q.shape[1], p.q.shape[-1]
     P, _, Hkv, page, _ = p.pool.shape
@@ -34,16 +34,16 @@ def _paged_capi(p, ws):
     rc = lib.akt_decode_paged_fwd(N.ptr(p.q), N.ptr(p.pool), N.ptr(p.indptr), N.ptr(p.indices),
                                   N.ptr(p.last_len), N.ptr(o), N.ptr(lse), B, Hq, Hkv, D, page,
                                   p.indices.numel(), P, N.strides(p.q), N.strides(p.pool),
-                                  1.0 / math.sqrt(D), 0, N.ptr(ws), ws.numel(),
+                                  1.0 / math.sqrt(D), chunk, N.ptr(ws), ws.numel(),
                                   N.stream_of(p.q))
     N.check(rc, "akt_decode_paged_fwd")
     return o, lse
 
 
-def _need(p):
+def _need(p, chunk=0):
     B, Hq, D = p.q.shape[0], p.q.shape[1], p.q.shape[-1]
     _, _, Hkv, page, _ = p.pool.shape
-    return N.load().akt_decode_paged_workspace_size(B, Hq, Hkv, D, page, p.indices.numel(), 0)
+    return N.load().akt_decode_paged_workspace_size(B, Hq, Hkv, D, page, p.indices.numel(), chunk)
 
 
 @pytest.mark.parametrize("case", ["config3", "over_32768_units"])
@@ -105,3 +105,72 @@ def test_paged_auto_path_on_dirty_workspace_matches_oracle(dev, lens, page, Hq, 
         lerr = float((lse.cpu().double() - rl).abs().max())
         assert err <= 2e-3 and lerr <= 1e-4, (err, lerr)
         assert int(ws[: N.WORKSPACE_ZERO_BYTES].count_nonzero()) == 0
+
+
+# Page tables that break the contract (indptr outside [0, total_pages] or
+# decreasing): every kernel takes the entries clamped to the table and made
+# non-decreasing, reads no position outside it and stores no partial past the
+# workspace that the table's size asks for.
+_LOW, _HIGH = -(1 << 31), (1 << 31) - 1
+_TABLES = {
+    "consistent": [0, 3, 3, 9, 12, 17, 20],
+    "negative": [-5, 3, 3, 9, 12, 17, 20],
+    "past the end": [0, 3, 3, 9, 12, 17, 999],
+    "decreasing": [0, 9, 4, 2, 12, 17, 20],
+    "overlapping": [0, 20, 0, 20, 0, 20, 20],
+    "extremes": [_LOW, _HIGH, _LOW, 5, _HIGH, _LOW, 20],
+    "late start": [7, 7, 9, 8, 12, 40, 13],
+}
+
+
+def _check_table(dev, indptr, page, Hkv, chunk, T, seed):
+    from oracle import naive
+
+    g = torch.Generator().manual_seed(seed)
+    B, G, D = len(indptr) - 1, 4, 64
+    pool = torch.randn(T + 3, 2, Hkv, page, D, generator=g).half()
+    indices = torch.randperm(T + 3, generator=g)[:T].to(torch.int32)
+    last = torch.randint(-1, page + 2, (B,), generator=g).to(torch.int32)
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    raw = torch.tensor(indptr, dtype=torch.int64)
+    start = raw.clamp(0, T).cummax(0).values.to(torch.int32)
+    ro, rl = naive.naive_paged_attention(q, pool, start, indices, last)
+    p = syn.Paged(q.to(dev), pool.to(dev), raw.to(torch.int32).to(dev), indices.to(dev),
+                  last.to(dev), None)
+    need = _need(p, chunk)
+    buf = torch.full((need + (1 << 20),), 0xA5, dtype=torch.uint8, device=dev)
+    buf[: min(N.WORKSPACE_ZERO_BYTES, need)] = 0
+    # Past 1024 sequences the rows of one that only the running maximum leaves
+    # without pages are not written.
+    keep = torch.ones(B, dtype=torch.bool)
+    if B > 1024:
+        keep = (raw[1:] <= raw[:-1]) | (start[1:] > start[:-1])
+    for _ in range(2):
+        o, lse = _paged_capi(p, buf[:need], chunk)
+        torch.cuda.synchronize(dev)
+        o, lse = o.cpu().double()[keep], lse.cpu().double()[keep]
+        assert float((o - ro[keep]).abs().max()) <= 2e-3
+        empty = torch.isinf(rl[keep])
+        assert torch.equal(torch.isinf(lse), empty)
+        assert float((lse - rl[keep])[~empty].abs().max()) <= 1e-4
+        assert int(buf[: min(N.WORKSPACE_ZERO_BYTES, need)].count_nonzero()) == 0
+        assert bool((buf[need:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("page,Hkv,chunk", [
+    (16, 2, 0), (32, 2, 0), (16, 2, 128), (16, 2, 640), (8, 2, 0),  # chunked kernel
+    (16, 32, 0), (64, 32, 0),                                       # stream-K kernel
+])
+@pytest.mark.parametrize("table", list(_TABLES))
+def test_paged_tables_outside_the_contract_stay_inside_their_arrays(dev, table, page, Hkv, chunk):
+    _check_table(dev, _TABLES[table], page, Hkv, chunk, 20, len(table) + page)
+
+
+@pytest.mark.parametrize("page", [16, 8])
+def test_paged_tables_outside_the_contract_past_1024_sequences(dev, page):
+    g = torch.Generator().manual_seed(page)
+    B = 1100
+    indptr = [0] + torch.randint(0, 30, (B,), generator=g).cumsum(0).tolist()
+    T = indptr[-1]
+    indptr[3], indptr[500], indptr[700] = -9, indptr[400], _HIGH
+    _check_table(dev, indptr, page, 2, 0, T, page)
