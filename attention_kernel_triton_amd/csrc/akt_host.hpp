@@ -67,18 +67,20 @@ inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
 constexpr int kMaxResidentDevices = 64;
 
-// Workgroups of `kernel` (blocks of `threads`) that fit the current device at
+// Workgroups of `Kernel` (blocks of `threads`) that fit the current device at
 // once (occupancy x CUs), cached per kernel instance and device; 0 if the
-// queries fail.
-template <typename Kernel>
-int resident_blocks(Kernel kernel, int threads) {
+// queries fail.  (The kernel is a template argument because instances of one
+// kernel template share a type: a cache per type would answer for all of them
+// with the first one launched.)
+template <auto Kernel>
+int resident_blocks(int threads) {
   static std::atomic<int> cache[kMaxResidentDevices];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxResidentDevices) return 0;
   int v = cache[dev].load(std::memory_order_relaxed);
   if (v > 0) return v;
   int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kernel, threads, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)Kernel, threads, 0) !=
           hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;

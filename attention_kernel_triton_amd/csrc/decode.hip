@@ -1029,10 +1029,10 @@ int pick_gt(int G, int D) {
 // min(items, resident workgroups); `grid` carries the item upper bound in x.
 template <int D, int GT, int MODE, bool ALIGNED, int GPW, bool PERSIST>
 int launch_split(const SplitParams& p, dim3 grid, hipStream_t st) {
-  auto kernel = split_kernel<D, GT, MODE, ALIGNED, GPW, PERSIST>;
+  constexpr auto kernel = split_kernel<D, GT, MODE, ALIGNED, GPW, PERSIST>;
   if (PERSIST) {
     const int64_t items = (int64_t)grid.x * grid.y;
-    const int cap = resident_blocks(kernel, kThreads);
+    const int cap = resident_blocks<kernel>(kThreads);
     if (cap <= 0) return set_error(AKT_ERR_HIP, "occupancy query failed");
     grid = dim3((unsigned)(items < cap ? items : cap), 1);
   }

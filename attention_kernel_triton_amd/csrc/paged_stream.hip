@@ -855,7 +855,7 @@ struct Stream {
   // Workgroups resident at once (at most kStreamMaxWaves waves); `unknown`
   // where no device can be queried.
   static int64_t blocks(int64_t unknown) {
-    const int64_t cap = resident_blocks(paged_stream_kernel<D, GT, DENSE>, kThreads);
+    const int64_t cap = resident_blocks<paged_stream_kernel<D, GT, DENSE>>(kThreads);
     return cap <= 0 ? unknown : std::min<int64_t>(cap, kStreamMaxWaves / kWaves);
   }
   static int64_t wave_cap() { return blocks(kStreamMaxWaves / kWaves) * kWaves; }
@@ -890,8 +890,8 @@ struct Stream {
   }
 
   static int launch(StreamParams p, hipStream_t st) {
-    auto kernel = paged_stream_kernel<D, GT, DENSE>;
-    if (resident_blocks(kernel, kThreads) <= 0)
+    constexpr auto kernel = paged_stream_kernel<D, GT, DENSE>;
+    if (resident_blocks<kernel>(kThreads) <= 0)
       return set_error(AKT_ERR_HIP, "occupancy query failed");
     p.wgs_log = DENSE ? dense_wgs_log((int64_t)p.Y * p.B, p.gpp) : -1;
     const int64_t g = DENSE ? dense_grid((int64_t)p.Y * p.B, p.gpp, p.wgs_log) : grid(p.N);

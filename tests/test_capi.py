@@ -4,12 +4,14 @@ No test here launches a kernel: argument checks return before any GPU call.
 """
 import ctypes as C
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
 import torch
 
 from attention_kernel_triton_amd import _native as N
+from attention_kernel_triton_amd.build import hipcc
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "akt_amd.h"
 
@@ -259,3 +261,38 @@ def test_host_layer_rejects_mismatched_k_and_v():
     nnz = torch.ones(1, 4, 1, dtype=torch.int32)
     with pytest.raises(ValueError, match="one shape"):
         _ops.sparse_decode(q, K, K[:, :1], ind, nnz, 0.1)
+
+
+def test_resident_workgroups_are_cached_per_kernel_instance(tmp_path):
+    """Kernel instances of one signature (all instances of a kernel template) keep
+    their own resident-workgroup count, whichever is asked for first.  Host code
+    alone: the runtime's queries are stand-ins that answer by kernel address."""
+    src = tmp_path / "resident.cpp"
+    src.write_text(r"""
+#include "akt_host.hpp"
+template <int N> void kernel(int) {}
+extern "C" hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+extern "C" hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  *v = 256;
+  return hipSuccess;
+}
+extern "C" hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int,
+                                                                   size_t) {
+  *n = f == (const void*)kernel<1> ? 1 : (f == (const void*)kernel<2> ? 2 : 3);
+  return hipSuccess;
+}
+int main() {
+  for (int turn = 0; turn < 2; ++turn) {
+    if (akt::resident_blocks<kernel<2>>(256) != 512) return 2;
+    if (akt::resident_blocks<kernel<1>>(256) != 256) return 1;
+    if (akt::resident_blocks<kernel<3>>(256) != 768) return 3;
+  }
+  return 0;
+}
+""")
+    exe = tmp_path / "resident"
+    csrc = HEADER.parents[1] / "attention_kernel_triton_amd" / "csrc"
+    subprocess.run([hipcc(), "-x", "c++", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", f"-I{csrc}",
+                    f"-I{Path(hipcc()).parents[1] / 'include'}", str(src), "-o", str(exe)],
+                   check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
