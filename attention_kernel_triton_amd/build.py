@@ -25,7 +25,11 @@ ARCH = "gfx950"
 # Packed FP32 instructions are switched off for all device code.  The atomic
 # optimizer is off: every atomic here is issued by one lane, and the optimizer's
 # rewrite of a uniform-address atomic reads the returned value at once, which
-# makes the wave wait (vmcnt(0)) for every load it has in flight.
+# makes the wave wait (vmcnt(0)) for every load it has in flight.  Vector registers
+# spill to scratch, never to AGPRs: with a 4-register query fragment spilled partly
+# to each, this compiler reloaded the scratch words into the fragment's AGPRs and
+# left the word that waited in an AGPR out (D = 256 with 8 heads to a unit, the
+# chunked kernel's 256-token instance: a stale word of q from the second item on).
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
@@ -36,6 +40,7 @@ COMMON_FLAGS = [
     "-Wno-pass-failed",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-mllvm", "-amdgpu-atomic-optimizer-strategy=None",
+    "-mllvm", "-amdgpu-spill-vgpr-to-agpr=0",
 ]
 # Extra flags of single sources.  prefill_wide.hip holds the head-dim 192 and 256
 # prefill instances (one wave per SIMD): LLVM's iterative ILP scheduler runs them
