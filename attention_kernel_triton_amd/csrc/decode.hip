@@ -563,7 +563,6 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     const int nch = w.nch;
     auto combine = [](float& M, float& L, float& E, float4_t& A, float m, float l, float e,
                       float4_t a) {
-      if (m == AKT_NEG_INF) return;
       if (m > M) {
         const float s = fast_exp2(M - m);  // 0 while M = -inf (A, L, E are 0 then)
         A *= s;
@@ -571,7 +570,9 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
         E *= s;
         M = m;
       }
-      const float f = fast_exp2(m - M);
+      // A state without usable tokens (m = -inf, sums 0) adds nothing; one whose
+      // every score is NaN has m = -inf too, and its NaN sums come through.
+      const float f = fast_exp2(m - (M == AKT_NEG_INF ? 0.f : M));
       A += f * a;
       L += f * l;
       E += f * e;
@@ -703,14 +704,15 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
       for (int w = 0; w < kWaves; ++w) M = fmaxf(M, sm_m[w][h]);
       L = E = 0.f;
       O = float4_t{0.f, 0.f, 0.f, 0.f};
-      if (M != AKT_NEG_INF) {
+      // A wave without usable tokens has weight and sums 0; NaN sums (a NaN in
+      // every score of a wave leaves its maximum at -inf) come through.
+      const float Mu = M == AKT_NEG_INF ? 0.f : M;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-          const float f = fast_exp2(sm_m[w][h] - M);
-          L += f * sm_l[w][h];
-          E += f * sm_e[w][h];
-          O += f * sm_o4[w * NV + vec];
-        }
+      for (int w = 0; w < kWaves; ++w) {
+        const float f = fast_exp2(sm_m[w][h] - Mu);
+        L += f * sm_l[w][h];
+        E += f * sm_e[w][h];
+        O += f * sm_o4[w * NV + vec];
       }
     };
     if (it.direct) {

@@ -672,7 +672,6 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   // Adds one state (its ml row and this lane's vectors).
   auto merge_add = [&](float4_t ml, const float4_t (&ov)[NVL]) __attribute__((always_inline)) {
     const float m = ml[0];
-    if (m == AKT_SNEG_INF) return;
     if (m > M) {
       const float sc = fast_exp2(M - m);  // 0 while M = -inf (Acc, L, E are 0 then)
 #pragma unroll
@@ -681,7 +680,9 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
       E *= sc;
       M = m;
     }
-    const float f = fast_exp2(m - M);
+    // A state without usable tokens (m = -inf, sums 0) adds nothing; one whose
+    // every score is NaN has m = -inf too, and its NaN sums come through.
+    const float f = fast_exp2(m - (M == AKT_SNEG_INF ? 0.f : M));
 #pragma unroll
     for (int i = 0; i < NVL; ++i) Acc[i] += f * ov[i];
     L += f * ml[1];

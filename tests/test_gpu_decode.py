@@ -508,3 +508,33 @@ def test_decode_infinite_v_elements(dev, paged, S, D, G):
                                             return_lse=True)
     _assert_same_with_nonfinite(o, ref, f"paged={paged} S={S} D={D} G={G}")
     assert_close(lse, rl, atol=1e-4, what="lse")
+
+
+# A query head with a NaN has NaN outputs, whatever kernel and however many waves
+# its tokens take, and no other head changes.
+@pytest.mark.parametrize("D,G", [(64, 1), (128, 4), (128, 16), (256, 8)])
+@pytest.mark.parametrize("paged,chunk,lens", [
+    (True, 0, [1, 16, 17, 300, 0]), (True, 128, [1, 130, 700]),     # chunked kernel
+    (True, 0, [5, 16 * 1100, 16 * 1100 - 3]),                       # stream-K kernel
+    (False, 0, [1]), (False, 0, [300]), (False, 0, [16 * 2100]),    # dense
+])
+def test_decode_nan_query_head(dev, paged, chunk, lens, D, G):
+    g = torch.Generator().manual_seed(sum(lens) + D + G)
+    Hkv, B = 2, len(lens)
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    bad = Hkv * G - 1
+    dirty = q.clone()
+    dirty[:, bad, 0, D // 3] = float("nan")
+    if paged:
+        indptr, indices, last, P = syn.block_table(g, lens, 16)
+        pool = torch.randn(P, 2, Hkv, 16, D, generator=g).half()
+        args = [t.to(dev) for t in (pool, indptr, indices, last)]
+        run = lambda x: _ops.decode_paged(x.to(dev), *args, chunk_tokens=chunk)  # noqa: E731
+    else:
+        K, V = (torch.randn(B, Hkv, lens[0], D, generator=g).half().to(dev) for _ in range(2))
+        run = lambda x: _ops.decode(x.to(dev), K, V, 0.1)[:, :, 0]  # noqa: E731
+    want, got = run(q), run(dirty)
+    nonempty = torch.tensor(lens, device=dev) > 0
+    assert torch.isnan(got[nonempty, bad]).all()
+    assert torch.equal(got[:, :bad], want[:, :bad])
+    assert torch.equal(got[~nonempty], want[~nonempty])
