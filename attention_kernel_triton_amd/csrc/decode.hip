@@ -354,7 +354,7 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
 
   // Computes the row addresses of group g and issues its K/V loads.  Every
   // load is issued unconditionally (a lane whose token is unusable reads the
-  // unit's own q row instead, which is always mapped and finite) so that no
+  // unit's own q row instead, which is always mapped) so that no
   // load sits behind a branch: the wait counts then only cover the buffer
   // being consumed.  Index and page lookups read clamped, in-range entries.
   // Paged caches of whole 16-token groups: a group is the 16 rows from row
@@ -364,12 +364,11 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
   // 4R + 2 (c16 / 8) + i, plus v_sb bytes per i) at dims dim0.
   const int dim0 = (D == 64) ? 8 * (c16 & 7) : VDIM * c16;
   const int tt0 = (D == 64) ? (4 * R + 2 * (c16 >> 3)) : 4 * R;
-  uint32_t lane_kofs = 0, lane_qofs = 0, lane_v0ofs = 0, lane_dofs = 0;
+  uint32_t lane_kofs = 0, lane_qofs = 0, lane_v0ofs = 0;
   if constexpr (MODE == kModePaged && ALIGNED) {
     lane_kofs = (uint32_t)(c16 * (int)p.k_sb + R * KPL) * 2u;
     lane_qofs = (uint32_t)(R * KPL) * 2u;
     lane_v0ofs = (uint32_t)(tt0 * (int)p.v_sb + dim0) * 2u;
-    lane_dofs = (uint32_t)dim0 * 2u;
   }
   auto issue = [&](const IssueCtx& cx, int g, Buf& bf) {
     const int t1 = cx.t1;
@@ -377,10 +376,9 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     if constexpr (MODE == kModePaged && ALIGNED) {
       // The usable tokens of the group are a prefix (positions below t1 of
       // a valid page).  K rows past it lie inside the page and load as they
-      // are (their scores are masked); the V rows of unusable tokens re-read
-      // the group's first row, a usable token whenever the group has one; a
-      // group without usable tokens (or with an invalid page id) reads the
-      // unit's q row instead, which is always mapped and finite.
+      // are (their scores are masked), those of an invalid page id the unit's q
+      // row, which is always mapped.  V rows of unusable tokens are read past
+      // the resource's end: zeros, and no memory touched.
       const int k = (g - cx.g_begin - wave) / kWaves;
       const int page = __builtin_amdgcn_readlane(cx.page_pref, k);
       const int gslot = __builtin_amdgcn_readlane(cx.slot_pref, k);
@@ -392,15 +390,18 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
       const uint32_t ko = page_ok ? lane_kofs : lane_qofs;
 #pragma unroll
       for (int s = 0; s < KS; ++s) bf.k[s] = ld16(kg + ko + 16 * s);
-      const char* vg = reinterpret_cast<const char*>(
-          nvalid > 0 ? cx.vb + (int64_t)page * p.v_sa + (int64_t)gslot * p.v_sb
-                     : cx.vb + cx.v_dummy);
+      const half_t* vg =
+          nvalid > 0 ? cx.vb + (int64_t)page * p.v_sa + (int64_t)gslot * p.v_sb : cx.vb + cx.v_dummy;
       const uint32_t vstep = (uint32_t)p.v_sb * 2u;
+      const auto vrs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)vg, 0, nvalid > 0 ? (int)(15u * vstep) + 2 * D : 0, kBufferWord3);
 #pragma unroll
       for (int i = 0; i < VTOK; ++i) {
-        const uint32_t vo = tt0 + i < nvalid ? lane_v0ofs + (uint32_t)i * vstep : lane_dofs;
+        const uint32_t vo = tt0 + i < nvalid ? lane_v0ofs + (uint32_t)i * vstep : 1u << 31;
 #pragma unroll
-        for (int j = 0; j < VLD; ++j) bf.v[i][j] = ld16(vg + vo + 16 * j);
+        for (int j = 0; j < VLD; ++j)
+          bf.v[i][j] = __builtin_bit_cast(
+              uint4_t, __builtin_amdgcn_raw_buffer_load_b128(vrs, vo + 16 * j, 0, 0));
       }
       return;
     }
@@ -464,8 +465,12 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
       for (int d = 0; d < VDIM; ++d) acc[h][d] = 0.f;
   };
 
-  // Scores, online softmax and P.V for a loaded group of the current item.
-  auto consume = [&](const Buf& bf) {
+  // Scores, online softmax and P.V for a loaded group of the current item.  The
+  // scores of unusable tokens are masked, and their V is zero: the q row that
+  // stands in for it could hold an infinity or NaN, and a probability of 0
+  // would not keep that out.  (Aligned paged groups load zeros; a branch here
+  // cost them up to 4%: B=1, 4000 tokens, Hq=32, Hkv=8, D=128 14.5 -> 15.1 us.)
+  auto consume = [&](Buf& bf) {
     const uint32_t vmask = bf.vmask;
     float4_t sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -502,6 +507,13 @@ __attribute__((amdgpu_waves_per_eu(split_min_waves<D, GT>(), 8))) void split_ker
     e_part += (pr[0] + pr[1]) + (pr[2] + pr[3]);
 
     // P.V
+    if (!(MODE == kModePaged && ALIGNED) && vmask != 0xffffu) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < VTOK; ++i)
+        if (!((vmask >> (tt0 + i)) & 1))
+#pragma unroll
+          for (int j = 0; j < VLD; ++j) bf.v[i][j] = uint4_t{0, 0, 0, 0};
+    }
     uint32_t vp[NPAIR][VDIM];
 #pragma unroll
     for (int q2 = 0; q2 < NPAIR; ++q2)

@@ -511,18 +511,22 @@ def test_decode_infinite_v_elements(dev, paged, S, D, G):
 
 
 # A query head with a NaN has NaN outputs, whatever kernel and however many waves
-# its tokens take, and no other head changes.
+# its tokens take, and no other head changes: neither the first head of a unit,
+# whose row stands in for rows that are not there, nor the last.
+@pytest.mark.parametrize("head", [0, -1])
 @pytest.mark.parametrize("D,G", [(64, 1), (128, 4), (128, 16), (256, 8)])
 @pytest.mark.parametrize("paged,chunk,lens", [
     (True, 0, [1, 16, 17, 300, 0]), (True, 128, [1, 130, 700]),     # chunked kernel
+    (True, 0, [3] * 1100),                                          # its batches past 1024
     (True, 0, [5, 16 * 1100, 16 * 1100 - 3]),                       # stream-K kernel
     (False, 0, [1]), (False, 0, [300]), (False, 0, [16 * 2100]),    # dense
 ])
-def test_decode_nan_query_head(dev, paged, chunk, lens, D, G):
+def test_decode_nan_query_head(dev, paged, chunk, lens, D, G, head):
     g = torch.Generator().manual_seed(sum(lens) + D + G)
     Hkv, B = 2, len(lens)
     q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
-    bad = Hkv * G - 1
+    bad = head % (Hkv * G)
+    rest = [h for h in range(Hkv * G) if h != bad]
     dirty = q.clone()
     dirty[:, bad, 0, D // 3] = float("nan")
     if paged:
@@ -536,5 +540,35 @@ def test_decode_nan_query_head(dev, paged, chunk, lens, D, G):
     want, got = run(q), run(dirty)
     nonempty = torch.tensor(lens, device=dev) > 0
     assert torch.isnan(got[nonempty, bad]).all()
-    assert torch.equal(got[:, :bad], want[:, :bad])
+    assert torch.equal(got[:, rest], want[:, rest])
     assert torch.equal(got[~nonempty], want[~nonempty])
+
+
+# The tokens past a sequence's end have probability 0, and no infinite or NaN V row
+# of a token that is there stands in for theirs: the last group's first row holds
+# an infinity, which reaches its own output element and nothing else.
+@pytest.mark.parametrize("D,G", [(64, 1), (128, 4), (128, 16), (256, 8)])
+@pytest.mark.parametrize("page,chunk,last", [(16, 0, 1), (16, 0, 7), (16, 256, 15), (48, 0, 5),
+                                             (8, 0, 3), (0, 0, 9)])
+def test_decode_infinite_v_at_the_start_of_a_partial_group(dev, page, chunk, last, D, G):
+    g = torch.Generator().manual_seed(10 * page + last + D + G)
+    Hkv, S = 2, 16 * 20 + last
+    q = torch.randn(1, Hkv * G, 1, D, generator=g).half()
+    K, V = (torch.randn(1, Hkv, S, D, generator=g).half() for _ in range(2))
+    K *= 0.25  # scores within a few units: every probability is well above fp16's smallest
+    V[0, 0, S - last, 3], V[0, 1, S - last, D - 1] = float("inf"), -float("inf")
+    scale = 1 / math.sqrt(D)
+    ref, rl = naive.decode(q, K, V, scale, G)
+    if page:
+        indptr, indices, lastl, P = syn.block_table(g, [S], page)
+        pool = torch.zeros(P, 2, Hkv, page, D).half()
+        for i, pg_id in enumerate(indices.tolist()):
+            n = min(page, S - i * page)
+            pool[pg_id, 0, :, :n] = K[0, :, i * page:i * page + n]
+            pool[pg_id, 1, :, :n] = V[0, :, i * page:i * page + n]
+        o, lse = _ops.decode_paged(q.to(dev), pool.to(dev), indptr.to(dev), indices.to(dev),
+                                   lastl.to(dev), return_lse=True, chunk_tokens=chunk)
+    else:
+        o, lse = _ops.decode(q.to(dev), K.to(dev), V.to(dev), scale, return_lse=True)
+    _assert_same_with_nonfinite(o, ref, f"page={page} last={last} D={D} G={G}")
+    assert_close(lse, rl, atol=1e-4, what="lse")
