@@ -1365,15 +1365,38 @@ static int64_t paged_grid_x(int64_t total_pages, int64_t page_size, int64_t chun
 // units 12.4 / 10.1, 500 in 1 24.7 / 21.1, 2000 in 8 16.5 / 14.0, 2448 in 128
 // 13.3 / 14.2, 4704 in 128 17.0 / 19.7; D = 256, 500 in 1 63.4 / 37.3, 2448 in
 // 128 18.2 / 18.8; D = 64, 1552 in 32 11.6 / 11.0, 2448 in 128 11.6 / 13.6.
+//
+// Those have four heads to a unit.  The split kernel's P.V runs on the VALU, in
+// time linear in the heads, and from 8 heads on at one wave per SIMD; the stream
+// kernel's runs on the matrix pipe, 16 heads at the cost of one, but its merge
+// grows with the heads and with the workgroups that a unit is spread over (as D
+// does).  So with many heads the small launches stay with it (even and ragged
+// lengths, graph replays, us, stream / split):
+// - D = 64, 16 heads: 64 groups in 16 units 8.1 / 12.7, 512 in 32 11.7 / 16.5,
+//   1936 in 96 12.9 / 30.8, 256 in 1 17.7 / 19.4 (worst: 2000 in 1 48.9 / 46.4);
+// - D = 64, 8 heads, from 512 groups up to 48 to a unit: 528 in 48 11.2 / 12.0,
+//   1040 in 24 11.7 / 12.5; but 144 in 48 10.0 / 9.0, 1504 in 16 14.9 / 13.8;
+// - D = 64, 4 heads, from 1536 groups in 32 units: 1728 in 48 11.5 / 12.1, 1736
+//   in 96 11.5 / 13.5, 1536 in 32 11.2 / 11.1; but 1024 in 64 10.9 / 10.3;
+// - D = 128, 16 heads, up to 12 groups to a unit: 200 in 16 15.4 / 17.1, 808 in
+//   96 16.3 / 18.4; but ragged 400 in 24 19.7 / 17.8, 1024 in 32 20.3 / 18.1, 512
+//   in 1 42.6 / 31.1.
+// D = 256 has no line that ragged lengths keep (8 heads, 48 units: 256 groups
+// 16.4 / 19.5, 216 16.4 / 15.3).
 static bool use_stream(int64_t chunk_tokens, int64_t batch, int64_t page_size,
-                       int64_t total_pages, int64_t Y) {
+                       int64_t total_pages, int64_t Y, int64_t D, int gt) {
   if (chunk_tokens != 0 || !paged_stream_eligible(batch, page_size, total_pages, Y)) return false;
-  return Y * total_pages * (page_size / 16) >= 2048 || batch * Y >= 128;
+  const int64_t groups = Y * total_pages * (page_size / 16), units = batch * Y;
+  if (groups >= 2048 || units >= 128) return true;
+  if (D == 64)
+    return gt == 16 || (gt == 8 && groups >= 512 && groups <= 48 * units) ||
+           (gt == 4 && groups >= 1536 && units >= 32);
+  return D == 128 && gt == 16 && units >= 8 && groups <= 12 * units;
 }
 
 static WsLayout paged_layout(int64_t batch, int64_t Y, int gt, int64_t D, int64_t page_size,
                              int64_t total_pages, int64_t chunk_tokens) {
-  if (use_stream(chunk_tokens, batch, page_size, total_pages, Y))
+  if (use_stream(chunk_tokens, batch, page_size, total_pages, Y, D, gt))
     return ws_layout(batch * Y, paged_stream_wave_cap((int)D, gt) + batch * Y, gt, D);
   const int64_t chunk = paged_chunk(chunk_tokens, total_pages, page_size, Y, batch);
   return ws_layout(batch * Y, paged_grid_x(total_pages, page_size, chunk, batch) * Y, gt, D);
@@ -1421,7 +1444,7 @@ int paged_decode_impl(const void* q, const void* kv_cache, const int32_t* kv_pag
   rc = check_workspace(wl, workspace, workspace_bytes);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
-  if (use_stream(chunk_tokens, batch, page_size, total_pages, Y)) {
+  if (use_stream(chunk_tokens, batch, page_size, total_pages, Y, D, gt)) {
     StreamParams sp = {};
     sp.q = (const half_t*)q;
     sp.kbase = (const half_t*)kv_cache;

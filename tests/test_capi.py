@@ -126,6 +126,28 @@ def test_automatic_chunk_length():
     assert dws(8, 64, 16, 1024, 64, 0) == dws(8, 64, 16, 1024, 64, 512)
 
 
+@pytest.mark.parametrize("batch,hq,hkv,dim,pages,stream", [
+    (4, 32, 8, 128, 255, False), (4, 32, 8, 128, 256, True),      # 2048 groups
+    (15, 32, 8, 128, 15, False), (16, 32, 8, 128, 16, True),      # 128 units
+    (1, 16, 1, 64, 1, True), (2, 128, 8, 64, 4, True),            # D = 64, 16 heads to a unit
+    (2, 64, 2, 64, 100, True),                                    # two units of 16 to a kv head
+    (6, 64, 8, 64, 63, False), (6, 64, 8, 64, 64, True),          # D = 64, 8 heads: 512 groups,
+    (2, 64, 8, 64, 96, True), (2, 64, 8, 64, 97, False),          # 48 to a unit
+    (4, 32, 8, 64, 191, False), (4, 32, 8, 64, 192, True),        # D = 64, 4 heads: 1536 groups
+    (31, 4, 1, 64, 1999, False),                                  # in 32 units
+    (1, 128, 8, 128, 12, True), (1, 128, 8, 128, 13, False),      # D = 128, 16 heads: 12 to a unit
+    (7, 16, 1, 128, 14, False),                                   # in 8 units
+    (12, 32, 8, 64, 120, False), (4, 128, 8, 256, 9, False),      # 4 heads below; D = 256
+])
+def test_automatic_paged_kernel(batch, hq, hkv, dim, pages, stream):
+    """Which kernel an automatic paged call takes on both sides of each line of its
+    rule (pages of 16 tokens: one group a page and kv head), read off the
+    workspace size: no chunk length asks for the stream-K kernel's."""
+    ws = N.load().akt_decode_paged_workspace_size
+    auto = ws(batch, hq, hkv, dim, 16, pages, 0)
+    assert (auto not in [ws(batch, hq, hkv, dim, 16, pages, c) for c in (128, 256, 512, 640)]) == stream
+
+
 def test_automatic_sparse_split_count():
     """Sparse rows get as many splits as fit one round of ~512 resident workgroups,
     at most 8 and at most one per 64 index slots of l_max; the workspace size shows
