@@ -359,14 +359,15 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sparse_kernel(SparseParams p) {
   float4_t O = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < kSpWaves; ++i) M = fmaxf(M, sm_m[i]);
-  if (M != AKT_NEG_INF) {
+  // A wave without usable tokens has weight and sums 0; NaN sums (a NaN in every
+  // score of a wave leaves its maximum at -inf) come through.
+  const float Mu = M == AKT_NEG_INF ? 0.f : M;
 #pragma unroll
-    for (int i = 0; i < kSpWaves; ++i) {
-      const float f = fast_exp2(sm_m[i] - M);
-      L += f * sm_l[i];
-      E += f * sm_e[i];
-      O += f * sm_o[i][vec];
-    }
+  for (int i = 0; i < kSpWaves; ++i) {
+    const float f = fast_exp2(sm_m[i] - Mu);
+    L += f * sm_l[i];
+    E += f * sm_e[i];
+    O += f * sm_o[i][vec];
   }
   auto write_out = [&]() __attribute__((always_inline)) {
     const float inv = L > 0.f ? 1.0f / L : 0.f;
@@ -405,7 +406,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sparse_kernel(SparseParams p) {
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const float m = ml[i][0];
-      if (c0 + i >= p.n_split || m == AKT_NEG_INF) continue;
+      if (c0 + i >= p.n_split) continue;
       if (m > M) {
         const float s = fast_exp2(M - m);  // 0 while M = -inf (O, L, E are 0 then)
         O *= s;
@@ -413,7 +414,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sparse_kernel(SparseParams p) {
         E *= s;
         M = m;
       }
-      const float f = fast_exp2(m - M);
+      const float f = fast_exp2(m - (M == AKT_NEG_INF ? 0.f : M));
       O += f * ov[i];
       L += f * ml[i][1];
       E += f * ml[i][2];

@@ -338,6 +338,41 @@ def test_sparse_splits_merge_deterministically(dev):
         assert torch.equal(o, o0) and torch.equal(lse, l0)
 
 
+# A query head with a NaN has NaN outputs however many waves and splits its tokens
+# take (one token leaves three waves without any), and no other head changes.
+@pytest.mark.parametrize("kind", ["dense", "paged", "magicpig"])
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("n,splits", [(1, 1), (5, 3), (200, 1), (200, 3), (700, 0), (700, 12)])
+def test_sparse_nan_query_head(dev, kind, D, n, splits):
+    g = torch.Generator().manual_seed(n + splits + D)
+    B, Hkv, G, S = 2, 2, 2, 1000
+    Hq = Hkv * G
+    q = torch.randn(B, Hq, 1, D, generator=g).half()
+    ind = torch.stack([torch.randperm(S, generator=g)[:n].sort().values for _ in range(B * Hq)])
+    ind = ind.reshape(B, Hq, n).to(torch.int32).to(dev)
+    nnz = torch.full((B, Hq, 1), n, dtype=torch.int32, device=dev)
+    if kind == "dense":
+        K, V = (torch.randn(B, Hkv, S, D, generator=g).half().to(dev) for _ in range(2))
+        run = lambda x: _ops.sparse_decode(x.to(dev), K, V, ind, nnz, 0.1,  # noqa: E731
+                                           num_splits=splits)[:, :, 0]
+    else:
+        indptr, indices, _, P = syn.block_table(g, [S] * B, 16)
+        pool = torch.randn(P, 2, Hkv, 16, D, generator=g).half().to(dev)
+        lsh = {}
+        if kind == "magicpig":
+            lsh = {"lsh_k": torch.full((B, Hq), 10.0, device=dev),
+                   "lsh_l": torch.full((B, Hq), 150.0, device=dev)}
+        run = lambda x: _ops.sparse_decode_paged(  # noqa: E731
+            x.to(dev), pool, indptr.to(dev), indices.to(dev), ind, nnz, num_splits=splits, **lsh)
+    bad = 1
+    dirty = q.clone()
+    dirty[:, bad, 0, D // 3] = float("nan")
+    want, got = run(q).reshape(B, Hq, D), run(dirty).reshape(B, Hq, D)
+    rest = [h for h in range(Hq) if h != bad]
+    assert torch.isnan(got[:, bad]).all()
+    assert torch.equal(got[:, rest], want[:, rest])
+
+
 def _reference_harness_fixture(dev):
     """The reference harness's sparse paged / MagicPIG case at its own shape
     (sparsetoken_decode_flash_attention_redundant_var_len_paged.py:296-330,
