@@ -112,8 +112,9 @@ def test_automatic_chunk_length():
     groups runs the stream-K kernel: its workspace holds one partial slot per
     (wave + unit), with the waves at their 4096 maximum where no device can be
     queried (this CPU-only process).  Explicit chunk lengths keep the chunked
-    kernel's layout, and dense decode keeps choosing its chunk (512 tokens for
-    config 2)."""
+    kernel's layout.  Automatic dense decode takes room for the stream-K kernel
+    (here on 256 workgroups, as assumed without a device) and, since its size
+    does not know the row strides, for the chunked one."""
     lib = N.load()
     ws = lib.akt_decode_paged_workspace_size
     # config 3: 32 sequences x 8 kv heads = 256 units of 4 heads, D = 128
@@ -121,9 +122,14 @@ def test_automatic_chunk_length():
     assert ws(32, 32, 8, 128, 16, 7208, 0) != ws(32, 32, 8, 128, 16, 7208, 640)
     # pages of 8 tokens (not whole groups) keep the chunked kernel at 256 tokens
     assert ws(32, 32, 8, 128, 8, 7208, 0) == ws(32, 32, 8, 128, 8, 7208, 256)
-    # config 2 (dense, 8 x 1024 tokens, 16 kv heads) stays at 512
     dws = lib.akt_decode_workspace_size
-    assert dws(8, 64, 16, 1024, 64, 0) == dws(8, 64, 16, 1024, 64, 512)
+    # config 2 (dense, 8 x 1024 tokens, 16 kv heads): two workgroups to each of 128
+    # units, as many partials as two 512-token chunks
+    assert dws(8, 64, 16, 1024, 64, 0) == _ws(128, 256, 4, 64) == dws(8, 64, 16, 1024, 64, 512)
+    # 8 units of 876 groups: 32 workgroups each, more than 28 chunks of 512 tokens
+    assert dws(1, 32, 8, 14001, 128, 0) == _ws(8, 256, 4, 128) > dws(1, 32, 8, 14001, 128, 512)
+    # 8 units of 63 groups, below the stream-K kernel's line: 128-token chunks
+    assert dws(1, 32, 8, 1000, 128, 0) == _ws(8, 64, 4, 128) == dws(1, 32, 8, 1000, 128, 128)
 
 
 @pytest.mark.parametrize("batch,hq,hkv,dim,pages,stream", [

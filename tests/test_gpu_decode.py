@@ -8,7 +8,7 @@ from attention_kernel_triton_amd import decode_flash_attention_redundant as dec
 from attention_kernel_triton_amd import decode_flash_attention_redundant_var_len_paged as pg
 from attention_kernel_triton_amd import _ops
 from attention_kernel_triton_amd import synthetic as syn
-from helpers import assert_close
+from helpers import assert_close, takes_stream_kernel
 from oracle import naive
 
 pytestmark = pytest.mark.gpu
@@ -84,42 +84,50 @@ def test_paged_reference_fixture(dev):
     assert_close(lse, rl, atol=1e-4, what="paged fixture lse")
 
 
+# B = 5: the chunked kernel; B = 64 (128 units): the stream-K kernel where pages hold
+# whole 16-token groups.
 @pytest.mark.parametrize("page", [1, 8, 16, 48, 64])
 @pytest.mark.parametrize("D", [64, 128, 256])
-def test_paged_page_sizes(dev, page, D):
-    p = syn.paged_config(seed=page * 3 + D, B=5, Hq=8, Hkv=2, D=D, page=page, min_len=1,
+@pytest.mark.parametrize("B", [5, 64])
+def test_paged_page_sizes(dev, page, D, B):
+    p = syn.paged_config(seed=page * 3 + D, B=B, Hq=8, Hkv=2, D=D, page=page, min_len=1,
                          max_len=700, extra_pages=7)
+    assert takes_stream_kernel(p.q, p.pool, p.indices) == (B == 64 and page % 16 == 0)
     o, lse = _paged_call(p, dev, return_lse=True)
     ro, rl = naive.naive_paged_attention(p.q, p.pool, p.indptr, p.indices, p.last_len)
     assert_close(o, ro, what=f"paged page={page} D={D}")
     assert_close(lse, rl, atol=1e-4, what="paged lse")
 
 
-def test_paged_empty_sequences_and_clamped_last_len(dev):
+@pytest.mark.parametrize("copies", [1, 16])  # 8 and 128 units: chunked and stream-K kernel
+def test_paged_empty_sequences_and_clamped_last_len(dev, copies):
     g = torch.Generator().manual_seed(9)
     pool = torch.randn(10, 2, 2, 16, 128, generator=g).half()
-    q = torch.randn(4, 8, 1, 128, generator=g).half()
-    indptr = torch.tensor([0, 0, 3, 3, 5], dtype=torch.int32)  # sequences 0 and 2 are empty
-    indices = torch.tensor([9, 2, 4, 0, 7], dtype=torch.int32)
-    last = torch.tensor([5, 40, 3, 0], dtype=torch.int32)       # 40 clamps to 16, 0 drops a page
+    q = torch.randn(4 * copies, 8, 1, 128, generator=g).half()
+    ends = torch.tensor([0, 3, 3, 5])  # sequences 0 and 2 (of each 4) are empty
+    indptr = torch.cat([torch.zeros(1), *(5 * c + ends for c in range(copies))]).to(torch.int32)
+    indices = torch.tensor([9, 2, 4, 0, 7] * copies, dtype=torch.int32)
+    last = torch.tensor([5, 40, 3, 0] * copies, dtype=torch.int32)  # 40 clamps to 16, 0 drops a page
+    assert takes_stream_kernel(q, pool, indices) == (copies == 16)
     o, lse = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev),
                                              indices.to(dev), last.to(dev), return_lse=True)
     ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)
     o, lse = o.cpu(), lse.cpu()
-    assert torch.equal(o[0], torch.zeros_like(o[0])) and torch.equal(o[2], torch.zeros_like(o[2]))
-    assert torch.isinf(lse[0]).all() and torch.isinf(lse[2]).all()
+    assert not o[0::4].any() and not o[2::4].any()
+    assert torch.isinf(lse[0::4]).all() and torch.isinf(lse[2::4]).all()
     assert_close(o, ro, what="paged edge cases")
 
 
-def test_paged_single_token_sequences_are_exact(dev):
+@pytest.mark.parametrize("B", [12, 32])  # 48 and 128 units: chunked and stream-K kernel
+def test_paged_single_token_sequences_are_exact(dev, B):
     """A one-token sequence returns its V row bit for bit (p = 1, l = 1)."""
     g = torch.Generator().manual_seed(10)
     pool = torch.randn(40, 2, 4, 16, 128, generator=g).half()
-    B = 12
     indptr = torch.arange(B + 1, dtype=torch.int32)
     indices = torch.randperm(40, generator=g)[:B].to(torch.int32)
     last = torch.ones(B, dtype=torch.int32)
     q = torch.randn(B, 16, 1, 128, generator=g).half()
+    assert takes_stream_kernel(q, pool, indices) == (B == 32)
     o = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev), indices.to(dev),
                                         last.to(dev)).cpu()
     for b in range(B):
@@ -203,9 +211,38 @@ def test_paged_invalid_page_ids_are_skipped(dev):
     assert_close(o, ro, what="invalid page skipped")
 
 
+# As above in launches of the stream-K kernel: pages of one and of several groups,
+# ids below 0 and past the pool anywhere but on a sequence's last page, whole
+# sequences of them among it.
+@pytest.mark.parametrize("page,Hkv,D", [(16, 4, 128), (64, 4, 64), (48, 2, 256)])
+def test_paged_invalid_page_ids_are_skipped_in_large_launches(dev, page, Hkv, D):
+    g = torch.Generator().manual_seed(page + D)
+    B, G = 64, 4
+    lens = torch.randint(1, 900, (B,), generator=g).tolist()
+    indptr, indices, last, P = syn.block_table(g, lens, page)
+    pool = torch.randn(P, 2, Hkv, page, D, generator=g).half()
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    bad = torch.rand(len(indices), generator=g) < 0.25
+    bad[indptr[1:].long() - 1] = False
+    bad[indptr[5]:indptr[6]] = True  # a sequence without any valid page
+    dirty = torch.where(bad, torch.tensor([-1, -(1 << 31), P, (1 << 31) - 1])[
+        torch.randint(0, 4, (len(indices),), generator=g)], indices.long()).to(torch.int32)
+    good = torch.zeros(B + 1, dtype=torch.int32)
+    for b in range(B):
+        good[b + 1] = good[b] + int((~bad[indptr[b]:indptr[b + 1]]).sum())
+    assert takes_stream_kernel(q, pool, dirty)
+    o, lse = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev),
+                                             dirty.to(dev), last.to(dev), return_lse=True)
+    ro, rl = naive.naive_paged_attention(q, pool, good, indices[~bad], last)
+    there = good[1:] > good[:-1]
+    assert_close(o, ro, what=f"page={page} D={D}")
+    assert_close(lse, rl, atol=1e-4, what="lse", mask=there)
+    assert not o.cpu()[~there].any() and torch.isinf(lse.cpu()[~there]).all()
+
+
 def test_paged_repeated_calls_are_bit_identical(dev):
-    """Dynamic work scheduling changes which workgroup runs a chunk, never the result;
-    the scheduling counters are left at zero by every call."""
+    """Which workgroup merges a unit depends on timing, never the result; the arrival
+    counters are left at zero by every call."""
     p = syn.paged_config(B=16, min_len=256, max_len=6000).to(dev)
     outs = [pg.flash_attention_decode_paged(p.q, p.pool, p.indptr, p.indices, p.last_len)
             for _ in range(4)]
@@ -261,13 +298,14 @@ def test_paged_on_two_streams_at_once(dev):
         assert torch.equal(o, ref2)
 
 
-def test_paged_page_ids_past_32_bit_byte_offsets(dev):
+# 16 and 128 units: the chunked and the stream-K kernel.
+@pytest.mark.parametrize("lens", [[100, 37], [100, 37] * 8])
+def test_paged_page_ids_past_32_bit_byte_offsets(dev, lens):
     """Pages near the end of a 4.6 GB pool: page id x page stride overflows 32 bits, so
     the row address must be formed in 64 bits.  Only the used pages are filled; the
     oracle runs on a compact copy of them."""
     Hq, Hkv, page, D = 8, 8, 16, 128
     P = 70000  # 70000 pages x 2 x 8 x 16 x 128 x 2 B = 4.6 GB
-    lens = [100, 37]
     npg = [(L + page - 1) // page for L in lens]
     used = torch.arange(P - 1, P - 1 - sum(npg), -1, dtype=torch.int32)  # highest ids first
     g = torch.Generator().manual_seed(21)
@@ -275,8 +313,9 @@ def test_paged_page_ids_past_32_bit_byte_offsets(dev):
     q = torch.randn(len(lens), Hq, 1, D, generator=g).half()
     pool = torch.empty(P, 2, Hkv, page, D, dtype=torch.float16, device=dev)
     pool[used.long().to(dev)] = content.to(dev)
-    indptr = torch.tensor([0, npg[0], npg[0] + npg[1]], dtype=torch.int32)
+    indptr = torch.tensor([0, *npg]).cumsum(0).to(torch.int32)
     last = torch.tensor([L - (n - 1) * page for L, n in zip(lens, npg)], dtype=torch.int32)
+    assert takes_stream_kernel(q, pool, used) == (len(lens) > 2)
     o, lse = pg.flash_attention_decode_paged(q.to(dev), pool, indptr.to(dev), used.to(dev),
                                              last.to(dev), return_lse=True)
     compact = torch.arange(len(used), dtype=torch.int32)
@@ -319,13 +358,15 @@ def test_paged_batch_past_the_lds_chunk_table(dev, page):
     assert torch.isinf(lse.cpu()[~nonempty]).all()
 
 
-@pytest.mark.parametrize("B", [1, 63, 64, 200, 1024])
-def test_paged_batches_up_to_the_lds_sequence_table(dev, B):
-    """The automatic path builds every workgroup's sequence table in LDS, up to
-    1024 sequences: batches from one sequence to that limit, with empty
-    sequences and clamped last-page lengths, match the oracle (O and LSE)."""
+@pytest.mark.parametrize("B,Hkv", [(1, 2), (63, 2), (64, 2), (200, 2), (1024, 2), (2, 64),
+                                   (63, 4)])
+def test_paged_batches_up_to_the_lds_sequence_table(dev, B, Hkv):
+    """Both paged kernels build every workgroup's sequence table in LDS, up to
+    1024 sequences (the stream-K kernel from 128 units on): batches from one
+    sequence to that limit, with empty sequences and clamped last-page lengths,
+    match the oracle (O and LSE)."""
     g = torch.Generator().manual_seed(70 + B)
-    Hq, Hkv, D, page = 8, 2, 128, 16
+    Hq, D, page = 4 * Hkv, 128, 16
     lens = torch.randint(1, 300, (B,), generator=g).tolist()
     for b in {0, B // 2, B - 1} if B > 2 else set():
         lens[b] = 0
@@ -334,6 +375,7 @@ def test_paged_batches_up_to_the_lds_sequence_table(dev, B):
         last[1] = 40  # clamps to the page size
     pool = torch.randn(P, 2, Hkv, page, D, generator=g).half()
     q = torch.randn(B, Hq, 1, D, generator=g).half()
+    assert takes_stream_kernel(q, pool, indices) == (B * Hkv >= 128)
     o, lse = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev),
                                              indices.to(dev), last.to(dev), return_lse=True)
     ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)
@@ -343,17 +385,23 @@ def test_paged_batches_up_to_the_lds_sequence_table(dev, B):
     assert torch.isinf(lse.cpu()[~nonempty]).all()
 
 
-@pytest.mark.parametrize("G,D", [(1, 128), (2, 64), (3, 128), (8, 256), (16, 128), (32, 64)])
-def test_paged_automatic_path_every_head_group_width(dev, G, D):
-    """Every heads-per-unit instance of the automatic path (GT = 1, 2, 4, 8,
+@pytest.mark.parametrize("G,D", [(1, 128), (2, 64), (3, 128), (8, 256), (16, 128), (32, 64),
+                                 (20, 128), (12, 256)])
+@pytest.mark.parametrize("B", [6, 64])
+def test_paged_automatic_path_every_head_group_width(dev, B, G, D):
+    """Every heads-per-unit width of the automatic path (GT = 1, 2, 4, 8,
     16; G = 3 leaves a unit's last column empty, G = 32 at D = 64 takes two
-    head groups of 16 per kv head) against the oracle, O and LSE."""
+    head groups of 16 per kv head, G = 20 and 12 leave their second one part
+    empty) against the oracle, O and LSE, with two groups to a page: on the
+    stream-K kernel with 64 sequences, and with 6 on the chunked one (except 16
+    heads to a unit at D = 64, which stay with the stream-K kernel)."""
     g = torch.Generator().manual_seed(90 + G + D)
     Hkv, page = 2, 32
-    lens = torch.randint(1, 900, (6,), generator=g).tolist()
+    lens = torch.randint(1, 900, (B,), generator=g).tolist()
     indptr, indices, last, P = syn.block_table(g, lens, page, extra_pages=2)
     pool = torch.randn(P, 2, Hkv, page, D, generator=g).half()
     q = torch.randn(len(lens), Hkv * G, 1, D, generator=g).half()
+    assert takes_stream_kernel(q, pool, indices) == (B == 64 or (G, D) == (32, 64))
     o, lse = pg.flash_attention_decode_paged(q.to(dev), pool.to(dev), indptr.to(dev),
                                              indices.to(dev), last.to(dev), return_lse=True)
     ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)

@@ -15,6 +15,7 @@ import torch
 from attention_kernel_triton_amd import _native as N
 from attention_kernel_triton_amd import _ops
 from attention_kernel_triton_amd import synthetic as syn
+from helpers import takes_stream_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -49,7 +50,7 @@ def _need(p, chunk=0):
 @pytest.mark.parametrize("case", ["config3", "over_32768_units"])
 def test_paged_decode_needs_only_the_documented_zero_prefix(dev, case):
     if case == "config3":
-        p = syn.paged_config().to(dev)  # 256 units, persistent split kernel
+        p = syn.paged_config().to(dev)  # 256 units, stream-K kernel
     else:
         # 1100 sequences x 32 kv heads = 35200 units: past the fixed counter
         # area, so the call zero-fills its extra counters itself (and, past
@@ -74,21 +75,28 @@ def test_paged_decode_needs_only_the_documented_zero_prefix(dev, case):
         assert int(ws[: N.WORKSPACE_ZERO_BYTES].count_nonzero()) == 0
 
 
-# Small launches of the automatic (stream-K) path: more waves than groups
-# (some waves empty) and fewer, units cut at many positions, paired
-# (512-thread) and unpaired (256-thread) instances.
-@pytest.mark.parametrize("lens,page,Hq,Hkv,D", [
-    ([40, 300, 1], 16, 8, 2, 128),           # 46 groups, 48 waves: two empty waves
-    ([360, 27, 4, 450, 140], 48, 8, 2, 128),  # 138 groups, 144 waves
-    ([1, 16, 17, 33], 16, 8, 1, 128),        # G = 8 (256-thread instance): 7 groups, 8 waves
-    ([700, 5, 1300], 16, 16, 4, 64),
-    ([513, 2, 90], 64, 4, 2, 256),
-    ([8192, 4000, 31, 6000], 16, 32, 8, 128),  # more groups than waves
+# Small launches of the automatic path, on the chunked kernel, and launches of the
+# stream-K kernel: more waves than groups (some waves empty) and fewer, units cut
+# at many positions, pages of several groups, one to 16 heads to a unit and two
+# units to a kv head, 512-thread and 256-thread (D = 256) instances.
+@pytest.mark.parametrize("lens,page,Hq,Hkv,D,stream", [
+    ([40, 300, 1], 16, 8, 2, 128, False),
+    ([360, 27, 4, 450, 140], 48, 8, 2, 128, False),
+    ([1, 16, 17, 33], 16, 8, 1, 128, False),
+    ([700, 5, 1300], 16, 16, 4, 64, False),
+    ([513, 2, 90], 64, 4, 2, 256, False),
+    ([8192, 4000, 31, 6000], 16, 32, 8, 128, True),    # 9112 groups on 2048 waves
+    ([40, 300, 1] * 22 + [9], 16, 8, 2, 128, True),    # 1014 groups, 1016 waves: two empty ones
+    ([360, 27, 4, 450, 140] * 13, 48, 8, 2, 128, True),
+    ([17] * 129, 16, 8, 1, 128, True),                 # 258 groups of G = 8, 264 waves
+    ([700, 5, 1300], 16, 64, 4, 64, True),             # 16 heads to a unit
+    ([3, 50], 32, 64, 2, 64, True),                    # two units to a kv head: 24 groups
+    ([513, 2, 90] * 22, 64, 4, 2, 256, True),          # G = 2, 256 threads
+    ([5] * 135, 16, 1, 1, 256, True),                  # 135 groups, 136 waves of 256-thread ones
 ])
-def test_paged_auto_path_on_dirty_workspace_matches_oracle(dev, lens, page, Hq, Hkv, D):
-    """Every unit's run of waves stores and counts its partials: the results
-    match the oracle on a workspace whose partial area holds garbage, and the
-    arrival counters are zero again after each of two calls."""
+def test_paged_auto_path_on_dirty_workspace_matches_oracle(dev, lens, page, Hq, Hkv, D, stream):
+    """The results match the oracle on a workspace whose partial area holds
+    garbage, and the arrival counters are zero again after each of two calls."""
     from oracle import naive
 
     g = torch.Generator().manual_seed(sum(lens) + page + D)
@@ -96,6 +104,7 @@ def test_paged_auto_path_on_dirty_workspace_matches_oracle(dev, lens, page, Hq, 
     pool = torch.randn(P, 2, Hkv, page, D, generator=g).half()
     q = torch.randn(len(lens), Hq, 1, D, generator=g).half()
     ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)
+    assert takes_stream_kernel(q, pool, indices) == stream
     p = syn.Paged(q.to(dev), pool.to(dev), indptr.to(dev), indices.to(dev), last.to(dev), lens)
     ws = _dirty_workspace(_need(p), dev)
     for _ in range(2):
