@@ -1166,9 +1166,10 @@ int check_workspace(const WsLayout& w, const void* ws, size_t ws_bytes) {
   return AKT_OK;
 }
 
-// Workgroups of the decode kernels resident at once on MI355X: two per CU
-// (VGPR-bound) on 256 CUs.
-constexpr int64_t kResidentWorkgroups = 512;
+constexpr int64_t kComputeUnits = 256;  // of MI355X
+// Workgroups of the decode kernels resident at once there: two per CU
+// (VGPR-bound).
+constexpr int64_t kResidentWorkgroups = 2 * kComputeUnits;
 
 // Automatic chunk length for dense / paged caches.  An item carries a fixed
 // cost (the workgroup merge, a partial, its share of the combine) that small
@@ -1240,9 +1241,46 @@ using namespace akt;
 // explicit chunk lengths, small launches and the few shapes it cannot address
 // keep the chunked split kernel (k_row, v_row: row strides; the workspace size does not
 // know them and covers both kernels).
-static bool dense_stream(int D, int64_t chunk_tokens, int64_t batch, int64_t seq_len, int64_t Y,
-                         int64_t k_row, int64_t v_row) {
-  return chunk_tokens == 0 && dense_stream_eligible(D, batch, seq_len, Y, k_row, v_row);
+//
+// Small: the split kernel's smaller workgroups start and merge sooner while its
+// chunks leave it one workgroup to a CU, the more so the fewer heads (its P.V is
+// linear in them, the stream kernel's free) and units (the stream kernel spreads
+// each over more workgroups).  Measured at 3108 shapes of 1 to 248 units, 384 to
+// 65536 groups (graph replays, us, stream / split):
+// - more split items (units x chunks) than CUs, where its time steps up: D = 128,
+//   one head, 96 units of 1211 tokens 18.8 / 23.0, 8 of 24571 26.9 / 27.4; 16
+//   heads, 8 of 24571 44.7 / 59.4;
+// - 192 units or more of up to 16 groups: D = 64, one head, 248 of 59 tokens 5.5 /
+//   8.9;
+// - else lines in units and groups by head dim and heads.  D = 64, one head, 4608
+//   groups in 64 units 11.2 / 11.0, in 8 13.5 / 11.0; 2 heads, 2048 in 16 9.5 /
+//   10.4; 16 heads, 1004 in 64 10.1 / 15.3, 4608 in 1 49.7 / 42.3.  D = 128, one
+//   head, 4608 in 64 15.2 / 14.1, in 8 17.5 / 13.8 (never before its items pass the
+//   CUs); 4 heads, 4608 in 64 15.2 / 15.7, in 8 18.5 / 16.2; 16 heads, 4608 in 32
+//   27.3 / 29.3, in 8 35.8 / 32.3.  D = 256, 8 heads, 4608 in 32 28.7 / 32.3, in 8
+//   37.7 / 35.1.
+// Over those shapes this takes 0.7% more than the better kernel each time; a line
+// at 4096 groups (1024 at D = 64) whatever the heads and units took 3.7% more, at
+// worst twice the split kernel's time.  What is left: unit counts that do not
+// fill the device evenly (D = 64, one head, 160 units of 507 tokens 11.7 / 9.3).
+static bool dense_stream(int D, int gt, int64_t chunk_tokens, int64_t batch, int64_t seq_len,
+                         int64_t Y, int64_t k_row, int64_t v_row) {
+  if (chunk_tokens != 0 || !dense_stream_eligible(batch, seq_len, Y, k_row, v_row)) return false;
+  const int64_t units = batch * Y, groups = units * ceil_div(seq_len, 16);
+  const int64_t items = units * ceil_div(seq_len, auto_chunk(seq_len * batch, Y));
+  if (units >= kComputeUnits || items > kComputeUnits || (units >= 192 && groups <= 16 * units))
+    return true;
+  if (D == 64) {
+    if (gt == 1) return units >= 64 && groups >= 3072;
+    if (gt == 2) return units >= 16 && groups >= 2048;
+    if (gt == 4) return groups >= (units >= 16 ? 1024 : 2048);
+    return groups >= 1024 && (gt == 8 || units >= 2);
+  }
+  if (D == 128)
+    return gt == 16 ? units >= 32 && groups >= 4096
+                    : gt >= 4 && units >= (gt == 4 ? 32 : 48) && groups >= 3072;
+  const int64_t min_units = gt == 1 ? 16 : gt == 2 ? 1 : gt == 4 ? 32 : 24;
+  return units >= min_units && groups >= 3072;
 }
 
 static WsLayout dense_split_layout(int64_t batch, int64_t Y, int gt, int64_t D, int64_t seq_len,
@@ -1265,7 +1303,7 @@ extern "C" size_t akt_decode_workspace_size(int64_t batch, int64_t num_q_heads,
   const int gt = pick_gt(G, (int)head_dim);
   const int64_t Y = num_kv_heads * ceil_div(G, gt);
   const WsLayout split = dense_split_layout(batch, Y, gt, head_dim, seq_len, chunk_tokens);
-  if (!dense_stream((int)head_dim, chunk_tokens, batch, seq_len, Y, 0, 0)) return split.total;
+  if (!dense_stream((int)head_dim, gt, chunk_tokens, batch, seq_len, Y, 0, 0)) return split.total;
   const WsLayout stream = dense_stream_layout(batch, Y, gt, head_dim, seq_len);
   return split.fits && split.total > stream.total ? split.total : stream.total;
 }
@@ -1291,7 +1329,8 @@ extern "C" int akt_decode_fwd(const void* q, const void* k, const void* v, void*
   const int gt = pick_gt(G, D);
   const int n_hg = (int)ceil_div(G, gt);
   const int64_t Y = num_kv_heads * n_hg;
-  const bool use_stream = dense_stream(D, chunk_tokens, batch, seq_len, Y, k_stride[2], v_stride[2]);
+  const bool use_stream =
+      dense_stream(D, gt, chunk_tokens, batch, seq_len, Y, k_stride[2], v_stride[2]);
   const WsLayout wl = use_stream
                           ? dense_stream_layout(batch, Y, gt, D, seq_len)
                           : dense_split_layout(batch, Y, gt, D, seq_len, chunk_tokens);

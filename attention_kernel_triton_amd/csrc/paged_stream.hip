@@ -159,7 +159,7 @@ __attribute__((amdgpu_waves_per_eu(stream_min_waves<D, GT>(), 8))) void paged_st
   constexpr int SEG1 = SEG * 4 > 16 * VROW * 2 ? SEG : 16 * VROW / 2;
   __shared__ __attribute__((aligned(16))) float sm_seg0[kSWaves][SEG];
   __shared__ __attribute__((aligned(16))) float sm_seg1[kSWaves][SEG1];
-  __shared__ float4_t sm_ml[kSWaves][2][GT];  // max, fp16-P normaliser, fp32 normaliser, -
+  __shared__ float4_t sm_ml[kSWaves][2][GT];  // max, normaliser, the same again, -
   __shared__ int sm_unit[kSWaves][2];         // unit of each slot (-1: unused)
 
   const int tid = threadIdx.x;
@@ -940,21 +940,11 @@ int paged_stream_launch(const StreamParams& p, int D, int gt, hipStream_t st) {
   return with_instance<false>(D, gt, [&](auto s) { return s.launch(p, st); });
 }
 
-// Small launches keep the chunked split kernel, whose smaller workgroups start
-// and merge sooner: below 4096 groups in all (1024 at D = 64), unless there is
-// a unit for every CU.  Measured (us, this kernel / split): D = 128, N = 504
-// 11.1 / 9.3, 2504 20.0 / 16.8, 2560 in 256 units 9.1 / 10.5, 4864 12.6 / 13.8,
-// 8192 17.2 / 18.3, 64000 91.4 / 99.5 and with 8 heads to a unit 43.5 / 62.0;
-// D = 256, N = 2016 15.8 / 13.9, 4864 18.9 / 19.9; D = 64, N = 504 9.1 / 8.6,
-// 2016 9.3 / 10.0, 8192 10.6 / 14.0.
-bool dense_stream_eligible(int D, int64_t batch, int64_t seq_len, int64_t Y, int64_t k_row,
+bool dense_stream_eligible(int64_t batch, int64_t seq_len, int64_t Y, int64_t k_row,
                            int64_t v_row) {
   const int64_t most = (int64_t)1 << 26;
-  if (batch < 1 || seq_len < 1 || k_row < 0 || k_row >= most || v_row < 0 || v_row >= most ||
-      batch >= ((int64_t)1 << 31) / Y / ceil_div(seq_len, 16))
-    return false;
-  const int64_t units = batch * Y, groups = units * ceil_div(seq_len, 16);
-  return groups >= (D == 64 ? 1024 : 4096) || units >= kCUs;
+  return batch >= 1 && seq_len >= 1 && k_row >= 0 && k_row < most && v_row >= 0 && v_row < most &&
+         batch < ((int64_t)1 << 31) / Y / ceil_div(seq_len, 16);
 }
 
 int64_t dense_stream_parts(int D, int gt, int64_t units, int64_t unit_groups) {

@@ -11,7 +11,7 @@ namespace akt {
 // Largest batch whose sequence table fits the kernel's LDS.
 constexpr int kStreamMaxBatch = 1024;
 // Most waves a launch uses.  (The paged workspace is sized for a partial slot
-// per wave and unit, the public contract, more than the merge needs.)
+// per wave and unit, the public contract, more than the slots below.)
 constexpr int kStreamMaxWaves = 4096;
 
 struct StreamParams {
@@ -25,7 +25,7 @@ struct StreamParams {
   float* lse;     // [B, Hq] or null
   int* arrive;    // [workgroups] arrival counters (zero between launches)
   float* part_o;  // [slots, GT, D], slots < workgroups + min(workgroups, B * Y)
-  float* part_ml; // [slots, GT, 4]: max, fp16-P normaliser, fp32 normaliser, pad
+  float* part_ml; // [slots, GT, 4]: max, normaliser, the same again, pad
   int64_t q_sb, q_sh;
   int64_t k_sa, k_head, v_sa, v_head;  // page (dense: batch) and kv-head strides (elements)
   int k_sb, v_sb;                      // row strides (elements, < 2^26)
@@ -51,8 +51,8 @@ struct StreamParams {
 bool paged_stream_eligible(int64_t batch, int64_t page_size, int64_t total_pages, int64_t Y);
 
 // Waves a launch of instance (D, gt) uses at most on the current device
-// (resident workgroups x 4, at most kStreamMaxWaves; kStreamMaxWaves when the
-// device cannot be queried).
+// (its resident workgroups' waves, eight each up to D = 128 and four at 256, at
+// most kStreamMaxWaves; kStreamMaxWaves when the device cannot be queried).
 int64_t paged_stream_wave_cap(int D, int gt);
 
 // Launches the kernel for head dim D with gt heads per unit; the range fields
@@ -60,8 +60,8 @@ int64_t paged_stream_wave_cap(int D, int gt);
 int paged_stream_launch(const StreamParams& p, int D, int gt, hipStream_t st);
 
 // The same for a dense cache.  Eligible: row strides that 32-bit offsets of 16
-// rows can hold, a group axis below 2^31 and a launch large enough to gain.
-bool dense_stream_eligible(int D, int64_t batch, int64_t seq_len, int64_t Y, int64_t k_row,
+// rows can hold and a group axis below 2^31.
+bool dense_stream_eligible(int64_t batch, int64_t seq_len, int64_t Y, int64_t k_row,
                            int64_t v_row);
 int64_t dense_stream_parts(int D, int gt, int64_t units, int64_t unit_groups);
 int dense_stream_launch(const StreamParams& p, int D, int gt, hipStream_t st);

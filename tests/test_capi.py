@@ -126,9 +126,10 @@ def test_automatic_chunk_length():
     # config 2 (dense, 8 x 1024 tokens, 16 kv heads): two workgroups to each of 128
     # units, as many partials as two 512-token chunks
     assert dws(8, 64, 16, 1024, 64, 0) == _ws(128, 256, 4, 64) == dws(8, 64, 16, 1024, 64, 512)
-    # 8 units of 876 groups: 32 workgroups each, more than 28 chunks of 512 tokens
-    assert dws(1, 32, 8, 14001, 128, 0) == _ws(8, 256, 4, 128) > dws(1, 32, 8, 14001, 128, 512)
-    # 8 units of 63 groups, below the stream-K kernel's line: 128-token chunks
+    # 32 units of 129 groups: 8 workgroups each, more than 5 chunks of 512 tokens
+    assert dws(4, 32, 8, 2051, 128, 0) == _ws(32, 256, 4, 128) > dws(4, 32, 8, 2051, 128, 512)
+    # 8 units, below the stream-K kernel's lines: 512- and 128-token chunks
+    assert dws(1, 32, 8, 14001, 128, 0) == _ws(8, 8 * 28, 4, 128) == dws(1, 32, 8, 14001, 128, 512)
     assert dws(1, 32, 8, 1000, 128, 0) == _ws(8, 64, 4, 128) == dws(1, 32, 8, 1000, 128, 128)
 
 

@@ -480,6 +480,9 @@ def test_paged_units_over_many_workgroups(dev, lens, G, D):
     (256, 1, 4, 17, 64), (16, 16, 1, 33, 128), (16, 16, 2, 1, 256),   # a workgroup per unit
     (64, 2, 4, 1029, 64), (64, 2, 3, 1040, 128), (52, 1, 8, 1297, 256),
     (3, 2, 20, 12001, 64), (7, 8, 8, 1999, 128), (1, 5, 16, 14001, 128), (300, 1, 1, 250, 256),
+    (1, 5, 16, 28001, 128), (96, 1, 1, 1211, 128), (1, 1, 4, 68805, 256),  # more split items than CUs
+    (200, 1, 1, 200, 128), (1, 1, 8, 16390, 64), (16, 1, 2, 2045, 64),      # lines of the rule
+    (32, 1, 16, 2043, 128), (16, 1, 1, 3071, 256),
 ])
 @pytest.mark.parametrize("layout", ["contiguous", "padded", "sequence-major"])
 def test_dense_auto_path_layouts_and_edges(dev, B, Hkv, G, S, D, layout):
@@ -521,10 +524,10 @@ def _assert_same_with_nonfinite(got, ref, what):
 
 # An infinite V element of a used token makes its output element infinite, both
 # signs together or a NaN make it NaN, and nothing else changes; on every kernel
-# that a decode can take (stream-K from 4096 groups here, the chunked one below).
+# that a decode can take (stream-K for the longest, the chunked one for the shortest).
 # Scores are within +-6, so every probability is far above fp16's smallest.
 @pytest.mark.parametrize("D,G", [(64, 4), (128, 4), (128, 16), (256, 8)])
-@pytest.mark.parametrize("S", [300, 16 * 2050 + 5])
+@pytest.mark.parametrize("S", [300, 16 * 2050 + 5, 16 * 4300 + 5])
 @pytest.mark.parametrize("paged", [False, True])
 def test_decode_infinite_v_elements(dev, paged, S, D, G):
     g = torch.Generator().manual_seed(S + D + G)
@@ -567,7 +570,8 @@ def test_decode_infinite_v_elements(dev, paged, S, D, G):
     (True, 0, [1, 16, 17, 300, 0]), (True, 128, [1, 130, 700]),     # chunked kernel
     (True, 0, [3] * 1100),                                          # its batches past 1024
     (True, 0, [5, 16 * 1100, 16 * 1100 - 3]),                       # stream-K kernel
-    (False, 0, [1]), (False, 0, [300]), (False, 0, [16 * 2100]),    # dense
+    (False, 0, [1]), (False, 0, [300]), (False, 0, [16 * 2100]),    # dense, either kernel
+    (False, 0, [16 * 4300]),                                        # dense, stream-K kernel
 ])
 def test_decode_nan_query_head(dev, paged, chunk, lens, D, G, head):
     g = torch.Generator().manual_seed(sum(lens) + D + G)
