@@ -104,9 +104,9 @@ constexpr int kNBuf = 4;    // LDS tile buffers
 // waves per SIMD of an instance: two blocks and 64-key tiles at D = 64, one
 // block and 32-key tiles from D = 128.  Up to D = 128 that holds a wave in 256
 // VGPRs and a workgroup's four K + V buffers in 64 KB, so two waves share each
-// SIMD.  Large launches at D = 128 run eight waves over 64-key tiles (128 KB) in a
-// workgroup, one to a CU: half the barriers, tile loads and LDS stores per wave
-// (see wide_workgroups).  (Two blocks at one wave per SIMD, 128 KB of LDS, were slower at D = 128
+// SIMD.  Large launches of long sequences at D = 128 run eight waves over 64-key
+// tiles (128 KB) in a workgroup, one to a CU: half the barriers, tile loads and
+// LDS stores per wave (see wide_workgroups).  (Two blocks at one wave per SIMD, 128 KB of LDS, were slower at D = 128
 // at every length: 536-578 against 524 us on B=1, Hq=32, Hkv=8, S=8192.)  At
 // D = 192 and 256 the register budget allows one wave per SIMD.
 __host__ __device__ constexpr int rblocks_for(int D) { return D == 64 ? 2 : 1; }
@@ -297,10 +297,10 @@ void prefill_kernel(PrefillParams p) {
   half_t* __restrict__ Oh = p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
 
   // ---- K/V tile staging through registers: chunk i of this thread is
-  // 16-byte chunk tid + 256 i of the K (then V) tile: row st_r[i], global
+  // 16-byte chunk tid + 64 WAVES i of the K (then V) tile: row st_r[i], global
   // chunk st_c[i], stored at chunk position st_c[i] ^ tswz(row).  Tile j is
   // read through a buffer resource based at its first row whose range ends
-  // with row min(64, key_lim - 64 j) - 1: rows past it read as zeros, and the
+  // with row min(kBN, key_lim - kBN j) - 1: rows past it read as zeros, and the
   // per-lane offsets are loop invariants, so a tile costs no address VALU.
   constexpr int PER_T = kBN * CPR / kPThreads;  // chunks per thread per matrix
   uint4_t kst[PER_T], vst[PER_T];
@@ -602,7 +602,7 @@ void prefill_kernel(PrefillParams p) {
   // Publishes tile j + 1 (stored before the previous barrier) and retires the
   // buffer of tile j - 2, which now takes tile j + 2 from the staging
   // registers; tile j + 3 is then fetched into them.  Step t reads K of step
-  // t + 1 and V of step t - 1, so a step's turn comes at its own tile.
+  // t + 1 and V of step t, so a step's turn comes at its own tile.
   auto tile_turn = [&](int j) {
     __syncthreads();
     if (j + 2 < n_tiles) store_tile(j + 2);
@@ -929,16 +929,26 @@ bool use_split_keys(int head_dim, int64_t heads, int64_t seq_len, bool causal) {
 
 // Whether a launch runs eight-wave workgroups (D = 128): at least 768 workgroups
 // of four slots (one and a half rounds of the resident ones; below that the
-// eight waves crowd on one CU while others idle), and, if causal, a workgroup's
-// slots (8 / G row blocks) within an eighth of the sequence, so that its early
-// waves do not wait long for the last.  Measured (us, four / eight waves), causal
-// with G = 4 unless noted: 256 workgroups 29.4 / 34.2, 512 59.0 / 60.7, 752 93.8 /
-// 92.6, 1024 151.2 / 143.2, 2048 (S = 8192) 562.3 / 530.0; G = 1: 640 (S = 600)
-// 27.8 / 32.7, 1024 (S = 1024) 53.5 / 55.1, 2048 (S = 2048) 167.3 / 166.9;
-// non-causal 512 74.4 / 70.5, 1024 145.0 / 140.3, 2048 282.4 / 276.3.
-bool wide_workgroups(int head_dim, int64_t kv_heads, int64_t G, int64_t seq_len, bool causal) {
+// eight waves crowd on one CU while others idle); rows enough that the walk
+// repays the start of a workgroup that has its CU to itself; and, if causal, a
+// workgroup's slots (8 / G row blocks) within an eighth of the sequence, so that
+// its early waves do not wait long for the last.  Measured (us, four / eight
+// waves), causal with G = 4 unless noted: 256 workgroups 29.4 / 34.2, 512 59.0 /
+// 60.7, 752 93.8 / 92.6, 1024 151.2 / 143.2, 2048 (S = 8192) 562.3 / 530.0; G = 1:
+// 1024 (S = 1024) 53.5 / 55.1, 2048 (S = 2048) 167.3 / 166.9; non-causal 512 74.4 /
+// 70.5, 1024 145.0 / 140.3, 2048 282.4 / 276.3.  By rows, causal and not (both in one
+// process): B = 32, S = 300 71.0 / 83.3 and 95.9 / 105.5, B = 16, S = 600 96.6 / 100.0
+// and 144.4 / 152.0, B = 6, 48 heads, S = 1000 123.2 / 124.4 and 192.5 / 201.2, B = 8, S
+// = 1280 157.3 / 156.2 and 247.0 / 248.8, B = 4, S = 1800 149.1 / 144.9 and 259.0 /
+// 256.0, B = 16, S = 2048 677 / 664 and 1192 / 1137.  Padded sequences (64 to S rows)
+// walk less: B = 16, S = 600 65.5 / 71.8 and 110.7 / 119.5, B = 8, S = 1280 95.5 / 98.2
+// and 186.1 / 188.5, B = 4, S = 1800 111.7 / 112.1 and 212.4 / 213.6, B = 16, S = 2048
+// 304 / 315 and 698 / 687, B = 4, S = 3000 272.4 / 268.5 and 511.5 / 503.5.
+bool wide_workgroups(int head_dim, int64_t kv_heads, int64_t G, int64_t seq_len, bool causal,
+                     bool varlen) {
+  const int64_t min_rows = !varlen ? 1280 : causal ? 2560 : 1920;
   return head_dim == 128 && kv_heads * ceil_div(G * ceil_div(seq_len, 32), 4) >= 768 &&
-         (!causal || G * seq_len >= 2048);
+         seq_len >= min_rows && (!causal || G * seq_len >= 2048);
 }
 
 template <int D, bool CAUSAL, bool VARLEN, bool BF16>
@@ -1056,7 +1066,10 @@ int prefill_impl(const void* q, const void* k, const void* v, void* o, float* ls
   p.G = (int)(num_q_heads / num_kv_heads);
   p.S = (int)seq_len;
   p.n_rb = (int)ceil_div(seq_len, rows_for((int)head_dim));
-  p.waves = wide_workgroups((int)head_dim, batch * num_kv_heads, p.G, seq_len, causal != 0) ? 8 : 4;
+  p.waves = wide_workgroups((int)head_dim, batch * num_kv_heads, p.G, seq_len, causal != 0,
+                            varlen != nullptr)
+                ? 8
+                : 4;
   p.n_sg = (int)ceil_div((int64_t)p.G * p.n_rb, p.waves);
   p.grid1d = (batch > 65535 || p.n_sg > 65535) ? 1 : 0;
   p.fast_div = ((int64_t)p.G * p.n_rb + p.waves < (1ll << 22)) ? 1 : 0;

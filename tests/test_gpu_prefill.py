@@ -239,8 +239,8 @@ def test_prefill_long_sequence(dev, D):
 
 @pytest.mark.parametrize("case", ["non-causal", "var-len", "bf16", "G=1"])
 def test_prefill_d128_long_sequence_instance(dev, case):
-    """From 4096 rows, D = 128 runs its long-sequence instance (two 32-row
-    blocks per wave, 64-key tiles, one wave per SIMD).  S = 4100 also leaves a
+    """Long sequences of few heads at D = 128: four-wave workgroups that walk many
+    tiles (too few of them for the eight-wave ones).  S = 4100 also leaves a
     partial last row block and key tile."""
     B, Hq, Hkv, S, D = 1, 4, 2, 4100, 128
     if case == "G=1":
@@ -374,12 +374,17 @@ def test_prefill_large_launch_edges(dev, D, B, Hkv, G, S, causal):
     _check_prefill(dev, Q, K, V, causal, 1 / math.sqrt(D))
 
 
-# Eight-wave workgroups over 64-key tiles: large launches at D = 128.
+# Large launches at D = 128: four-wave workgroups up to 1279 rows (padded: 2559 causal,
+# 1919 not), from there eight-wave ones over 64-key tiles.
 @pytest.mark.parametrize("B,Hkv,G,S,causal", [(24, 8, 4, 130, False), (12, 4, 16, 130, True),
                                               (6, 8, 8, 257, True), (12, 4, 3, 700, True),
-                                              (48, 16, 1, 33, False)])
+                                              (48, 16, 1, 33, False), (3, 4, 7, 1281, True),
+                                              (1, 16, 4, 1537, False), (13, 2, 3, 1279, True),
+                                              (2, 2, 20, 1280, False), (3, 2, 7, 2570, True)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_prefill_d128_eight_wave_workgroups(dev, B, Hkv, G, S, causal, dtype):
     Q, K, V = _prefill_inputs(S + G, B, Hkv * G, Hkv, S, 128, dtype)
-    lens = [(37 * b) % (S + 1) for b in range(B)] if causal and dtype == torch.float16 else None
+    lens = None
+    if causal and dtype == torch.float16:
+        lens = [(37 * b) % (S + 1) if B > 5 else S // (b + 1) for b in range(B)]
     _check_prefill(dev, Q, K, V, causal, 1 / math.sqrt(128), lens)
