@@ -1171,17 +1171,17 @@ constexpr int64_t kComputeUnits = 256;  // of MI355X
 // (VGPR-bound).
 constexpr int64_t kResidentWorkgroups = 2 * kComputeUnits;
 
-// Automatic chunk length for dense / paged caches.  An item carries a fixed
-// cost (the workgroup merge, a partial, its share of the combine) that small
-// chunks do not amortise, while the last items set the launch's tail:
+// Automatic chunk length of the split kernel.  An item carries a fixed cost (the
+// workgroup merge, a partial, its share of the combine) that small chunks do not
+// amortise, while the last items set the launch's tail:
 // - the smallest of 128, 256 and 512 that cuts the launch into at most ~256
-//   items (in practice 512 unless the launch is tiny): measured on MI355X,
-//   512 beats 128 and 256 for config 2 (dense, 256 items) and config 3;
+//   items (in practice 512 unless the launch is tiny);
 // - 640 when even a lower bound on its item count (total tokens / 640 per
 //   unit) leaves each of the ~512 resident workgroups (two per CU) at least
-//   2.75 items.  Config 3 (paged, 1569 items), nine in-process pairs on
-//   three MI355X boxes: 92.3-94.4 us against 94.0-96.7 at 512 (mean -1.2 us);
-//   768-token chunks (2.6 items per workgroup) took 97-98 us.
+//   2.75 items.  Only launches that the stream-K kernel cannot address get that
+//   large (row strides or a group axis past its 32-bit offsets); 115096 tokens of
+//   8 kv heads in pages, 1569 such items, took 92.3-94.4 us against 94.0-96.7 at
+//   512 and 97-98 at 768.
 int64_t auto_chunk(int64_t total_tokens, int64_t units) {
   if ((total_tokens / 640) * units * 4 >= kResidentWorkgroups * 11) return 640;
   const int64_t want = ceil_div(total_tokens * units, 256);
@@ -1200,17 +1200,23 @@ int64_t paged_chunk(int64_t chunk_tokens, int64_t total_pages, int64_t page_size
   return chunk_tokens > 0 ? chunk_tokens : auto_chunk(total_pages * page_size, Y);
 }
 
-// Automatic split count of sparse rows: as many splits per row as fit one
-// round of resident workgroups, at most kMaxAutoSplits and at most one per 64
+// Automatic split count of sparse rows: as many splits per row as keep the launch
+// within kResidentWorkgroups, at most kMaxAutoSplits and at most one per 64
 // index slots.  A sparse workgroup is a chain of dependent round trips (nnz,
-// page table, indices, page ids, rows) whatever its token count, so a second
-// round of workgroups costs a whole second chain, and a split of a few
-// groups pays the chain for little streaming.  Measured on MI355X (split
-// kernel, settled, rotated inputs):
-//   config 4a (32 rows):  32 splits 16.4 us, 16 splits 9.8 us, 12 / 8 / 4
-//                         splits 9.1 / 9.2 / 9.1 us, 2 splits 11.4 us;
-//   config 4b (96 rows):  11 splits 23.8 us, 8 splits 29.1 us, 5 splits
-//                         18.7 us, 4 splits 19.3 us, 2 splits 20.4 us.
+// page table, indices, page ids, rows) whatever its token count, so past one
+// round of workgroups each costs a whole chain, and a split of a few groups pays
+// the chain and a merge for little streaming.  Measured over 32 to 512 rows of
+// 81 to 2560 kept tokens, dense, paged and MagicPIG (graph replays, us by splits, *
+// the automatic count):
+//   D = 128, 32 rows of 640   1: 10.7, 2: 9.3, 4: 8.2, 8*: 7.9, 16: 9.4
+//                    of 2560  1: 28.6, 4: 13.0, 8*: 12.4, 16: 14.6
+//   D = 256, 96 rows of 640   1: 20.9, 2: 16.4, 5*: 17.5, 8: 20.4
+//                    of 2560  1: 72.6, 2: 45.8, 5*: 44.2, 8: 44.4
+// On average it takes 1-3% more than the best count from 1280 tokens a row on (at
+// worst 14%: 64 rows at D = 64), 5% at 640.  Short rows would do with fewer
+// splits, most with one: 9% at 320 tokens, 17% at 81 (32 rows, D = 128 1: 4.7, 2*:
+// 5.9; at worst 39%), since the cap of one per 64 slots lets a merge in that
+// costs more than the few groups that it saves.
 constexpr int64_t kMaxAutoSplits = 8;
 int64_t auto_splits(int64_t rows, int64_t l_max) {
   int64_t s = kResidentWorkgroups / (rows > 0 ? rows : 1);

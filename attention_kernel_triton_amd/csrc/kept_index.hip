@@ -20,7 +20,9 @@
 // Measured against 32 consecutive elements to a thread (64 cache lines to a load,
 // 32 byte loads a thread for masks) and shuffles for the prefix (us): 32 rows of
 // 32000 draws, 2% kept 6.9 -> 5.3, of 100000 19.4 -> 13.5; masks 17.3 -> 5.6 and
-// 54.0 -> 9.8.  (A ballot per element instead of the packed counts: 7.9.)
+// 54.0 -> 9.8.  (A ballot per element instead of the packed counts: 7.9.)  The
+// slot of each kept element costs more: where half is kept, 32 rows of 8191 draws
+// 6.9 -> 7.5.
 #include "akt_common.hpp"
 #include "akt_host.hpp"
 

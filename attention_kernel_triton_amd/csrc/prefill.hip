@@ -920,7 +920,10 @@ void prefill_split_kernel(PrefillParams p) {
 // sequences still gain at twice that (their later rounds are the light row
 // blocks): 1024, S=1024 24.4 / 18.8, 608, S=600 16.7 / 10.9, 1216, S=600 17.3 / 18.0.
 // At D = 128 two steps of keys (S <= 64) repay one workgroup to a CU but not a
-// second: 256, S=64 7.3 / 5.9, 288, S=55 with the LSE 7.40 / 7.48.
+// second, causal or not, with the LSE or without: 192, S=48 6.9 / 5.7, 256, S=64
+// 7.4 / 6.4, 272 7.8 / 8.4, 288, S=55 7.7 / 8.1, 320, S=48 7.0 / 7.5, 512, S=64 8.3 /
+// 8.8 (up to S=33 the two are within 4% there); longer ones repay it: 288, S=96
+// 8.5 / 8.2, 320, S=130 8.9 / 8.1, 192, S=65 non-causal 8.2 / 6.0.
 bool use_split_keys(int head_dim, int64_t heads, int64_t seq_len, bool causal) {
   const int64_t wgs = heads * ceil_div(seq_len, 32);
   if (head_dim == 64 && causal && seq_len >= 512) return wgs <= 1024;

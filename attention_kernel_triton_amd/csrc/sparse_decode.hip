@@ -18,9 +18,10 @@
 // four groups' during the current ones, and every group's row loads go out
 // from registers, one group ahead.  (With an index and a page lookup before
 // each group's rows, waiting for them also waited, in order, for the previous
-// group's rows: B=3, Hq=32, D=256, 2% of 8192-32768 tokens 18.0 -> 16.2 us, with
-// MagicPIG 19.3 -> 18.9; B=1, Hq=32, D=128, 2% of 32000 tokens 8.3 -> 7.2; one
-// workgroup a row, 8%: 52.8 -> 38.6.)
+// group's rows.  Graph replays: B=3, Hq=32, D=256, 2% of 8192-32768 tokens 17.4 ->
+// 15.0 us, with MagicPIG 18.2 -> 17.5; B=1, Hq=32, D=128, 2% of 32000 tokens 9.1 ->
+// 7.8.  Rows that keep nearly everything lose: 1024 of 2000 out of 2048 tokens,
+// D = 128 146 -> 152, D = 256 280 -> 298.)
 //
 // Per group: D/32 v_mfma_f32_16x16x32_f16 give the scores, the query in all 16
 // columns, so that lane (R, c) holds tokens 4R .. 4R+3 in any column; the online

@@ -186,10 +186,12 @@ int akt_decode_fwd(const void* q, const void* k, const void* v, void* o, float* 
  *   clamped and as a running maximum, and nothing outside the arrays is touched.
  *   o: contiguous [batch, num_q_heads, head_dim]; lse optional [batch, num_q_heads].
  *   chunk_tokens 0 (automatic) runs the stream-K kernel when batch <= 1024,
- *   page_size is a multiple of 16 and the launch is not small: every wave of the launch takes a fixed
- *   range of 16-token groups, and its workspace holds one partial per wave
- *   the device keeps resident plus one per (sequence, head group), so the
- *   workspace size depends on the current device.  Otherwise, and for the
+ *   page_size is a multiple of 16 and the launch is not small: every wave of
+ *   the launch takes a fixed range of 16-token groups.  Its workspace has room
+ *   for one partial per wave the device keeps resident plus one per (sequence,
+ *   head group), more than the kernel stores (one per workgroup and one per
+ *   unit that reaches into another workgroup's range), so the workspace size
+ *   depends on the current device.  Otherwise, and for the
  *   explicit lengths 128, 256, 512 or 640, the chunked split kernel runs.
  */
 size_t akt_decode_paged_workspace_size(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
