@@ -409,6 +409,42 @@ def test_paged_automatic_path_every_head_group_width(dev, B, G, D):
     assert_close(lse, rl, atol=1e-4, what=f"paged lse G={G} D={D}")
 
 
+# Small launches with many heads to a unit, on both sides of the lines that choose
+# their kernel, against the oracle and the chunked kernel: ragged lengths with an
+# empty sequence, pages of one and several groups, a pool with padded strides, head
+# counts that leave part of a unit empty.
+@pytest.mark.parametrize("B,Hkv,G,D,page,mean,stream", [
+    (1, 1, 16, 64, 16, 1, True), (5, 2, 9, 64, 48, 700, True), (3, 2, 20, 64, 16, 400, True),
+    (8, 8, 8, 64, 16, 240, True), (8, 8, 5, 64, 32, 60, False), (2, 4, 7, 64, 16, 900, False),
+    (10, 4, 4, 64, 16, 700, True), (10, 4, 3, 64, 16, 400, False),
+    (12, 8, 16, 128, 64, 60, True), (12, 8, 13, 128, 16, 330, False), (2, 2, 16, 128, 16, 90, False),
+])
+def test_paged_small_launches_with_many_heads(dev, B, Hkv, G, D, page, mean, stream):
+    g = torch.Generator().manual_seed(B + G + D + mean)
+    lens = [mean] * B if mean == 1 else torch.randint(mean // 2, 3 * mean // 2, (B,),
+                                                      generator=g).tolist()
+    if B > 3:
+        lens[1] = 0
+    indptr, indices, last, P = syn.block_table(g, lens, page, extra_pages=2)
+    pool = torch.full((P, 2, Hkv, page + 3, D + 8), float("nan")).half()[:, :, :, :page, :D]
+    pool.copy_(torch.randn(P, 2, Hkv, page, D, generator=g))
+    q = torch.randn(B, Hkv * G, 1, D, generator=g).half()
+    assert takes_stream_kernel(q, pool, indices) == stream
+    big = torch.full((P, 2, Hkv, page + 3, D + 8), float("nan"), dtype=torch.float16, device=dev)
+    big[:, :, :, :page, :D] = pool.to(dev)
+    args = (q.to(dev), big[:, :, :, :page, :D], indptr.to(dev), indices.to(dev), last.to(dev))
+    o, lse = _ops.decode_paged(*args, return_lse=True)
+    oc, lc = _ops.decode_paged(*args, return_lse=True, chunk_tokens=128)
+    ro, rl = naive.naive_paged_attention(q, pool, indptr, indices, last)
+    there = torch.tensor(lens) > 0
+    # Two orders of fp32 sums: the fp16 results differ by at most one ulp (|o| < 4: 2^-9).
+    assert_close(o, oc, atol=2 ** -9, what="chunked kernel")
+    assert_close(lse, lc, atol=1e-4, what="chunked lse", mask=there)
+    assert_close(o, ro, what="oracle")
+    assert_close(lse, rl, atol=1e-4, what="oracle lse", mask=there)
+    assert torch.isinf(lse.cpu()[~there]).all()
+
+
 def test_paged_merges_are_coherent_across_launches(dev):
     """The last workgroup of a unit merges partials other workgroups (on any XCD)
     stored in the same launch.  Alternating two inputs over one workspace, every
